@@ -20,6 +20,11 @@ struct Mlp {
    // per-batch scratch
    size_t rows_capacity = 0;
    DeviceBuffer x, y, acts, dz0, dz1, loss;
+   // fused passes: padded widths (hidden_pad 0: the network is too wide, generic passes), packed weights
+   // and the places of the parameters in them, partial gradients of a pass's work-groups
+   uint32_t in_pad = 0, hidden_pad = 0, forward_groups = 0;
+   DeviceBuffer packed, packed_t, packed_at, packed_t_at, partial;
+   DeviceBuffer train_x, train_y, losses;  // the training set and the minibatches' losses
 
    Mlp(Context* c, uint32_t n_in, uint32_t n_hidden, uint32_t n_hidden_layers, uint64_t seed);
    void setParameters(const float* p);       // host f32 -> master, BF16 copy
@@ -34,10 +39,17 @@ struct Mlp {
 
   private:
    void reserve(size_t n);
+   float* estimates() const;        // the output unit of the last forward pass
    float* act(size_t layer) const;  // output of layer `layer` (n x dims[layer + 1])
    void forwardDevice(const float* x_dev, size_t n);
    float backwardDevice(const float* x_dev, const float* y_dev, size_t n);  // fills grad; returns the sum of squares
    void refreshCopies();
+   bool fused() const { return hidden_pad != 0; }
+   void setupFused();
+   struct MlpFused fusedPass(const float* x_dev, size_t n) const;
+   // loss and gradients of n rows: into grad, or (adam_lr != null) applied by Adam; *loss_dev receives
+   // the sum of squares
+   void fusedTrainPass(const float* x_dev, const float* y_dev, size_t n, float* loss_dev, const float* adam_lr);
 };
 
 }  // namespace rdb
