@@ -514,20 +514,13 @@ class DeviceTable:
         return self._with_bitmap(filt, run)
 
     def aggregate(self, filt, dims: list) -> list:
-        cap = 1 << 20
-        nd = max(len(dims), 1)
-        ids = np.zeros(cap * nd, np.uint32)
-        counts = np.zeros(cap, np.uint64)
+        ids, counts = _group_buffers(len(dims))
         n = _u64()
 
         def run(b):
-            _check(lib().rdb_aggregate(self._h, b.handle, ",".join(dims).encode(), _p(ids), _p(counts), cap,
+            _check(lib().rdb_aggregate(self._h, b.handle, ",".join(dims).encode(), _p(ids), _p(counts), len(counts),
                                        ctypes.byref(n)), self._ctx())
-            out = []
-            for i in range(n.value):
-                key = tuple(None if int(x) == 0xFFFFFFFF else int(x) for x in ids[i * len(dims):(i + 1) * len(dims)])
-                out.append((key, int(counts[i])))
-            return out
+            return _groups(ids, counts, n.value, len(dims))
         return self._with_bitmap(filt, run)
 
     def lane_bytes(self, max_queries: int, row_capacity: int) -> int:
@@ -570,6 +563,26 @@ class MutationArrays(tuple):
         return list(zip(*(c.tolist() for c in self)))
 
 
+_GROUP_CAPACITY = 1 << 20  # groups of one Aggregated result
+
+
+def _group_buffers(n_dims: int):
+    # not zeroed: the call writes what is read back, and clearing 8 MB or more costs ten times the query
+    return np.empty(_GROUP_CAPACITY * max(n_dims, 1), np.uint32), np.empty(_GROUP_CAPACITY, np.uint64)
+
+
+def _groups(ids: np.ndarray, counts: np.ndarray, n: int, n_dims: int) -> list:
+    """Groups as ((id per dimension, None = null), count) in the engine's order."""
+    table = ids[: n * n_dims].reshape(n, n_dims)
+    columns = []
+    for d in range(n_dims):
+        column = table[:, d].tolist()
+        if 0xFFFFFFFF in column:
+            column = [None if x == 0xFFFFFFFF else x for x in column]
+        columns.append(column)
+    return list(zip(zip(*columns) if columns else [()] * n, counts[:n].tolist()))
+
+
 def _mutation_rows(bufs, k: int, arrays: bool):
     if arrays:
         return MutationArrays(tuple(b[:k].copy() for b in bufs))
@@ -608,16 +621,10 @@ class Batch:
 
     def aggregate(self, q: int) -> list:
         dims = self.queries[q].get("dims", [])
-        cap = 1 << 20
-        ids = np.zeros(cap * max(len(dims), 1), np.uint32)
-        counts = np.zeros(cap, np.uint64)
+        ids, counts = _group_buffers(len(dims))
         n = _u64()
-        _check(lib().rdb_batch_aggregate(self._h, q, _p(ids), _p(counts), cap, ctypes.byref(n)), self.table._ctx())
-        out = []
-        for i in range(n.value):
-            key = tuple(None if int(x) == 0xFFFFFFFF else int(x) for x in ids[i * len(dims):(i + 1) * len(dims)])
-            out.append((key, int(counts[i])))
-        return out
+        _check(lib().rdb_batch_aggregate(self._h, q, _p(ids), _p(counts), len(counts), ctypes.byref(n)), self.table._ctx())
+        return _groups(ids, counts, n.value, len(dims))
 
     def results(self, arrays: bool = False) -> list:
         """Every query's result in submission order (Mutations rows as in DeviceTable.mutations_query,
