@@ -182,9 +182,9 @@ void Mlp::fusedTrainPass(const float* x_dev, const float* y_dev, size_t n, float
       u.m1 = m1.as<float>();
       u.m2 = m2.as<float>();
       u.eff = eff.as<float>();
-      u.w = bf16.as<__hip_bfloat16>();
-      u.packed = packed.as<__hip_bfloat16>();
-      u.packed_t = packed_t.as<__hip_bfloat16>();
+      u.w = bf16.as<uint16_t>();
+      u.packed = packed.as<uint16_t>();
+      u.packed_t = packed_t.as<uint16_t>();
       u.packed_at = packed_at.as<uint32_t>();
       u.packed_t_at = packed_t_at.as<uint32_t>();
       u.lr = *adam_lr;

@@ -372,11 +372,11 @@ __global__ __launch_bounds__(256) void mlpUpdateKernel(MlpUpdate u) {
       const float v = u.master[i] - u.lr * (a / u.c1) / (sqrtf(b / u.c2) + u.eps);
       u.master[i] = v;
       const __hip_bfloat16 w = __float2bfloat16(v);
-      u.w[i] = w;
+      reinterpret_cast<__hip_bfloat16*>(u.w)[i] = w;
       u.eff[i] = __bfloat162float(w);
       const uint32_t at = u.packed_at[i], at_t = u.packed_t_at[i];
-      if (at != kNotPacked) u.packed[at] = w;
-      if (at_t != kNotPacked) u.packed_t[at_t] = w;
+      if (at != kNotPacked) reinterpret_cast<__hip_bfloat16*>(u.packed)[at] = w;
+      if (at_t != kNotPacked) reinterpret_cast<__hip_bfloat16*>(u.packed_t)[at_t] = w;
    }
 }
 

@@ -2,7 +2,6 @@
 // the *Bf16 variant are BF16 parameter matrices.
 #pragma once
 
-#include <hip/hip_bf16.h>
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
@@ -43,9 +42,9 @@ struct MlpUpdate {
    float* m1 = nullptr;
    float* m2 = nullptr;
    float* eff = nullptr;
-   __hip_bfloat16* w = nullptr;
-   __hip_bfloat16* packed = nullptr;
-   __hip_bfloat16* packed_t = nullptr;
+   uint16_t* w = nullptr;         // BF16
+   uint16_t* packed = nullptr;    // BF16
+   uint16_t* packed_t = nullptr;  // BF16
    const uint32_t* packed_at = nullptr;    // parameter -> its place in packed / packed_t, or kNotPacked
    const uint32_t* packed_t_at = nullptr;
    float lr = 0, b1 = 0, b2 = 0, eps = 0, c1 = 1, c2 = 1;
