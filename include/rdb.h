@@ -223,7 +223,7 @@ int rdb_mutations_query(rdb_table* table, const char* filter, const char* column
 /* No counterpart in the reference.  rdb_mutations_query for callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc): the
  * same results, but every device buffer the call needs beyond the table (staged filter program,
- * filter words, partial sums, accumulators, rows) is carved from one file-scope device array of
+ * filter words, partial sums, accumulators) is carved from one file-scope device array of
  * 128 MiB per GPU, held until the process ends; the call makes no hipMalloc, hipFree or pinned
  * allocation.  RDB_EINVAL when the table needs more scratch than that (about 8 KiB per chunk for
  * the filter plus 4 bytes per (position, symbol) slot per chunk group).  All calls on one GPU share

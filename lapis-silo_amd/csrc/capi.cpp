@@ -1,7 +1,9 @@
 // The C ABI (include/rdb.h): status codes at the boundary, exceptions inside.
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstring>
+#include <new>
 #include <string>
 
 #include "capi_internal.h"
@@ -32,6 +34,14 @@ void Context::init(int dev) {
    for (auto& e : stage_events) hipCheck(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
    for (auto& e : prof_events) hipCheck(hipEventCreate(&e), "hipEventCreate");
    hipCheck(noallocScratch(dev, &noalloc_scratch), "allocation-free scratch address");
+   void* m = nullptr;
+   hipCheck(hipHostMalloc(&m, sizeof(Mail), hipHostMallocDefault), "pinned mail");
+   mail = new (m) Mail{0, 0};
+}
+
+unsigned long long Context::waitMail(uint32_t seq) {
+   pollHost([&] { return __atomic_load_n(&mail->seq, __ATOMIC_ACQUIRE) == seq; });
+   return mail->value;
 }
 
 void Context::profileAccumulate(int which) {
@@ -52,6 +62,7 @@ Context::~Context() {
    }
    if (stage_host) (void)hipHostFree(stage_host);
    if (pinned) (void)hipHostFree(pinned);
+   if (mail) (void)hipHostFree(mail);
    if (stream) (void)hipStreamDestroy(stream);
 }
 
@@ -107,12 +118,24 @@ const DeviceBitmap& filterOf(const Table& t, const rdb_bitmap* f) {
 // for the packed counters (at most 15 chunks per group).  When each wavefront takes its own chunks,
 // a group per four chunks (one per wavefront); when the work-group shares each tile, a group per
 // three and a half chunks (measured fastest on 62-chunk tables: 18 groups, every work-group
-// resident at once at six wavefronts per SIMD).
+// resident at once at six wavefronts per SIMD), or a chunk each up to kResidentParts chunks.
+constexpr uint32_t kResidentParts = 18;  // parts of a 66-block column resident at once: 1,188 work-groups
 uint32_t mutationGroups(const Table& t, const SeqColumn& /*col*/) {
-   if (t.ctx->mutation_groups) return std::clamp<uint32_t>(t.ctx->mutation_groups, 1u, kMaxGroups);
-   const uint32_t at_least = std::max<uint32_t>(1, (t.n_chunks + 14) / 15);
-   const uint32_t groups = t.ctx->mutation_coop ? (2 * t.n_chunks + 6) / 7 : (t.n_chunks + 3) / 4;
+   if (t.ctx->mutation_groups) {
+      return std::clamp<uint32_t>(t.ctx->mutation_groups, 1 + t.n_chunks / kMaxGroupChunks, kMaxGroups);
+   }
+   const uint32_t at_least = std::max<uint32_t>(1, std::min(kMaxGroups, (t.n_chunks + 14) / 15));
+   const uint32_t groups = t.ctx->mutation_coop ? std::max((2 * t.n_chunks + 6) / 7, std::min(t.n_chunks, kResidentParts))
+                                                : (t.n_chunks + 3) / 4;
    return std::clamp<uint32_t>(groups, at_least, kMaxGroups);
+}
+// Work-groups sharing each tile where the chunks alone leave most of the chip idle: the 132 tiles of a
+// 100 k-row table's 2 chunks (the whole query: 64 us unsplit, 56, 55, 56 and 65 with 2, 3, 4 and 9
+// work-groups a tile; more parts are more partial sums to write and add).
+constexpr uint32_t kSplitParts = 6;
+uint32_t mutationSplits(const Table& t, uint32_t groups) {
+   if (t.ctx->mutation_groups || !t.ctx->mutation_coop || t.n_chunks == 0) return 1;
+   return std::max<uint32_t>(1, kSplitParts / groups);
 }
 
 // Launch description of the Mutations kernels for column `idx` under filter `f`, with the
@@ -125,6 +148,7 @@ MutationsLaunch mutationsLaunch(Table& t, int idx, const DeviceBitmap& f) {
    m.chunk_sizes = t.chunk_sizes_dev.as<uint32_t>();
    m.n_chunks = t.n_chunks;
    m.n_groups = mutationGroups(t, col);
+   m.n_splits = mutationSplits(t, m.n_groups);
    m.unroll = t.ctx->mutation_unroll;
    m.coop = t.ctx->mutation_coop != 0;
    m.filter = f.words;
@@ -135,7 +159,10 @@ MutationsLaunch mutationsLaunch(Table& t, int idx, const DeviceBitmap& f) {
    m.heavy_sums = t.ctx->mutation_packed ? t.heavy_sums.as<uint32_t>() : nullptr;
    m.sparse_counts = col.sparse_counts.as<uint32_t>();
    m.sparse_bnd = col.sparse_bnd.as<int32_t>();
-   m.totals = t.totals.as<int64_t>();
+   auto* state = t.query_state.as<QueryState>();
+   m.totals = state->totals[t.totals_turn];
+   t.totals_turn ^= 1;
+   m.totals_next = state->totals[t.totals_turn];
    return m;
 }
 
@@ -628,17 +655,10 @@ int rdb_filter(rdb_table* table, const char* filter, rdb_bitmap** out, uint64_t*
       requireFinalized(t);
       if (!filter || !out) fail(RDB_EINVAL, "null argument");
       auto op = query::compileFilter(t, filter);
-      auto* bm = new rdb_bitmap;
-      bm->b = op->evaluate();
-      if (cardinality) {
-         try {
-            *cardinality = bm->b.cardinality();
-         } catch (...) {
-            delete bm;
-            throw;
-         }
-      }
-      *out = bm;
+      auto bm = std::make_unique<rdb_bitmap>();
+      bm->b = op->evaluate(cardinality != nullptr);
+      if (cardinality) *cardinality = bm->b.cardinality();
+      *out = bm.release();
    });
 }
 
@@ -694,7 +714,7 @@ int rdb_count(rdb_table* table, const char* filter, uint64_t* count) {
       requireFinalized(t);
       if (!filter || !count) fail(RDB_EINVAL, "null argument");
       auto op = query::compileFilter(t, filter);
-      DeviceBitmap b = op->evaluate();
+      DeviceBitmap b = op->evaluate(true);
       *count = b.cardinality();
    });
 }
@@ -715,7 +735,6 @@ int rdb_mutation_counts(rdb_table* table, const rdb_bitmap* filter, const char* 
       try {
          MutationsLaunch m = mutationsLaunch(t, idx, f);
          m.counts_out = static_cast<uint32_t*>(dev);
-         m.n_rows = t.mut_rows.as<uint32_t>();
          hipCheck(launchMutations(m, t.ctx->stream), "mutations kernels");
          hipCheck(hipMemcpyAsync(counts, dev, bytes, hipMemcpyDeviceToHost, t.ctx->stream), "copy counts");
          hipCheck(hipStreamSynchronize(t.ctx->stream), "synchronize");
@@ -731,44 +750,32 @@ int rdb_mutation_counts(rdb_table* table, const rdb_bitmap* filter, const char* 
 
 namespace rdb::capi {
 
-// Mutations rows under a device filter: kernels, one readback, reference output order
-// (mutations_node.cpp:292-366).
-std::vector<MutationRowDev> mutationRows(Table& t, const DeviceBitmap& f, int idx, double min_proportion) {
-   // device buffer: a 16-byte header holding the row count, then the rows
-   auto* base = t.mut_rows.as<uint8_t>();
-   auto* n_dev = reinterpret_cast<uint32_t*>(base);
-   auto* rows_dev = reinterpret_cast<MutationRowDev*>(base + 16);
-   const uint32_t row_cap = static_cast<uint32_t>((t.mut_rows.bytes() - 16) / sizeof(MutationRowDev));
+// Mutations rows under a device filter: kernels whose last one writes the rows to pinned host memory in
+// the reference's output order (mutations_node.cpp:292-366).
+ResultRows mutationResult(Table& t, const DeviceBitmap& f, int idx, double min_proportion) {
+   Context& ctx = *t.ctx;
+   void* pinned = ctx.pinnedBuffer(t.result_bytes);
    MutationsLaunch m = mutationsLaunch(t, idx, f);
    m.min_proportion = min_proportion;
-   m.rows = rows_dev;
-   m.row_capacity = row_cap;
-   m.n_rows = n_dev;
-   if (t.ctx->profiling) {
-      m.count_start = t.ctx->prof_events[0];
-      m.count_stop = t.ctx->prof_events[1];
+   const ResultRows r(pinned, t.seq[idx]->view);
+   m.rows = const_cast<MutationRowDev*>(r.rows);
+   m.stamps = static_cast<unsigned long long*>(pinned);
+   m.stamp = ++ctx.mail_seq;
+   if (ctx.profiling) {
+      m.count_start = ctx.prof_events[0];
+      m.count_stop = ctx.prof_events[1];
    }
-   hipCheck(launchMutations(m, t.ctx->stream), "mutations kernels");
-   if (t.ctx->profiling) t.ctx->profileAccumulate(0);
-   // one copy brings the count and the first rows; a second one only for long outputs
-   constexpr size_t kFirst = 2048;
-   const size_t first_bytes = std::min(16 + kFirst * sizeof(MutationRowDev), t.mut_rows.bytes());
-   auto* host = static_cast<uint8_t*>(t.ctx->pinnedBuffer(first_bytes));
-   hipCheck(hipMemcpyAsync(host, base, first_bytes, hipMemcpyDeviceToHost, t.ctx->stream), "copy rows");
-   hipCheck(hipStreamSynchronize(t.ctx->stream), "synchronize");
-   uint32_t rows_n = 0;
-   std::memcpy(&rows_n, host, 4);
-   if (rows_n > row_cap) fail(RDB_EDEVICE, "internal: mutation row buffer overflow");
-   std::vector<MutationRowDev> rows(rows_n);
-   const size_t in_first = std::min<size_t>(rows_n, (first_bytes - 16) / sizeof(MutationRowDev));
-   if (in_first) std::memcpy(rows.data(), host + 16, in_first * sizeof(MutationRowDev));
-   if (rows_n > in_first) {
-      hipCheck(hipMemcpyAsync(rows.data() + in_first, rows_dev + in_first, (rows_n - in_first) * sizeof(MutationRowDev),
-                              hipMemcpyDeviceToHost, t.ctx->stream),
-               "copy rows");
-      hipCheck(hipStreamSynchronize(t.ctx->stream), "synchronize");
-   }
-   sortMutationRows(rows);
+   hipCheck(launchMutations(m, ctx.stream), "mutations kernels");
+   if (ctx.profiling) ctx.profileAccumulate(0);
+   r.wait(ctx, m.stamp);
+   return r;
+}
+
+std::vector<MutationRowDev> mutationRows(Table& t, const DeviceBitmap& f, int idx, double min_proportion) {
+   const ResultRows r = mutationResult(t, f, idx, min_proportion);
+   std::vector<MutationRowDev> rows;
+   rows.reserve(r.size());
+   r.forEach([&](const MutationRowDev& row) { rows.push_back(row); });
    return rows;
 }
 
@@ -779,19 +786,33 @@ void sortMutationRows(std::vector<MutationRowDev>& rows) {
    });
 }
 
+template <typename Rows, typename Each>
+static void emitRows(const SeqColumn& col, const Rows& rows, uint32_t* position, uint8_t* from, uint8_t* to,
+                     uint32_t* count, uint32_t* coverage, double* proportion, uint64_t capacity, uint64_t* n, Each each) {
+   *n = rows.size();
+   if (*n > capacity) fail(RDB_ENOMEM, "output capacity too small");
+   size_t i = 0;
+   each([&](const MutationRowDev& r) {
+      if (position) position[i] = r.position + 1;
+      if (from) from[i] = col.reference[r.position];
+      if (to) to[i] = static_cast<uint8_t>(r.symbol);
+      if (count) count[i] = r.count;
+      if (coverage) coverage[i] = r.coverage;
+      if (proportion) proportion[i] = static_cast<double>(r.count) / static_cast<double>(r.coverage);
+      ++i;
+   });
+}
+
 void emitMutationRows(const SeqColumn& col, const std::vector<MutationRowDev>& rows, uint32_t* position, uint8_t* from,
                       uint8_t* to, uint32_t* count, uint32_t* coverage, double* proportion, uint64_t capacity,
                       uint64_t* n) {
-   *n = rows.size();
-   if (rows.size() > capacity) fail(RDB_ENOMEM, "output capacity too small");
-   for (size_t i = 0; i < rows.size(); ++i) {
-      if (position) position[i] = rows[i].position + 1;
-      if (from) from[i] = col.reference[rows[i].position];
-      if (to) to[i] = static_cast<uint8_t>(rows[i].symbol);
-      if (count) count[i] = rows[i].count;
-      if (coverage) coverage[i] = rows[i].coverage;
-      if (proportion) proportion[i] = static_cast<double>(rows[i].count) / static_cast<double>(rows[i].coverage);
-   }
+   emitRows(col, rows, position, from, to, count, coverage, proportion, capacity, n,
+            [&](auto&& f) { for (const MutationRowDev& r : rows) f(r); });
+}
+
+void emitMutationRows(const SeqColumn& col, const ResultRows& rows, uint32_t* position, uint8_t* from, uint8_t* to,
+                      uint32_t* count, uint32_t* coverage, double* proportion, uint64_t capacity, uint64_t* n) {
+   emitRows(col, rows, position, from, to, count, coverage, proportion, capacity, n, [&](auto&& f) { rows.forEach(f); });
 }
 
 int mutationColumn(const Table& t, const char* column, double min_proportion) {
@@ -809,7 +830,7 @@ void runMutations(Table& t, const DeviceBitmap& f, const char* column, double mi
                   uint8_t* from, uint8_t* to, uint32_t* count, uint32_t* coverage, double* proportion,
                   uint64_t capacity, uint64_t* n) {
    const int idx = capi::mutationColumn(t, column, min_proportion);
-   const auto rows = capi::mutationRows(t, f, idx, min_proportion);
+   const ResultRows rows = capi::mutationResult(t, f, idx, min_proportion);
    capi::emitMutationRows(*t.seq[idx], rows, position, from, to, count, coverage, proportion, capacity, n);
 }
 
@@ -863,16 +884,14 @@ int rdb_mutations_query_noalloc(rdb_table* table, const char* filter, const char
       query::Emitter program;
       query::compileFilter(t, filter)->emit(program);
       query::programDepth(*t.ctx, program);
-      const std::vector<uint8_t> blob = query::programBlob(program);
+      const std::vector<uint8_t> blob = query::programInline(program) ? std::vector<uint8_t>() : query::programBlob(program);
       const uint32_t L = col.genome_length;
       const uint32_t n_slots = col.view.n_slots;
-      const uint32_t n_pblocks = (L + kMutPosBlock - 1) / kMutPosBlock;
-      const size_t row_cap = std::max<size_t>(static_cast<size_t>(L) * 32, 2048);
       // carve the scratch; fewer chunk groups (partial sums) when the table needs it
       struct Carve {
-         size_t blob, words, card, partial, heavy, totals, sparse_counts, sparse_bnd, rows, end;
+         size_t blob, words, card, partial, heavy, state, sparse_counts, sparse_bnd, end;
       } c{};
-      auto layout = [&](uint32_t groups) {
+      auto layout = [&](uint32_t parts) {
          size_t o = 0;
          auto take = [&](size_t bytes) {
             const size_t at = o;
@@ -882,19 +901,22 @@ int rdb_mutations_query_noalloc(rdb_table* table, const char* filter, const char
          c.blob = take(blob.size());
          c.words = take(static_cast<size_t>(t.n_chunks) * kChunkWords * 8);
          c.card = take(64 + 4ULL * t.n_chunks);  // cardinality, then the per-chunk cardinalities
-         c.partial = take(4ULL * groups * n_slots);
+         c.partial = take(4ULL * parts * n_slots);
          c.heavy = take(4ULL * n_slots);
-         c.totals = take(static_cast<size_t>(n_pblocks) * 3 * sizeof(int64_t));
+         c.state = take(QueryState::bytes(t.n_chunks));
          c.sparse_counts = take(4ULL * L * col.abc->count);
          c.sparse_bnd = take(4ULL * 3 * L);
-         c.rows = take(16 + row_cap * sizeof(MutationRowDev));
          c.end = o;
       };
-      uint32_t groups = mutationGroups(t, col);
-      layout(groups);
-      while (c.end > kNoAllocScratchBytes && groups > 1) {
-         groups = (groups + 1) / 2;
-         layout(groups);
+      uint32_t groups = mutationGroups(t, col), splits = mutationSplits(t, groups);
+      layout(groups * splits);
+      while (c.end > kNoAllocScratchBytes && groups * splits > 1) {
+         if (splits > 1) {
+            splits = (splits + 1) / 2;
+         } else {
+            groups = (groups + 1) / 2;
+         }
+         layout(groups * splits);
       }
       if (c.end > kNoAllocScratchBytes) {
          fail(RDB_EINVAL, "table too large for rdb_mutations_query_noalloc: needs " + std::to_string(c.end) +
@@ -902,10 +924,15 @@ int rdb_mutations_query_noalloc(rdb_table* table, const char* filter, const char
       }
       auto* base = static_cast<uint8_t*>(t.ctx->noalloc_scratch);
       hipStream_t stream = t.ctx->stream;
-      hipCheck(hipMemcpyAsync(base + c.blob, blob.data(), blob.size(), hipMemcpyHostToDevice, stream), "stage program");
+      if (!blob.empty()) {
+         hipCheck(hipMemcpyAsync(base + c.blob, blob.data(), blob.size(), hipMemcpyHostToDevice, stream), "stage program");
+      }
       auto* card = reinterpret_cast<unsigned long long*>(base + c.card);
       auto* chunk_cards = reinterpret_cast<uint32_t*>(base + c.card + 64);
-      query::launchProgram(t, program, base + c.blob, reinterpret_cast<uint64_t*>(base + c.words), card, chunk_cards);
+      auto* state = reinterpret_cast<QueryState*>(base + c.state);
+      hipCheck(launchFill(reinterpret_cast<uint32_t*>(state), 0, QueryState::bytes(t.n_chunks) / 4, stream), "clear query state");
+      query::launchProgram(t, program, base + c.blob, reinterpret_cast<uint64_t*>(base + c.words), card, chunk_cards, state,
+                           nullptr, 0);
       // the accumulators that must start at zero: heavy sums and the sparse arrays (earlier calls
       // leave whatever they left)
       hipCheck(launchFill(reinterpret_cast<uint32_t*>(base + c.heavy), 0, n_slots, stream), "clear heavy sums");
@@ -919,6 +946,7 @@ int rdb_mutations_query_noalloc(rdb_table* table, const char* filter, const char
       m.chunk_sizes = t.chunk_sizes_dev.as<uint32_t>();
       m.n_chunks = t.n_chunks;
       m.n_groups = groups;
+      m.n_splits = splits;
       m.unroll = t.ctx->mutation_unroll;
       m.coop = t.ctx->mutation_coop != 0;
       m.filter = reinterpret_cast<const uint64_t*>(base + c.words);
@@ -929,24 +957,17 @@ int rdb_mutations_query_noalloc(rdb_table* table, const char* filter, const char
       m.heavy_sums = t.ctx->mutation_packed ? reinterpret_cast<uint32_t*>(base + c.heavy) : nullptr;
       m.sparse_counts = reinterpret_cast<uint32_t*>(base + c.sparse_counts);
       m.sparse_bnd = reinterpret_cast<int32_t*>(base + c.sparse_bnd);
-      m.totals = reinterpret_cast<int64_t*>(base + c.totals);
+      m.totals = state->totals[0];
+      m.totals_next = state->totals[1];
       m.min_proportion = min_proportion;
-      m.n_rows = reinterpret_cast<uint32_t*>(base + c.rows);
-      m.rows = reinterpret_cast<MutationRowDev*>(base + c.rows + 16);
-      m.row_capacity = static_cast<uint32_t>(row_cap);
+      // the rows go to the pinned buffer that the table's finalize made large enough
+      void* pinned = t.ctx->pinnedBuffer(t.result_bytes);
+      const ResultRows rows(pinned, col.view);
+      m.rows = const_cast<MutationRowDev*>(rows.rows);
+      m.stamps = static_cast<unsigned long long*>(pinned);
+      m.stamp = ++t.ctx->mail_seq;
       hipCheck(launchMutations(m, stream), "mutations kernels");
-      uint32_t rows_n = 0;
-      hipCheck(hipMemcpyAsync(&rows_n, base + c.rows, 4, hipMemcpyDeviceToHost, stream), "copy row count");
-      hipCheck(hipStreamSynchronize(stream), "synchronize");
-      if (rows_n > row_cap) fail(RDB_EDEVICE, "internal: mutation row buffer overflow");
-      std::vector<MutationRowDev> rows(rows_n);
-      if (rows_n) {
-         hipCheck(hipMemcpyAsync(rows.data(), base + c.rows + 16, rows_n * sizeof(MutationRowDev), hipMemcpyDeviceToHost,
-                                 stream),
-                  "copy rows");
-         hipCheck(hipStreamSynchronize(stream), "synchronize");
-      }
-      capi::sortMutationRows(rows);
+      rows.wait(*t.ctx, m.stamp);
       capi::emitMutationRows(col, rows, position, from, to, count, coverage, proportion, capacity, n);
    });
 }
@@ -1000,7 +1021,7 @@ struct RowArrays {
 };
 
 RowArrays mutationRowArrays(Table& t, const DeviceBitmap& f, int idx, double min_proportion) {
-   const auto rows = capi::mutationRows(t, f, idx, min_proportion);
+   const ResultRows rows = capi::mutationResult(t, f, idx, min_proportion);
    RowArrays a;
    const size_t n = rows.size();
    a.position.resize(n);

@@ -67,13 +67,17 @@ void decodeBins(const std::vector<AggDim>& ds, const uint32_t* stride, const std
 void aggregateRows(Table& t, const DeviceBitmap& f, const char* dims, std::vector<uint32_t>& ids,
                    std::vector<uint64_t>& counts);
 
-// Mutations of column `idx` under a device filter, rows sorted in the reference's output order.
+// Mutations of column `idx` under a device filter, rows in the reference's output order; the result lies
+// in the context's pinned buffer until its next use.
+ResultRows mutationResult(Table& t, const DeviceBitmap& f, int idx, double min_proportion);
 std::vector<MutationRowDev> mutationRows(Table& t, const DeviceBitmap& f, int idx, double min_proportion);
 void sortMutationRows(std::vector<MutationRowDev>& rows);
 // Rows into the caller's arrays (position 1-based, from = original reference, proportion in double).
 void emitMutationRows(const SeqColumn& col, const std::vector<MutationRowDev>& rows, uint32_t* position, uint8_t* from,
                       uint8_t* to, uint32_t* count, uint32_t* coverage, double* proportion, uint64_t capacity,
                       uint64_t* n);
+void emitMutationRows(const SeqColumn& col, const ResultRows& rows, uint32_t* position, uint8_t* from, uint8_t* to,
+                      uint32_t* count, uint32_t* coverage, double* proportion, uint64_t capacity, uint64_t* n);
 // Column index of a Mutations query; RDB_EQUERY for an unknown column or a bad minProportion.
 int mutationColumn(const Table& t, const char* column, double min_proportion);
 

@@ -50,7 +50,10 @@ constexpr uint32_t kPadSlot = 4095;
 constexpr uint32_t kLightMaxRows = 32;
 constexpr uint32_t kMaxGroups = 32;         // chunk groups of the Mutations kernel
 constexpr uint32_t kInvalidId = 0xFFFFFFFFu;
-constexpr uint32_t kMutPosBlock = 256;      // positions per work-group of the Mutations finalize kernels
+constexpr uint32_t kMutPosBlock = 256;      // positions per work-group of the batched finalize kernels
+constexpr uint32_t kResultPos = 64;         // positions per work-group of the single-query result kernel
+constexpr uint32_t kMaxResultBlocks = 1024; // its work-groups at the longest genome (below 2^16)
+constexpr uint32_t kMaxGroupChunks = 16384; // chunks of one chunk group of the Mutations kernel
 constexpr uint32_t kRunBucket = 256;        // positions per start bucket of the missing-run index
 constexpr uint32_t kShortRun = 1024;        // longer missing runs go to a per-chunk list of their own
 
@@ -78,6 +81,9 @@ struct ContainerArenas {
 // Boundary pseudo-symbols follow the alphabet's real symbols.
 enum BoundaryKind : uint32_t { BND_COV_START = 0, BND_COV_END = 1, BND_N_START = 2, BND_N_END = 3 };
 
+constexpr uint32_t kBoundarySlotBits = 28;
+constexpr uint32_t kBoundarySlotMask = (1u << kBoundarySlotBits) - 1;
+
 struct SeqColumnView {
    uint32_t genome_length;
    uint32_t n_symbols;   // alphabet size (16 or 28); pseudo-symbols are n_symbols + BoundaryKind
@@ -96,6 +102,9 @@ struct SeqColumnView {
    const uint32_t* heavy_ptr;         // [n_blocks * n_chunks + 1] into vert.desc
    const uint32_t* slot_info;         // [n_slots] position | symbol << 16
    const uint32_t* pos_slot_ptr;      // [genome_length + 1]
+   // per position: its first boundary slot, and above kBoundarySlotBits a bit per BoundaryKind it has a
+   // slot of (those slots follow each other)
+   const uint32_t* boundary_slots;    // [genome_length]
    const uint8_t* local_ref;          // [genome_length]
    const uint8_t* reference;          // [genome_length]
    const uint32_t* cov;               // [n_chunks * 2^16] start | end << 16

@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <chrono>
 #include <cstdint>
 #include <functional>
 #include <map>
@@ -109,6 +110,16 @@ class DevicePool {
    std::map<size_t, std::vector<void*>> free_;
 };
 
+// Table scratch of the single-query kernels (one query at a time runs on the context's stream).  The
+// filter's counters are zero between queries; the two sets of totals take turns, each cleared by the
+// Mutations query that uses the other.  Per-chunk counters of the filter kernel follow it in memory.
+struct QueryState {
+   unsigned long long totals[2][3 * kMaxResultBlocks];
+   unsigned long long filter_total;
+   uint32_t* chunkCounters() { return reinterpret_cast<uint32_t*>(this + 1); }
+   static size_t bytes(uint32_t n_chunks) { return sizeof(QueryState) + 4 * static_cast<size_t>(n_chunks); }
+};
+
 struct Context {
    static constexpr size_t kStageSlots = 64;
    static constexpr size_t kStageSlotBytes = 1 << 20;
@@ -126,6 +137,25 @@ struct Context {
    void* pinned = nullptr;
    size_t pinned_bytes = 0;
    void* pinnedBuffer(size_t bytes);
+   // where the last kernel of a query reports to the host, and the number of the last request
+   Mail* mail = nullptr;
+   uint32_t mail_seq = 0;
+   // Polls until `arrived` holds (what the last kernels enqueued on the stream store in pinned memory): no
+   // interrupt and no copy on the way (8 us less than a copy and a stream synchronization).
+   template <typename Arrived>
+   void pollHost(Arrived arrived) {
+      const auto begin = std::chrono::steady_clock::now();
+      for (uint32_t spin = 1; !arrived(); ++spin) {
+         __builtin_ia32_pause();
+         // long kernels, or ones that failed: let the runtime wait and report
+         if (spin % 1024 == 0 && std::chrono::steady_clock::now() - begin > std::chrono::milliseconds(20)) {
+            hipCheck(hipStreamSynchronize(stream), "synchronize");
+            if (!arrived()) fail(RDB_EDEVICE, "internal: a query's kernels ended without their result");
+         }
+      }
+   }
+   // The value posted as answer to request `seq`, the last one.
+   unsigned long long waitMail(uint32_t seq);
    // ring of (pinned host slot, device slot, event) for small asynchronous uploads
    void* stage_host = nullptr;
    DeviceBuffer stage_dev;
@@ -210,6 +240,7 @@ struct SeqColumn {
    std::vector<uint32_t> coverage;           // covered rows per position (planner statistics)
    uint64_t row_major_bytes = 0;             // row-major mutation CSR (sparse path)
    RawVector<uint32_t> row_mut_ptr, row_nrun_ptr;  // host copies over padded rows (traffic accounting)
+   DeviceBuffer boundary_slots;
    DeviceBuffer sparse_counts, sparse_bnd;   // zero between calls; cleared by the sparse finalize
    // wall time (ms) of the index build's phases: checks, adaptation, containers, slots and tiles,
    // row-level arrays, layout checks, upload
@@ -271,7 +302,9 @@ struct Table {
    TableView view{};
 
    // per-call scratch (sized at finalize)
-   DeviceBuffer slot_counts, heavy_sums, totals, mut_rows, mut_n, labels_scratch[4], hist;
+   DeviceBuffer slot_counts, heavy_sums, query_state, labels_scratch[4], hist;
+   uint32_t totals_turn = 0;  // the set of query_state's totals that the next Mutations query uses
+   size_t result_bytes = 0;  // pinned host memory of the largest Mutations result (see ResultRows)
    size_t hist_bins_capacity = 0;
    // lanes of the batched path (created on demand)
    std::vector<std::shared_ptr<BatchLane>> lanes;
@@ -352,6 +385,45 @@ struct DeviceBitmap {
 
    uint64_t cardinality();
    std::vector<uint32_t> rows();
+};
+
+// A Mutations result in pinned host memory as the result kernel writes it: the rows of each block of
+// positions, in output order, at a place of the block's own.
+struct ResultRows {
+   const uint64_t* stamps = nullptr;       // [n_blocks]: the block's number of rows, and the query's stamp above
+   const MutationRowDev* rows = nullptr;   // block b's at rows + b * block_rows
+   uint32_t n_blocks = 0, block_rows = 0;
+
+   ResultRows() = default;
+   ResultRows(void* pinned, const SeqColumnView& col)
+       : stamps(static_cast<const uint64_t*>(pinned)),
+         rows(reinterpret_cast<const MutationRowDev*>(static_cast<uint8_t*>(pinned) + kMaxResultBlocks * 8)),
+         n_blocks(resultBlocks(col)),
+         block_rows(resultBlockRows(col)) {}
+   static size_t bytes(const SeqColumnView& col) {
+      return kMaxResultBlocks * 8 + sizeof(MutationRowDev) * resultBlocks(col) * static_cast<size_t>(resultBlockRows(col));
+   }
+   uint32_t count(uint32_t b) const { return static_cast<uint32_t>(stamps[b]); }
+   void wait(Context& ctx, uint32_t stamp) const {
+      uint32_t b = 0;  // the first block not seen yet
+      ctx.pollHost([&] {
+         while (b < n_blocks && static_cast<uint32_t>(__atomic_load_n(stamps + b, __ATOMIC_ACQUIRE) >> 32) == stamp) ++b;
+         return b == n_blocks;
+      });
+   }
+   size_t size() const {
+      size_t n = 0;
+      for (uint32_t b = 0; b < n_blocks; ++b) n += count(b);
+      return n;
+   }
+   template <typename F>
+   void forEach(F f) const {
+      for (uint32_t b = 0; b < n_blocks; ++b) {
+         const MutationRowDev* r = rows + static_cast<size_t>(b) * block_rows;
+         const uint32_t n = count(b);
+         for (uint32_t k = 0; k < n; ++k) f(r[k]);
+      }
+   }
 };
 
 }  // namespace rdb

@@ -39,22 +39,76 @@ hipError_t launchFilter(const TableView& tv, const ProgramDesc* progs, const Ins
                         uint32_t* chunk_cards, uint32_t max_blocks, hipStream_t stream,
                         const uint32_t* n_queries_dev = nullptr);
 
+// A value that a kernel leaves for the host in pinned memory: the host polls `seq` for the number of
+// its request.
+struct alignas(64) Mail {
+   unsigned long long value;
+   uint32_t seq;
+};
+
+// One filter program for launchFilterSingle: its instructions, ranges and prefetch codes as words,
+// passed with the kernel's arguments (4 KiB in all) or, when longer, staged in device memory.
+// chunk_counters [n_chunks] and total_counter are zero on entry and zero again on exit; the
+// cardinality goes to `mail` under mail_seq too, unless that is null.
+constexpr uint32_t kInlineProgramWords = 768;
+struct SingleProgram {
+   ProgramDesc desc;               // ranges and prefetch codes counted from the end of the instructions
+   const uint32_t* staged;
+   uint32_t* chunk_counters;
+   unsigned long long* total_counter;
+   Mail* mail;
+   uint32_t mail_seq;
+   alignas(16) uint32_t words[kInlineProgramWords];
+};
+// Evaluates one program over the table (at least one chunk): words, cardinality and per-chunk
+// cardinalities are all written, whatever they held.
+hipError_t launchFilterSingle(const TableView& tv, const SingleProgram& program, uint32_t depth, uint64_t* out,
+                              unsigned long long* card, uint32_t* chunk_cards, hipStream_t stream);
+
+// Work-groups of the result kernel of one Mutations query, and the rows each may write.
+inline uint32_t resultBlocks(const SeqColumnView& c) { return (c.genome_length + kResultPos - 1) / kResultPos; }
+inline uint32_t resultBlockRows(const SeqColumnView& c) { return kResultPos * c.n_valid; }
+
+// What the result kernel of one Mutations query reads and writes (the members of MutationsLaunch).
+constexpr uint32_t kResultThreads = 256;
+struct MutationsResult {
+   const uint32_t* partial = nullptr;
+   uint32_t n_parts = 0;
+   uint32_t* heavy = nullptr;
+   uint32_t* sparse_counts = nullptr;
+   int32_t* sparse_bnd = nullptr;
+   const unsigned long long* totals = nullptr;
+   unsigned long long* totals_next = nullptr;
+   const unsigned long long* filter_card = nullptr;
+   long long sparse_max = -1;
+   double min_proportion = 0.0;
+   uint32_t* counts_out = nullptr;
+   MutationRowDev* rows = nullptr;
+   uint32_t block_rows = 0;
+   unsigned long long* stamps = nullptr;
+   uint32_t stamp = 0;
+};
+
 // Mutations for one filter.  Two methods, both launched; the filter's device-side cardinality
 // picks one:
 //  * dense (cardinality > sparse_max, or sparse_max < 0): per-slot AND-popcounts of the vertical
-//    index against the filter (one partial sum per chunk group, n_groups <= kMaxGroups, `partial`
-//    holds n_groups * n_slots u32);
+//    index against the filter (one partial sum per chunk group and split of its tiles, n_groups *
+//    n_splits <= kMaxGroups, `partial` holds n_groups * n_splits * n_slots u32);
 //  * sparse (cardinality <= sparse_max): each filter row adds its own mutations and boundaries;
 //    sparse_counts ([n_symbols][L] u32) and sparse_bnd ([3][L] i32) must be zero on entry and are
 //    zero again on exit.
 // Then boundary prefix sums, the implicit (reference) count and thresholding.  counts_out
-// ([n_symbols][L]) and rows may be null.
+// ([n_symbols][L]) and rows may be null.  Rows come in output order per block of kResultPos positions,
+// in pinned host memory: block b's at rows + b * resultBlockRows, complete when stamps[b] holds `stamp`
+// in its high half (their number in the low half).  totals and totals_next [3 * kMaxResultBlocks]:
+// totals is zero on entry, totals_next on exit.
 struct MutationsLaunch {
    const SeqColumnView* col_dev = nullptr;
    const SeqColumnView* col_host = nullptr;
    const uint32_t* chunk_sizes = nullptr;  // device
    uint32_t n_chunks = 0;
    uint32_t n_groups = 1;
+   uint32_t n_splits = 1;                  // work-groups sharing each tile
    uint32_t unroll = 8;                    // 16-byte loads in flight per lane in the dense kernel (8 or 16)
    bool coop = false;                      // a work-group's wavefronts count each chunk tile together
    const uint64_t* filter = nullptr;
@@ -65,12 +119,13 @@ struct MutationsLaunch {
    uint32_t* heavy_sums = nullptr;         // [n_slots], zero; set: 16-bit packed LDS counters (more CU occupancy)
    uint32_t* sparse_counts = nullptr;
    int32_t* sparse_bnd = nullptr;
-   int64_t* totals = nullptr;
+   unsigned long long* totals = nullptr;
+   unsigned long long* totals_next = nullptr;
    double min_proportion = 0.0;
    uint32_t* counts_out = nullptr;
    MutationRowDev* rows = nullptr;
-   uint32_t row_capacity = 0;
-   uint32_t* n_rows = nullptr;
+   unsigned long long* stamps = nullptr;
+   uint32_t stamp = 0;
    hipEvent_t count_start = nullptr;  // recorded around the dense counting kernel when set
    hipEvent_t count_stop = nullptr;
 };

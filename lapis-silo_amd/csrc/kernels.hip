@@ -5,7 +5,9 @@
 // lane, so ballots over 64 consecutive rows map directly onto a word.
 #include <hip/hip_runtime.h>
 
+#include <cstddef>
 #include <cstdint>
+#include <type_traits>
 
 #include "device_abi.h"
 #include "kernels.h"
@@ -49,6 +51,25 @@ __device__ inline const G* toGlobal(const void* p) {
    return (const G*)(p);
 }
 
+
+// Stores to pinned host memory that a kernel reports through a Mail: written through to the system one
+// by one, and waited for by the wavefront that issued them.  A system fence instead writes back every
+// dirty line of the XCD's L2; one in each work-group of the result kernel took 30 us of its 41.
+template <typename T>
+__device__ inline void storeHost(T* p, T v) {
+   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+__device__ inline void storeHostRow(u32x4* p, u32x4 v) {
+   asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1" : : "v"(p), "v"(v) : "memory");
+}
+__device__ inline void hostStoresDone() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// Publishes a value to the host: `mail` is pinned host memory that the host polls (Context::waitMail).
+__device__ inline void postMail(Mail* mail, uint32_t seq, unsigned long long value) {
+   storeHost(&mail->value, value);
+   hostStoresDone();
+   __hip_atomic_store(&mail->seq, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 __device__ inline uint64_t layoutMask(uint32_t chunk_size, uint32_t word) {
    const uint32_t lo = word * 64;
@@ -153,6 +174,22 @@ __device__ inline uint32_t waveSum(uint32_t v) {
    return v;
 }
 
+// The sum over the wavefront, valid in every lane: adds along DPP rows (16 lanes) and row broadcasts,
+// without the LDS pipe that __shfl goes through.
+template <int kCtrl, int kRowMask, int kBankMask>
+__device__ inline uint32_t dppAdd(uint32_t v) {
+   return v + static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), kCtrl, kRowMask, kBankMask, false));
+}
+__device__ inline uint32_t waveSumDpp(uint32_t v) {
+   v = dppAdd<0x111, 0xF, 0xF>(v);  // row_shr:1
+   v = dppAdd<0x112, 0xF, 0xF>(v);  // row_shr:2
+   v = dppAdd<0x114, 0xF, 0xE>(v);  // row_shr:4
+   v = dppAdd<0x118, 0xF, 0xC>(v);  // row_shr:8
+   v = dppAdd<0x142, 0xA, 0xF>(v);  // row_bcast:15
+   v = dppAdd<0x143, 0xC, 0xF>(v);  // row_bcast:31
+   return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), 63));
+}
+
 __device__ inline uint64_t waveSum64(uint64_t v) {
    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
    return v;
@@ -163,7 +200,16 @@ __device__ inline uint64_t waveSum64(uint64_t v) {
 // programs (queries) are spread over the grid.  The operand stack lives in LDS, one 64-word row
 // slice per entry, so any operator tree depth fits that the host sized the launch for.
 // ------------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(kVmThreads) void filterVmKernel(TableView tv, const ProgramDesc* __restrict__ progs,
+//
+// kSingle: one program, read from the kernel's own arguments (or from `single.staged` when it is too
+// long for them), so that no copy precedes the launch; counters that the kernel leaves zero, so that
+// no clear does either; and the cardinality stored where the host polls for it, so that no copy
+// follows.  A count over 100 k rows is then one launch: 42 us with the copy, the clear and the copy
+// back (each 3 to 11 us on the stream), 16 us without.
+struct NoProgram {};
+template <bool kSingle>
+__global__ __launch_bounds__(kVmThreads) void filterVmKernel(std::conditional_t<kSingle, SingleProgram, NoProgram> single,
+                                                             TableView tv, const ProgramDesc* __restrict__ progs,
                                                              const Instr* __restrict__ instrs,
                                                              const uint32_t* __restrict__ ranges, uint32_t n_items,
                                                              uint32_t depth, uint64_t* __restrict__ out,
@@ -172,6 +218,16 @@ __global__ __launch_bounds__(kVmThreads) void filterVmKernel(TableView tv, const
                                                              const uint32_t* __restrict__ n_queries_dev,
                                                              uint32_t unit_slices) {
    extern __shared__ uint64_t lds[];
+   if constexpr (kSingle) {
+      // the program's words: in this kernel's argument segment, whose first argument `single` is
+      const uint32_t* words = single.staged;
+      if (words == nullptr) {
+         words = reinterpret_cast<const uint32_t*>(reinterpret_cast<uintptr_t>(__builtin_amdgcn_kernarg_segment_ptr()) +
+                                                   offsetof(SingleProgram, words));
+      }
+      instrs = reinterpret_cast<const Instr*>(words);
+      ranges = words + single.desc.n_instr * (sizeof(Instr) / 4);
+   }
    const uint32_t wave = threadIdx.x >> 6;
    const uint32_t lane = threadIdx.x & 63;
    uint64_t* stack = lds + static_cast<size_t>(wave) * (depth + 1) * 64;
@@ -196,7 +252,12 @@ __global__ __launch_bounds__(kVmThreads) void filterVmKernel(TableView tv, const
    const uint32_t unit_item = unit * unit_slices;
    const uint32_t qi = unit_item / per_query;
    const uint32_t chunk = (unit_item - qi * per_query) / kSlicesPerChunk;
-   const ProgramDesc pd = progs[qi];
+   ProgramDesc pd;
+   if constexpr (kSingle) {
+      pd = single.desc;
+   } else {
+      pd = progs[qi];
+   }
    uint32_t prog_base = 0;  // the LDS copy holds instructions prog_base .. prog_base + kProgCache - 1
    {
       waveSync();  // the previous unit's reads of the records and the program are done
@@ -212,7 +273,7 @@ __global__ __launch_bounds__(kVmThreads) void filterVmKernel(TableView tv, const
       {
          const uint32_t n_pf = pd.n_pf < kPrefetchSlots ? pd.n_pf : kPrefetchSlots;
          if (lane < n_pf) {
-            const uint32_t code = ranges[pd.pf_begin + lane];
+            const uint32_t code = toGlobal<GlobalU32>(ranges)[pd.pf_begin + lane];
             uint32_t* dst = pf + lane * 8;
             if (code >> 31) {
                const u32x2 d = toGlobal<GlobalU32x2>(tv.store.desc)[static_cast<size_t>(code & 0x7FFFFFFFu) * n_chunks + chunk];
@@ -516,8 +577,8 @@ __global__ __launch_bounds__(kVmThreads) void filterVmKernel(TableView tv, const
                const uint32_t g0 = (chunk << 16) + my_word * 64u;
                uint64_t word = 0;
                for (uint32_t j = 0; j < ins.b; ++j) {
-                  const uint32_t lo = ranges[pd.range_begin + 2 * (ins.a + j)];
-                  const uint32_t hi = ranges[pd.range_begin + 2 * (ins.a + j) + 1];
+                  const uint32_t lo = toGlobal<GlobalU32>(ranges)[pd.range_begin + 2 * (ins.a + j)];
+                  const uint32_t hi = toGlobal<GlobalU32>(ranges)[pd.range_begin + 2 * (ins.a + j) + 1];
                   const uint32_t a = lo > g0 ? lo : g0;
                   const uint32_t b = hi < g0 + 64 ? hi : g0 + 64;
                   if (a < b) word |= rangeMask(a - g0, b - 1 - g0);
@@ -643,12 +704,27 @@ __global__ __launch_bounds__(kVmThreads) void filterVmKernel(TableView tv, const
       // unit that completes the chunk leaves the chunk's rows alone in it and adds them to the
       // filter's cardinality, so that the cardinality takes one atomic per chunk (atomics on one
       // address serialise), and a unit waits for one atomic, not one per slice.
-      uint32_t* cc = &chunk_cards[static_cast<size_t>(pd.query) * n_chunks + chunk];
+      uint32_t* const card_out = &chunk_cards[static_cast<size_t>(pd.query) * n_chunks + chunk];
+      uint32_t* cc = card_out;
+      if constexpr (kSingle) cc = single.chunk_counters + chunk;
       const uint32_t old = atomicAdd(cc, (unit_slices << 20) | n);
       if ((old >> 20) + unit_slices == kSlicesPerChunk) {
          const uint32_t total = (old & 0xFFFFFu) + n;
-         *cc = total;
-         if (total) atomicAdd(&cards[pd.query], static_cast<unsigned long long>(total));
+         *card_out = total;
+         if constexpr (kSingle) {
+            // the last chunk to finish has every chunk's rows (the counter's low 40 bits; the
+            // finished chunks above them)
+            *cc = 0;
+            const unsigned long long was = atomicAdd(single.total_counter, (1ull << 40) | total);
+            if ((was >> 40) + 1 == n_chunks) {
+               const unsigned long long card = (was & ((1ull << 40) - 1)) + total;
+               *single.total_counter = 0;
+               cards[0] = card;
+               if (single.mail != nullptr) postMail(single.mail, single.mail_seq, card);
+            }
+         } else if (total) {
+            atomicAdd(&cards[pd.query], static_cast<unsigned long long>(total));
+         }
       }
    }
    }
@@ -697,11 +773,22 @@ __device__ inline uint32_t rangePopcount(const uint64_t* f, uint32_t a, uint32_t
 // 65,536 rows of a chunk, add to the global `heavy` sums instead.
 constexpr uint32_t kPackedMaxChunks = 15;
 
+//
+// split / n_splits: the part of every tile counted here (tables of few chunks split their tiles over
+// several work-groups).  totals (may be null): the block's sums of the boundary quantities per
+// kResultPos positions are added to it.
+
+// The boundary quantity a slot's symbol counts towards: 0 range starts, 1 range ends, 2 missing runs
+// started minus ended.
+__device__ inline uint32_t boundaryKind(uint32_t kind) { return kind < BND_N_START ? kind : 2u; }
+
 template <uint32_t kUnroll, bool kPacked, bool kCoop>
 __device__ __forceinline__ void countBlock(const SeqColumnView& col, uint32_t b, uint32_t g, uint32_t n_chunks,
-                                           uint32_t n_groups, const uint64_t* __restrict__ filter,
+                                           uint32_t n_groups, uint32_t split, uint32_t n_splits,
+                                           const uint64_t* __restrict__ filter,
                                            const uint32_t* __restrict__ filter_chunk_cards, uint32_t* __restrict__ out,
-                                           uint64_t (*fs)[kChunkWords], uint32_t* cnt, uint32_t* __restrict__ heavy) {
+                                           uint64_t (*fs)[kChunkWords], uint32_t* cnt, uint32_t* __restrict__ heavy,
+                                           unsigned long long* __restrict__ totals) {
    const uint32_t tid = threadIdx.x;
    const uint32_t lane = tid & 63;
    const uint32_t wave = tid >> 6;
@@ -721,6 +808,19 @@ __device__ __forceinline__ void countBlock(const SeqColumnView& col, uint32_t b,
          atomicAdd(&cnt[slot], v);
       }
    };
+   // the boundary records of this wavefront's first position groups, used at the end
+   static_assert(kResultPos == 64, "a position per lane");
+   constexpr uint32_t kRecords = 2;
+   uint32_t p_lo = 0, p_hi = 0, rec[kRecords] = {};
+   if (totals != nullptr) {
+      p_lo = col.block_pos_start[b];
+      p_hi = col.block_pos_start[b + 1];
+#pragma unroll
+      for (uint32_t u = 0; u < kRecords; ++u) {
+         const uint32_t p = (p_lo / kResultPos + wave + u * kMutWaves) * kResultPos + lane;
+         rec[u] = p >= p_lo && p < p_hi ? toGlobal<GlobalU32>(col.boundary_slots)[p] : 0u;
+      }
+   }
    uint64_t* f = fs[kCoop ? 0 : wave];
    const uint32_t* fw = reinterpret_cast<const uint32_t*>(f);
    const Desc* __restrict__ desc = col.vert.desc;
@@ -728,6 +828,19 @@ __device__ __forceinline__ void countBlock(const SeqColumnView& col, uint32_t b,
    const GlobalU32* group_ptr = toGlobal<GlobalU32>(col.group_ptr);
    const GlobalU32* heavy_ptr = toGlobal<GlobalU32>(col.heavy_ptr);
    auto countTile = [&](uint32_t l0, uint32_t l1, uint32_t g0, uint32_t g1, uint32_t h0, uint32_t h1) {
+         if (n_splits > 1) {
+            // this work-group's part: whole 16-byte groups of light entries, row groups, containers
+            const auto cut = [&](uint32_t n, uint32_t k) {
+               return static_cast<uint32_t>(static_cast<uint64_t>(n) * k / n_splits);
+            };
+            const uint32_t nl = (l1 - l0) >> 2, ng = g1 - g0, nd = h1 - h0;
+            l1 = l0 + 4 * cut(nl, split + 1);
+            l0 += 4 * cut(nl, split);
+            g1 = g0 + cut(ng, split + 1);
+            g0 += cut(ng, split);
+            h1 = h0 + cut(nd, split + 1);
+            h0 += cut(nd, split);
+         }
          // light entries: each lane walks a contiguous span of kUnroll / 2 16-byte groups per round;
          // the next round's groups are loaded before this round's are used (kUnroll in flight), all filter lookups of a round
          // are issued before any result is used, and consecutive entries of a slot are summed before
@@ -894,7 +1007,15 @@ __device__ __forceinline__ void countBlock(const SeqColumnView& col, uint32_t b,
             n = waveSum(n);
             if (lane == 0 && n) {
                if (kPacked) {
-                  atomicAdd(&heavy[s0 + descSlot(dd.w0)], n);
+                  const uint32_t slot = s0 + descSlot(dd.w0);
+                  atomicAdd(&heavy[slot], n);
+                  // (the block's own totals, below, only see the LDS counters)
+                  const uint32_t x = toGlobal<GlobalU32>(col.slot_info)[slot];
+                  if (totals != nullptr && (x >> 16) >= col.n_symbols) {
+                     const uint32_t k = (x >> 16) - col.n_symbols;
+                     atomicAdd(&totals[boundaryKind(k) * kMaxResultBlocks + (x & 0xFFFFu) / kResultPos],
+                               k == BND_N_END ? 0ull - n : static_cast<unsigned long long>(n));
+                  }
                } else {
                   atomicAdd(&cnt[descSlot(dd.w0)], n);
                }
@@ -965,8 +1086,33 @@ __device__ __forceinline__ void countBlock(const SeqColumnView& col, uint32_t b,
       }
    }
    __syncthreads();
-   for (uint32_t i = tid; i < ns; i += kMutThreads) {
-      out[s0 + i] = kPacked ? (cnt[i >> 1] >> ((i & 1u) << 4)) & 0xFFFFu : cnt[i];
+   const auto sum = [&](uint32_t i) { return kPacked ? (cnt[i >> 1] >> ((i & 1u) << 4)) & 0xFFFFu : cnt[i]; };
+   for (uint32_t i = tid; i < ns; i += kMutThreads) out[s0 + i] = sum(i);
+   if (totals == nullptr) return;
+   // a wavefront takes kResultPos positions: each lane one, its boundary slots named by one record
+   uint32_t u = 0;
+   for (uint32_t q = p_lo / kResultPos + wave; q * kResultPos < p_hi; q += kMutWaves, ++u) {
+      const uint32_t p = q * kResultPos + lane;
+      uint32_t x = 0;
+      if (u < kRecords) {
+         x = u == 0 ? rec[0] : rec[1];
+      } else if (p >= p_lo && p < p_hi) {
+         x = toGlobal<GlobalU32>(col.boundary_slots)[p];
+      }
+      uint32_t slot = (x & kBoundarySlotMask) - s0;
+      uint32_t n[4];
+#pragma unroll
+      for (uint32_t k = 0; k < 4; ++k) {
+         const bool stored = (x >> (kBoundarySlotBits + k)) & 1u;
+         n[k] = stored ? sum(slot) : 0u;
+         slot += stored ? 1u : 0u;
+      }
+      // at most one start and one end a row, and the runs open at the positions' end less those at their
+      // start: magnitudes within the group's rows (kMaxGroupChunks keeps them below 2^31)
+      const uint32_t t0 = waveSumDpp(n[BND_COV_START]), t1 = waveSumDpp(n[BND_COV_END]);
+      const int32_t t2 = static_cast<int32_t>(waveSumDpp(n[BND_N_START] - n[BND_N_END]));
+      const long long v = lane == 0 ? static_cast<long long>(t0) : lane == 1 ? static_cast<long long>(t1) : t2;
+      if (lane < 3 && v) atomicAdd(&totals[lane * kMaxResultBlocks + q], static_cast<unsigned long long>(v));
    }
 }
 
@@ -982,13 +1128,15 @@ __global__ __launch_bounds__(kMutThreads) __attribute__((amdgpu_waves_per_eu(kCo
                                                                     const unsigned long long* __restrict__ filter_card,
                                                                     long long sparse_max,
                                                                     uint32_t* __restrict__ partial,
-                                                                    uint32_t* __restrict__ heavy) {
+                                                                    uint32_t* __restrict__ heavy, uint32_t n_splits,
+                                                                    unsigned long long* __restrict__ totals) {
    __shared__ uint64_t fs[kCoop ? 1 : kMutWaves][kChunkWords];
    __shared__ uint32_t cnt[kPacked ? (kMaxBlockSlots + 1) / 2 : kMaxBlockSlots + 1];
    if (!denseActive(filter_card, sparse_max)) return;
    const SeqColumnView& col = *colp;
-   countBlock<kUnroll, kPacked, kCoop>(col, blockIdx.x, blockIdx.y, n_chunks, n_groups, filter, filter_chunk_cards,
-                                partial + static_cast<size_t>(blockIdx.y) * col.n_slots, fs, cnt, heavy);
+   countBlock<kUnroll, kPacked, kCoop>(col, blockIdx.x, blockIdx.y / n_splits, n_chunks, n_groups, blockIdx.y % n_splits,
+                                       n_splits, filter, filter_chunk_cards,
+                                       partial + static_cast<size_t>(blockIdx.y) * col.n_slots, fs, cnt, heavy, totals);
 }
 
 
@@ -1013,6 +1161,8 @@ struct SparseTable {
    int32_t* vals;
    uint32_t* counts;
    int32_t* bnd;
+   int32_t* tot = nullptr;  // LDS sums of the boundary quantities per kResultPos positions, or null
+   uint32_t length = 0;     // genome length (with tot)
 
    __device__ void clear() const {
       for (uint32_t i = threadIdx.x; i < kSparseTable; i += blockDim.x) {
@@ -1037,7 +1187,12 @@ struct SparseTable {
    }
    __device__ void flushOne(uint32_t key, int32_t v) const {
       if (key & kSparseBndKey) {
-         atomicAdd(&bnd[key & ~kSparseBndKey], v);
+         const uint32_t at = key & ~kSparseBndKey;
+         atomicAdd(&bnd[at], v);
+         if (tot != nullptr) {
+            const uint32_t kind = at >= 2 * length ? 2u : at >= length ? 1u : 0u;
+            atomicAdd(&tot[kind * kMaxResultBlocks + (at - kind * length) / kResultPos], v);
+         }
       } else {
          atomicAdd(&counts[key], static_cast<uint32_t>(v));
       }
@@ -1128,34 +1283,25 @@ __global__ __launch_bounds__(256) void sparseCountKernel(const SeqColumnView* __
                                                          const uint64_t* __restrict__ filter,
                                                          const unsigned long long* __restrict__ filter_card,
                                                          long long sparse_max, uint32_t* __restrict__ counts,
-                                                         int32_t* __restrict__ bnd) {
+                                                         int32_t* __restrict__ bnd,
+                                                         unsigned long long* __restrict__ totals) {
    __shared__ uint32_t keys[kSparseTable];
    __shared__ int32_t vals[kSparseTable];
+   __shared__ int32_t tot[3 * kMaxResultBlocks];
    if (!sparseActive(filter_card, sparse_max)) return;
-   const SparseTable tb{keys, vals, counts, bnd};
+   const SparseTable tb{keys, vals, counts, bnd, tot, colp->genome_length};
    tb.clear();
+   for (uint32_t i = threadIdx.x; i < 3 * kMaxResultBlocks; i += blockDim.x) tot[i] = 0;
    __syncthreads();
    sparseCountRows(*colp, chunk_sizes, filter, n_words, tb, blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6),
                    gridDim.x * (blockDim.x / 64));
    __syncthreads();
    tb.flush();
-}
-
-// Sums the chunk groups' partial slot counts into group 0, in place (one thread per slot).
-__global__ __launch_bounds__(256) void reducePartialsKernel(uint32_t* __restrict__ partial, uint32_t n_groups,
-                                                            uint32_t n_slots,
-                                                            const unsigned long long* __restrict__ filter_card,
-                                                            long long sparse_max, uint32_t* __restrict__ heavy) {
-   if (!denseActive(filter_card, sparse_max)) return;
-   const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-   if (s >= n_slots) return;
-   uint32_t v = partial[s];
-   for (uint32_t g = 1; g < n_groups; ++g) v += partial[static_cast<size_t>(g) * n_slots + s];
-   if (heavy) {
-      v += heavy[s];
-      heavy[s] = 0;
+   __syncthreads();
+   for (uint32_t i = threadIdx.x; i < 3 * kMaxResultBlocks; i += blockDim.x) {
+      const int32_t v = tot[i];
+      if (v) atomicAdd(&totals[i], static_cast<unsigned long long>(static_cast<long long>(v)));
    }
-   partial[s] = v;
 }
 
 // Values of one block of kPosBlock positions, staged in LDS by the totals and finalize kernels:
@@ -1299,13 +1445,6 @@ struct SparseSource {
    }
 };
 
-__device__ inline bool sourceActive(const SlotSource&, const unsigned long long* card, long long sparse_max) {
-   return denseActive(card, sparse_max);
-}
-__device__ inline bool sourceActive(const SparseSource&, const unsigned long long* card, long long sparse_max) {
-   return sparseActive(card, sparse_max);
-}
-
 template <typename T>
 __device__ inline T waveInclusiveScan(T v) {
    const uint32_t lane = threadIdx.x & 63;
@@ -1354,15 +1493,6 @@ __device__ __forceinline__ void totalsBody(const Src& src, uint32_t pblock, int6
    }
 }
 
-template <typename Src>
-__global__ __launch_bounds__(kPosBlock) void mutationsTotalsKernel(Src src, const unsigned long long* __restrict__ filter_card,
-                                                                   long long sparse_max, int64_t* __restrict__ totals,
-                                                                   uint32_t* __restrict__ n_rows) {
-   if (!sourceActive(src, filter_card, sparse_max)) return;
-   if (blockIdx.x == 0 && threadIdx.x == 0) *n_rows = 0;  // the finalize kernel appends rows after this one
-   totalsBody(src, blockIdx.x, totals);
-}
-
 // LDS of the finalize step, one instance per kernel whichever sources it finalizes
 struct FinalizeShared {
    BlockValues bv;
@@ -1378,7 +1508,7 @@ __device__ inline FinalizeShared& finalizeShared() {
 template <typename Src>
 __device__ __forceinline__ void finalizeBody(const Src& src, uint32_t pblock, const int64_t* __restrict__ totals,
                                              uint32_t n_pblocks, uint64_t filter_card, double min_proportion,
-                                             uint32_t* __restrict__ counts_out, MutationRowDev* __restrict__ rows,
+                                             MutationRowDev* __restrict__ rows,
                                              uint32_t row_capacity, uint32_t* __restrict__ n_rows) {
    FinalizeShared& sh = finalizeShared();
    BlockValues& bv = sh.bv;
@@ -1432,10 +1562,9 @@ __device__ __forceinline__ void finalizeBody(const Src& src, uint32_t pblock, co
    for (uint32_t sym = 0; sym < ns; ++sym) {
       uint32_t v = bv.v[sym][t];
       if (sym == implicit) v += implicit_count;
-      if (counts_out) counts_out[static_cast<size_t>(sym) * L + p] = v;
       if ((col.valid_mask >> sym) & 1u) total += v;
    }
-   if (total != 0 && rows != nullptr) {
+   if (total != 0) {
       const uint32_t thr = min_proportion == 0.0
                               ? 0u
                               : static_cast<uint32_t>(ceil(static_cast<double>(total) * min_proportion) - 1.0);
@@ -1452,13 +1581,177 @@ __device__ __forceinline__ void finalizeBody(const Src& src, uint32_t pblock, co
    }
 }
 
-template <typename Src>
-__global__ __launch_bounds__(kPosBlock) void mutationsFinalizeKernel(
-   Src src, const int64_t* __restrict__ totals, uint32_t n_pblocks, const unsigned long long* __restrict__ filter_card,
-   long long sparse_max, double min_proportion, uint32_t* __restrict__ counts_out, MutationRowDev* __restrict__ rows,
-   uint32_t row_capacity, uint32_t* __restrict__ n_rows) {
-   if (!sourceActive(src, filter_card, sparse_max)) return;
-   finalizeBody(src, blockIdx.x, totals, n_pblocks, *filter_card, min_proportion, counts_out, rows, row_capacity, n_rows);
+// Results of one Mutations query (see MutationsResult).  Work-group b takes kResultPos positions: it sums
+// the counting kernel's parts per slot (or reads the sparse counts) into LDS, turns the boundary
+// quantities into the covered rows of each position with the totals of the blocks before it, and
+// writes its rows in output order into its own place, so that nothing is sorted afterwards, and then a
+// stamp with their number that the host polls for.  It also clears its share of the totals that the
+// next query will use (two sets take turns).
+//
+// Latency-bound (a few dependent loads, 4 to 17 MB of partial sums): 64 positions a work-group put 468
+// of them on the chip where the three kernels this replaces (sum of the parts, totals, finalize: 25 us
+// on 4 M rows, and the launches between them) had 117.  10 us now.  A counter of finished
+// work-groups whose last one told the host took 2 us more than the stamps.
+__global__ __launch_bounds__(kResultThreads) void mutationsResultKernel(const SeqColumnView* __restrict__ colp,
+                                                                        MutationsResult r) {
+   __shared__ uint32_t v[kMaxSymbols][kResultPos];
+   __shared__ uint32_t start[kResultPos], end[kResultPos];
+   __shared__ int32_t runs[kResultPos];
+   __shared__ int64_t part[4][4];
+   __shared__ int64_t scan[3][kResultPos];
+   __shared__ uint32_t stored[kResultPos], valid_sum[kResultPos];
+   __shared__ uint32_t n_of[4][kResultPos];
+   extern __shared__ u32x4 rows[];  // block_rows, when rows are asked for
+   const SeqColumnView& col = *colp;
+   const uint32_t t = threadIdx.x, lane = t & 63, wave = t >> 6;
+   const uint32_t L = col.genome_length, ns = col.n_symbols;
+   const uint32_t block = blockIdx.x, n_blocks = gridDim.x;
+   const uint32_t p0 = block * kResultPos;
+   const uint32_t n_pos = L - p0 < kResultPos ? L - p0 : kResultPos;
+   const unsigned long long card = *r.filter_card;
+   const bool sparse = r.sparse_max >= 0 && card <= static_cast<unsigned long long>(r.sparse_max);
+   // (all of the next set: another column's query may have used more of it)
+   for (uint32_t i = block * kResultThreads + t; i < 3 * kMaxResultBlocks; i += n_blocks * kResultThreads) r.totals_next[i] = 0;
+   // totals of the blocks before this one (a, b, c) and of all (a)
+   int64_t sums[4] = {0, 0, 0, 0};
+   for (uint32_t k = t; k < n_blocks; k += kResultThreads) {
+      const int64_t a = static_cast<int64_t>(r.totals[k]);
+      const int64_t b = static_cast<int64_t>(r.totals[kMaxResultBlocks + k]);
+      const int64_t c = static_cast<int64_t>(r.totals[2 * kMaxResultBlocks + k]);
+      sums[3] += a;
+      if (k < block) {
+         sums[0] += a;
+         sums[1] += b;
+         sums[2] += c;
+      }
+   }
+   if (!sparse) {
+      for (uint32_t i = t; i < ns * kResultPos; i += kResultThreads) (&v[0][0])[i] = 0;
+      if (t < kResultPos) {
+         start[t] = 0;
+         end[t] = 0;
+         runs[t] = 0;
+      }
+      __syncthreads();
+      const GlobalU32* pos_ptr = toGlobal<GlobalU32>(col.pos_slot_ptr);
+      const GlobalU32* info = toGlobal<GlobalU32>(col.slot_info);
+      const GlobalU32* partial = toGlobal<GlobalU32>(r.partial);
+      const uint32_t s0 = pos_ptr[p0], s1 = pos_ptr[p0 + n_pos];
+      for (uint32_t s = s0 + t; s < s1; s += kResultThreads) {
+         const uint32_t x = info[s];
+         uint32_t n = r.heavy ? r.heavy[s] : 0u;
+         if (r.heavy && n) r.heavy[s] = 0;
+         uint32_t g = 0;
+         for (; g + 6 <= r.n_parts; g += 6) {
+            uint32_t y[6];
+#pragma unroll
+            for (uint32_t u = 0; u < 6; ++u) y[u] = partial[static_cast<size_t>(g + u) * col.n_slots + s];
+#pragma unroll
+            for (uint32_t u = 0; u < 6; ++u) n += y[u];
+         }
+         for (; g < r.n_parts; ++g) n += partial[static_cast<size_t>(g) * col.n_slots + s];
+         const uint32_t p = (x & 0xFFFFu) - p0, sym = x >> 16;
+         if (sym < ns) {
+            v[sym][p] = n;
+         } else if (sym - ns == BND_COV_START) {
+            start[p] = n;
+         } else if (sym - ns == BND_COV_END) {
+            end[p] = n;
+         } else {
+            atomicAdd(&runs[p], sym - ns == BND_N_START ? static_cast<int32_t>(n) : -static_cast<int32_t>(n));
+         }
+      }
+   } else {
+      // the sparse counts, left zero for the next query
+      for (uint32_t i = t; i < (ns + 3) * kResultPos; i += kResultThreads) {
+         const uint32_t k = i / kResultPos, p = i % kResultPos;
+         uint32_t n = 0;
+         if (p < n_pos) {
+            uint32_t* src = k < ns ? r.sparse_counts + static_cast<size_t>(k) * L + p0 + p
+                                   : reinterpret_cast<uint32_t*>(r.sparse_bnd) + static_cast<size_t>(k - ns) * L + p0 + p;
+            n = *src;
+            if (n) *src = 0;
+         }
+         if (k < ns) {
+            v[k][p] = n;
+         } else if (k == ns) {
+            start[p] = n;
+         } else if (k == ns + 1) {
+            end[p] = n;
+         } else {
+            runs[p] = static_cast<int32_t>(n);
+         }
+      }
+   }
+   for (int q = 0; q < 4; ++q) {
+      const int64_t x = waveTotal(sums[q]);
+      if (lane == 0) part[q][wave] = x;
+   }
+   __syncthreads();
+   // boundary prefix sums, one wavefront each, and the positions' symbol sums in the fourth
+   if (wave < 3) {
+      const int64_t x = wave == 0 ? static_cast<int64_t>(start[lane])
+                        : wave == 1 ? static_cast<int64_t>(end[lane])
+                                    : static_cast<int64_t>(runs[lane]);
+      const int64_t before = part[wave][0] + part[wave][1] + part[wave][2] + part[wave][3];
+      scan[wave][lane] = waveInclusiveScan<int64_t>(x) + before;
+   } else {
+      uint32_t all = 0, valid = 0;
+      for (uint32_t sym = 0; sym < ns; ++sym) {
+         const uint32_t n = v[sym][lane];
+         all += n;
+         if ((col.valid_mask >> sym) & 1u) valid += n;
+      }
+      stored[lane] = all;
+      valid_sum[lane] = valid;
+   }
+   __syncthreads();
+   // thread (position lane, quarter of the symbols)
+   const uint32_t p = p0 + lane;
+   const bool have = lane < n_pos;
+   const uint32_t implicit = !have ? 0u : sparse ? col.reference[p] : col.local_ref[p];
+   const uint32_t orig = have ? col.reference[p] : 0u;
+   const int64_t all_starts = part[3][0] + part[3][1] + part[3][2] + part[3][3];
+   // rows covered at p: not starting after p, not ended at or before p, not inside a missing run
+   const int64_t covered = static_cast<int64_t>(card) - (all_starts - scan[0][lane]) - scan[1][lane] - scan[2][lane];
+   const uint32_t implicit_count = card == 0 ? 0u : static_cast<uint32_t>(covered - static_cast<int64_t>(stored[lane]));
+   const uint32_t total = valid_sum[lane] + (((col.valid_mask >> implicit) & 1u) ? implicit_count : 0u);
+   const uint32_t per = (ns + 3) / 4, sym0 = wave * per, sym1 = sym0 + per < ns ? sym0 + per : ns;
+   const auto count = [&](uint32_t sym) { return v[sym][lane] + (sym == implicit ? implicit_count : 0u); };
+   if (r.counts_out != nullptr && have) {
+      for (uint32_t sym = sym0; sym < sym1; ++sym) r.counts_out[static_cast<size_t>(sym) * L + p] = count(sym);
+   }
+   if (r.rows != nullptr) {
+      const uint32_t thr = r.min_proportion == 0.0
+                              ? 0u
+                              : static_cast<uint32_t>(ceil(static_cast<double>(total) * r.min_proportion) - 1.0);
+      const auto listed = [&](uint32_t sym) {
+         return ((col.valid_mask >> sym) & 1u) && sym != orig && count(sym) > thr;
+      };
+      uint32_t n = 0;
+      if (have && total != 0) {
+         for (uint32_t sym = sym0; sym < sym1; ++sym) n += listed(sym) ? 1u : 0u;
+      }
+      n_of[wave][lane] = n;
+      __syncthreads();
+      const uint32_t at_pos = n_of[0][lane] + n_of[1][lane] + n_of[2][lane] + n_of[3][lane];
+      const uint32_t upto = waveInclusiveScan<uint32_t>(at_pos);
+      if (n) {
+         uint32_t o = upto - at_pos;
+         for (uint32_t w = 0; w < wave; ++w) o += n_of[w][lane];
+         for (uint32_t sym = sym0; sym < sym1; ++sym) {
+            if (listed(sym)) rows[o++] = u32x4{p, sym, count(sym), total};
+         }
+      }
+      // the rows leave in order, 1 KiB a wavefront: scattered 8-byte stores took 45 us more for 25 k rows
+      __syncthreads();
+      const uint32_t n_rows = __shfl(upto, 63, 64);
+      u32x4* dst = reinterpret_cast<u32x4*>(r.rows + static_cast<size_t>(block) * r.block_rows);
+      for (uint32_t i = t; i < n_rows; i += kResultThreads) storeHostRow(dst + i, rows[i]);
+      hostStoresDone();
+      __syncthreads();
+      if (t == 0) storeHost(r.stamps + block, n_rows | (static_cast<unsigned long long>(r.stamp) << 32));
+   }
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1506,9 +1799,10 @@ __global__ __launch_bounds__(kMutThreads) __attribute__((amdgpu_waves_per_eu(kCo
    if (b >= col.n_blocks) return;
    const uint32_t e = i % n_dense;
    const uint32_t q = m.lists[e];
-   countBlock<kUnroll, false, kCoop>(col, b, 0, m.n_chunks, 1, m.filters + static_cast<size_t>(q) * m.n_chunks * kChunkWords,
-                       m.chunk_cards + static_cast<size_t>(q) * m.n_chunks, m.partial + static_cast<size_t>(e) * col.n_slots,
-                              fs, cnt, nullptr);
+   countBlock<kUnroll, false, kCoop>(col, b, 0, m.n_chunks, 1, 0, 1,
+                                     m.filters + static_cast<size_t>(q) * m.n_chunks * kChunkWords,
+                                     m.chunk_cards + static_cast<size_t>(q) * m.n_chunks,
+                                     m.partial + static_cast<size_t>(e) * col.n_slots, fs, cnt, nullptr, nullptr);
 }
 
 // ---- shared scan: four dense queries per pass over the index --------------------------------------
@@ -2366,13 +2660,13 @@ __global__ __launch_bounds__(kPosBlock) void mutationsFinalizeBatchKernel(Mutati
    if (y < n_dense) {
       const uint32_t q = m.lists[y];
       finalizeBody(denseSource(m, y, dense_parts), blockIdx.x, m.totals + static_cast<size_t>(y) * n_pblocks * 3,
-                   n_pblocks, m.cards[q], m.min_proportion[q], nullptr, m.rows + static_cast<size_t>(q) * m.row_capacity,
+                   n_pblocks, m.cards[q], m.min_proportion[q], m.rows + static_cast<size_t>(q) * m.row_capacity,
                    m.row_capacity, m.n_rows + q);
    } else if (y - n_dense < m.list_counts[1]) {
       const uint32_t e = y - n_dense;
       const uint32_t q = m.lists[m.max_queries + e];
       finalizeBody(sparseSource(m, e), blockIdx.x, m.totals + (static_cast<size_t>(m.max_queries) + e) * n_pblocks * 3,
-                   n_pblocks, m.cards[q], m.min_proportion[q], nullptr, m.rows + static_cast<size_t>(q) * m.row_capacity,
+                   n_pblocks, m.cards[q], m.min_proportion[q], m.rows + static_cast<size_t>(q) * m.row_capacity,
                    m.row_capacity, m.n_rows + q);
    }
 }
@@ -2742,8 +3036,11 @@ hipError_t launchFill(uint32_t* p, uint32_t value, size_t n, hipStream_t stream)
 
 hipError_t configureFilterKernel(size_t max_lds_bytes) {
    if (max_lds_bytes <= 64 * 1024) return hipSuccess;
-   return hipFuncSetAttribute(reinterpret_cast<const void*>(&filterVmKernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                              static_cast<int>(max_lds_bytes));
+   const hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(&filterVmKernel<false>),
+                                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(max_lds_bytes));
+   if (err != hipSuccess) return err;
+   return hipFuncSetAttribute(reinterpret_cast<const void*>(&filterVmKernel<true>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(max_lds_bytes));
 }
 
 size_t filterLdsBytes(uint32_t depth) {
@@ -2753,27 +3050,46 @@ size_t filterLdsBytes(uint32_t depth) {
                                            kProgCache * sizeof(Instr) + kVmUnitSlices * 64 * sizeof(uint64_t));
 }
 
+namespace {
+// Slices per unit and work-groups of a filter launch over n_items slices: more slices a unit only
+// where the units still outnumber the wavefronts well (a single query needs every slice in
+// parallel); unit_slices divides kSlicesPerChunk
+uint32_t filterUnit(uint32_t n_items) {
+   static_assert(kSlicesPerChunk % kVmUnitSlices == 0, "units stay inside a chunk");
+   return n_items >= kVmUnitSlices * kVmUnitMinUnits ? kVmUnitSlices : n_items >= 2 * kVmUnitMinUnits ? 2u : 1u;
+}
+}  // namespace
+
 hipError_t launchFilter(const TableView& tv, const ProgramDesc* progs, const Instr* instrs, const uint32_t* ranges,
                         uint32_t n_queries, uint32_t depth, uint64_t* out, unsigned long long* cards,
                         uint32_t* chunk_cards, uint32_t max_blocks, hipStream_t stream,
                         const uint32_t* n_queries_dev) {
    const uint32_t n_items = n_queries * tv.n_chunks * kSlicesPerChunk;
    if (n_items == 0) return hipSuccess;
-   // more slices a unit only where the units still outnumber the wavefronts well (a single query
-   // needs every slice in parallel); unit_slices divides kSlicesPerChunk
-   const uint32_t unit = n_items >= kVmUnitSlices * kVmUnitMinUnits ? kVmUnitSlices
-                         : n_items >= 2 * kVmUnitMinUnits           ? 2u
-                                                                    : 1u;
-   static_assert(kSlicesPerChunk % kVmUnitSlices == 0, "units stay inside a chunk");
+   const uint32_t unit = filterUnit(n_items);
    uint32_t blocks = (n_items / unit + kVmWaves - 1) / kVmWaves;
    if (max_blocks && blocks > max_blocks) blocks = max_blocks;
-   hipLaunchKernelGGL(filterVmKernel, dim3(blocks), dim3(kVmThreads), filterLdsBytes(depth), stream, tv, progs,
-                      instrs, ranges, n_items, depth, out, cards, chunk_cards, n_queries_dev, unit);
+   hipLaunchKernelGGL(filterVmKernel<false>, dim3(blocks), dim3(kVmThreads), filterLdsBytes(depth), stream,
+                      NoProgram{}, tv, progs, instrs, ranges, n_items, depth, out, cards, chunk_cards, n_queries_dev,
+                      unit);
+   return hipGetLastError();
+}
+
+hipError_t launchFilterSingle(const TableView& tv, const SingleProgram& program, uint32_t depth, uint64_t* out,
+                              unsigned long long* card, uint32_t* chunk_cards, hipStream_t stream) {
+   const uint32_t n_items = tv.n_chunks * kSlicesPerChunk;
+   if (n_items == 0) return hipErrorInvalidValue;
+   const uint32_t unit = filterUnit(n_items);
+   hipLaunchKernelGGL(filterVmKernel<true>, dim3((n_items / unit + kVmWaves - 1) / kVmWaves), dim3(kVmThreads),
+                      filterLdsBytes(depth), stream, program, tv, static_cast<const ProgramDesc*>(nullptr),
+                      static_cast<const Instr*>(nullptr), static_cast<const uint32_t*>(nullptr), n_items, depth, out, card,
+                      chunk_cards, static_cast<const uint32_t*>(nullptr), unit);
    return hipGetLastError();
 }
 
 hipError_t launchMutations(const MutationsLaunch& m, hipStream_t stream) {
-   if (m.n_groups == 0 || m.n_groups > kMaxGroups) return hipErrorInvalidValue;
+   const uint32_t n_parts = m.n_groups * m.n_splits;
+   if (m.n_groups == 0 || m.n_splits == 0 || n_parts > kMaxGroups) return hipErrorInvalidValue;
    if (m.sparse_max >= 0 && (m.sparse_counts == nullptr || m.sparse_bnd == nullptr)) return hipErrorInvalidValue;
    hipError_t err = hipSuccess;
    const SeqColumnView& h = *m.col_host;
@@ -2781,10 +3097,11 @@ hipError_t launchMutations(const MutationsLaunch& m, hipStream_t stream) {
    // packed counters need at most kPackedMaxChunks chunks per work-group and the heavy sums
    const bool packed = m.heavy_sums != nullptr && (m.n_chunks + m.n_groups - 1) / m.n_groups <= kPackedMaxChunks;
    uint32_t* heavy = packed ? m.heavy_sums : nullptr;
-   const dim3 grid(h.n_blocks, m.n_groups);
+   const dim3 grid(h.n_blocks, n_parts);
 #define RDB_LAUNCH_K1(U, P, C)                                                                                         \
    hipLaunchKernelGGL((mutationsCountKernel<U, P, C>), grid, dim3(kMutThreads), 0, stream, m.col_dev, m.n_chunks,         \
-                      m.n_groups, m.filter, m.filter_chunk_cards, m.filter_card, m.sparse_max, m.partial, heavy)
+                      m.n_groups, m.filter, m.filter_chunk_cards, m.filter_card, m.sparse_max, m.partial, heavy,          \
+                      m.n_splits, m.totals)
 #define RDB_LAUNCH_K1_C(U, P)       \
    if (m.coop) {                    \
       RDB_LAUNCH_K1(U, P, true);    \
@@ -2820,33 +3137,30 @@ hipError_t launchMutations(const MutationsLaunch& m, hipStream_t stream) {
 #undef RDB_LAUNCH_K1
    if ((err = hipGetLastError()) != hipSuccess) return err;
    if (m.count_stop && (err = hipEventRecord(m.count_stop, stream)) != hipSuccess) return err;
-   if ((m.n_groups > 1 || heavy) && h.n_slots > 0) {
-      hipLaunchKernelGGL(reducePartialsKernel, dim3((h.n_slots + 255) / 256), dim3(256), 0, stream, m.partial,
-                         m.n_groups, h.n_slots, m.filter_card, m.sparse_max, heavy);
+   const uint32_t n_words = m.n_chunks * kChunkWords;
+   if (m.sparse_max >= 0 && n_words > 0) {
+      hipLaunchKernelGGL(sparseCountKernel, dim3((n_words + 255) / 256), dim3(256), 0, stream, m.col_dev, m.chunk_sizes,
+                         n_words, m.filter, m.filter_card, m.sparse_max, m.sparse_counts, m.sparse_bnd, m.totals);
       if ((err = hipGetLastError()) != hipSuccess) return err;
    }
-   const uint32_t n_pblocks = (h.genome_length + kPosBlock - 1) / kPosBlock;
-   const SlotSource dense{m.col_dev, m.partial};
-   hipLaunchKernelGGL(mutationsTotalsKernel<SlotSource>, dim3(n_pblocks), dim3(kPosBlock), 0, stream, dense,
-                      m.filter_card, m.sparse_max, m.totals, m.n_rows);
-   if ((err = hipGetLastError()) != hipSuccess) return err;
-   hipLaunchKernelGGL(mutationsFinalizeKernel<SlotSource>, dim3(n_pblocks), dim3(kPosBlock), 0, stream, dense,
-                      m.totals, n_pblocks, m.filter_card, m.sparse_max, m.min_proportion, m.counts_out, m.rows,
-                      m.row_capacity, m.n_rows);
-   if ((err = hipGetLastError()) != hipSuccess) return err;
-   if (m.sparse_max < 0) return hipSuccess;
-   const uint32_t n_words = m.n_chunks * kChunkWords;
-   if (n_words == 0) return hipSuccess;  // no chunks: no rows
-   hipLaunchKernelGGL(sparseCountKernel, dim3((n_words + 255) / 256), dim3(256), 0, stream, m.col_dev, m.chunk_sizes,
-                      n_words, m.filter, m.filter_card, m.sparse_max, m.sparse_counts, m.sparse_bnd);
-   if ((err = hipGetLastError()) != hipSuccess) return err;
-   const SparseSource sparse{m.col_dev, m.sparse_counts, m.sparse_bnd};
-   hipLaunchKernelGGL(mutationsTotalsKernel<SparseSource>, dim3(n_pblocks), dim3(kPosBlock), 0, stream, sparse,
-                      m.filter_card, m.sparse_max, m.totals, m.n_rows);
-   if ((err = hipGetLastError()) != hipSuccess) return err;
-   hipLaunchKernelGGL(mutationsFinalizeKernel<SparseSource>, dim3(n_pblocks), dim3(kPosBlock), 0, stream, sparse,
-                      m.totals, n_pblocks, m.filter_card, m.sparse_max, m.min_proportion, m.counts_out, m.rows,
-                      m.row_capacity, m.n_rows);
+   MutationsResult r;
+   r.partial = m.partial;
+   r.n_parts = n_parts;
+   r.heavy = heavy;
+   r.sparse_counts = m.sparse_counts;
+   r.sparse_bnd = m.sparse_bnd;
+   r.totals = m.totals;
+   r.totals_next = m.totals_next;
+   r.filter_card = m.filter_card;
+   r.sparse_max = m.sparse_max;
+   r.min_proportion = m.min_proportion;
+   r.counts_out = m.counts_out;
+   r.rows = m.rows;
+   r.block_rows = resultBlockRows(h);
+   r.stamps = m.stamps;
+   r.stamp = m.stamp;
+   const size_t lds = m.rows ? r.block_rows * sizeof(MutationRowDev) : 0;
+   hipLaunchKernelGGL(mutationsResultKernel, dim3(resultBlocks(h)), dim3(kResultThreads), lds, stream, m.col_dev, r);
    return hipGetLastError();
 }
 

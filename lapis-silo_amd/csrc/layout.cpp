@@ -269,6 +269,7 @@ void* Context::pinnedBuffer(size_t bytes) {
       pinned = nullptr;
       pinned_bytes = 0;
       hipCheck(hipHostMalloc(&pinned, bytes, hipHostMallocDefault), "pinned allocation");
+      std::memset(pinned, 0, std::min<size_t>(bytes, kMaxResultBlocks * 8));  // no query's stamps
       pinned_bytes = bytes;
    }
    return pinned;
@@ -1102,6 +1103,19 @@ void buildSequenceColumn(Table& t, SeqColumn& col, const uint8_t* is_null, const
    v.group_hdr = static_cast<const uint16_t*>(up(group_hdr.data(), group_hdr.size() * 2));
    v.slot_info = static_cast<const uint32_t*>(up(col.slot_info.data(), col.slot_info.size() * 4));
    v.pos_slot_ptr = static_cast<const uint32_t*>(up(col.pos_slot_ptr.data(), col.pos_slot_ptr.size() * 4));
+   {
+      std::vector<uint32_t> records(L, 0);  // (n_slots is below 2^28: at most 32 per position)
+      for (uint32_t p = 0; p < L; ++p) {
+         for (uint32_t s = col.pos_slot_ptr[p]; s < col.pos_slot_ptr[p + 1]; ++s) {
+            const uint32_t sym = col.slot_info[s] >> 16;
+            if (sym < nsym) continue;
+            if (records[p] == 0) records[p] = s;
+            records[p] |= 1u << (kBoundarySlotBits + sym - nsym);
+         }
+      }
+      col.boundary_slots = DeviceBuffer(records.data(), records.size() * 4);
+      v.boundary_slots = col.boundary_slots.as<uint32_t>();
+   }
    v.local_ref = static_cast<const uint8_t*>(up(col.local_ref.data(), L));
    v.reference = static_cast<const uint8_t*>(up(col.reference.data(), L));
    v.cov = static_cast<const uint32_t*>(up(cov.data(), cov.size() * 4));
@@ -1403,18 +1417,17 @@ void finalizeTable(Table& t) {
    t.view.chunk_sizes = t.chunk_sizes_dev.as<uint32_t>();
    t.view.seq = t.seq_views_dev.as<SeqColumnView>();
    t.view.ints = t.int_views_dev.as<IntColumnView>();
-   uint32_t max_slots = 1, max_L = 1;
-   for (const auto& c : t.seq) {
-      max_slots = std::max(max_slots, c->view.n_slots);
-      max_L = std::max(max_L, c->genome_length);
-   }
+   uint32_t max_slots = 1;
+   for (const auto& c : t.seq) max_slots = std::max(max_slots, c->view.n_slots);
    t.slot_counts = DeviceBuffer(static_cast<size_t>(max_slots) * 4 * kMaxGroups);
    t.heavy_sums = DeviceBuffer(static_cast<size_t>(max_slots) * 4);
    hipCheck(hipMemset(t.heavy_sums.as<void>(), 0, t.heavy_sums.bytes()), "clear heavy sums");
-   t.totals = DeviceBuffer(static_cast<size_t>((max_L + kMutPosBlock - 1) / kMutPosBlock) * 3 * sizeof(int64_t));
-   // at least the 2048 rows the Mutations path copies back in its first transfer
-   t.mut_rows = DeviceBuffer(16 + std::max<size_t>(static_cast<size_t>(max_L) * 32, 2048) * sizeof(MutationRowDev));
-   t.mut_n = DeviceBuffer(64);
+   t.query_state = DeviceBuffer(QueryState::bytes(t.n_chunks));
+   hipCheck(hipMemset(t.query_state.as<void>(), 0, t.query_state.bytes()), "clear query state");
+   // the context's pinned buffer holds the result of any of the columns from now on
+   t.result_bytes = 0;
+   for (const auto& c : t.seq) t.result_bytes = std::max(t.result_bytes, ResultRows::bytes(c->view));
+   t.ctx->pinnedBuffer(t.result_bytes);
    for (auto& c : t.seq) {
       // sparse-path accumulators start (and are left) zero
       const size_t L = c->genome_length;

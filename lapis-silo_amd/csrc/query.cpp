@@ -68,44 +68,70 @@ uint32_t programDepth(const Context& ctx, const Emitter& program) {
    return depth;
 }
 
+bool programInline(const Emitter& program) {
+   return program.code.size() * (sizeof(Instr) / 4) + program.ranges.size() + program.prefetch.size() <= kInlineProgramWords;
+}
+
 void launchProgram(Table& t, const Emitter& program, const uint8_t* dev_blob, uint64_t* words, unsigned long long* card,
-                   uint32_t* chunk_cards) {
+                   uint32_t* chunk_cards, QueryState* state, Mail* mail, uint32_t mail_seq) {
    Context& ctx = *t.ctx;
    const uint32_t depth = programDepth(ctx, program);
-   if (reinterpret_cast<uint8_t*>(chunk_cards) == reinterpret_cast<uint8_t*>(card) + 64) {
-      // the cardinality (64 bytes) directly followed by the per-chunk cardinalities: one clear
-      hipCheck(launchFill(reinterpret_cast<uint32_t*>(card), 0, (64 + 4 * static_cast<size_t>(t.n_chunks)) / 4, ctx.stream),
-               "clear cardinalities");
-   } else {
-      hipCheck(launchFill(reinterpret_cast<uint32_t*>(card), 0, 64 / 4, ctx.stream), "clear cardinality");
-      hipCheck(launchFill(chunk_cards, 0, t.n_chunks, ctx.stream), "clear chunk cardinalities");
+   if (t.n_chunks == 0) {  // no rows: nothing runs
+      hipCheck(launchFill(reinterpret_cast<uint32_t*>(card), 0, 2, ctx.stream), "clear cardinality");
+      return;
    }
+   SingleProgram sp;
+   sp.desc = ProgramDesc{0, static_cast<uint32_t>(program.code.size()), 0, 0, static_cast<uint32_t>(program.ranges.size()),
+                         static_cast<uint32_t>(program.prefetch.size())};
+   sp.staged = nullptr;
+   if (programInline(program)) {
+      uint32_t* at = sp.words;
+      const auto append = [&](const void* src, size_t n_words) {
+         if (n_words) std::memcpy(at, src, n_words * 4);
+         at += n_words;
+      };
+      append(program.code.data(), program.code.size() * (sizeof(Instr) / 4));
+      append(program.ranges.data(), program.ranges.size());
+      append(program.prefetch.data(), program.prefetch.size());
+   } else {
+      sp.staged = reinterpret_cast<const uint32_t*>(dev_blob + sizeof(ProgramDesc));
+   }
+   sp.chunk_counters = state->chunkCounters();
+   sp.total_counter = &state->filter_total;
+   sp.mail = mail;
+   sp.mail_seq = mail_seq;
    if (ctx.profiling) hipCheck(hipEventRecord(ctx.prof_events[2], ctx.stream), "hipEventRecord");
-   hipCheck(launchFilter(t.view, reinterpret_cast<const ProgramDesc*>(dev_blob),
-                         reinterpret_cast<const Instr*>(dev_blob + sizeof(ProgramDesc)),
-                         reinterpret_cast<const uint32_t*>(dev_blob + sizeof(ProgramDesc) + program.code.size() * sizeof(Instr)),
-                         1, depth, words, card, chunk_cards, 0, ctx.stream),
-            "filter kernel");
+   hipCheck(launchFilterSingle(t.view, sp, depth, words, card, chunk_cards, ctx.stream), "filter kernel");
    if (ctx.profiling) {
       hipCheck(hipEventRecord(ctx.prof_events[3], ctx.stream), "hipEventRecord");
       ctx.profileAccumulate(1);
    }
 }
 
-DeviceBitmap runProgram(Table& t, const Emitter& program) {
+DeviceBitmap runProgram(Table& t, const Emitter& program, bool post) {
    Context& ctx = *t.ctx;
    programDepth(ctx, program);
    DeviceBitmap out(&t);
-   const std::vector<uint8_t> blob = programBlob(program);
-   auto* dev = static_cast<uint8_t*>(ctx.stage(blob.data(), blob.size()));
-   launchProgram(t, program, dev, out.words, out.card_dev, out.chunk_cards);
+   const uint8_t* dev = nullptr;
+   if (!programInline(program)) {
+      const std::vector<uint8_t> blob = programBlob(program);
+      dev = static_cast<uint8_t*>(ctx.stage(blob.data(), blob.size()));
+   }
+   launchProgram(t, program, dev, out.words, out.card_dev, out.chunk_cards, t.query_state.as<QueryState>(),
+                 post ? ctx.mail : nullptr, post ? ++ctx.mail_seq : 0);
    return out;
 }
 
-DeviceBitmap Operator::evaluate() const {
+DeviceBitmap Operator::evaluate(bool post) const {
    Emitter e;
    emit(e);
-   return runProgram(*table, e);
+   DeviceBitmap out = runProgram(*table, e, post);
+   if (post) {
+      Context& ctx = *table->ctx;
+      out.card = table->n_chunks == 0 ? 0 : ctx.waitMail(ctx.mail_seq);
+      out.card_known = true;
+   }
+   return out;
 }
 
 // ---- predicates --------------------------------------------------------------------------------

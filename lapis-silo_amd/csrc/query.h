@@ -70,16 +70,20 @@ class Emitter {
    }
 };
 
-// Runs one emitted program over the table.
-DeviceBitmap runProgram(Table& table, const Emitter& program);
+// Runs one emitted program over the table.  `post`: the cardinality is reported to the context's mail
+// (as request ctx.mail_seq), to be waited for at once.
+DeviceBitmap runProgram(Table& table, const Emitter& program, bool post = false);
 // The staged form of one program: its ProgramDesc, instructions, ranges and prefetch codes.
 std::vector<uint8_t> programBlob(const Emitter& program);
 // The operand-stack depth the program needs (errors when it leaves a wrong stack or nests too deep).
 uint32_t programDepth(const Context& ctx, const Emitter& program);
-// Enqueues the filter kernel for a program staged on the device in programBlob's layout; clears
-// and writes the row words, the cardinality (64 bytes) and the per-chunk cardinalities.
+// Whether the program is passed with the filter kernel's arguments; longer ones are staged first.
+bool programInline(const Emitter& program);
+// Enqueues the filter kernel for a program (not inline: staged on the device in programBlob's layout),
+// which writes the row words, the cardinality and the per-chunk cardinalities; `state` (zero, and
+// left zero) has room for n_chunks counters.
 void launchProgram(Table& table, const Emitter& program, const uint8_t* dev_blob, uint64_t* words,
-                   unsigned long long* card, uint32_t* chunk_cards);
+                   unsigned long long* card, uint32_t* chunk_cards, QueryState* state, Mail* mail, uint32_t mail_seq);
 
 // ---- predicates (filter/operators/selection.h:24-166, is_in_covered_region.h) -------------------
 enum class Comparator { EQUALS, LESS, HIGHER, LESS_OR_EQUALS, HIGHER_OR_EQUALS, NOT_EQUALS };
@@ -156,7 +160,7 @@ class Operator {
    virtual std::string toString() const = 0;
    virtual void emit(Emitter& e) const = 0;
    // Operator::evaluate (filter/operators/operator.h:32) on the device.
-   DeviceBitmap evaluate() const;
+   DeviceBitmap evaluate(bool post = false) const;
    // Operator::negate (operator.cpp:23-67).
    static OperatorPtr negate(OperatorPtr&& op);
    Table* table;
