@@ -29,6 +29,7 @@ void Context::init(int dev) {
       (void)hipGetLastError();
       max_lds_bytes = 64 * 1024;
    }
+   hipCheck(configureHistogramKernel(max_lds_bytes), "histogram kernel");
    hipCheck(hipHostMalloc(&stage_host, kStageSlots * kStageSlotBytes, hipHostMallocDefault), "pinned staging");
    stage_dev = DeviceBuffer(kStageSlots * kStageSlotBytes);
    for (auto& e : stage_events) hipCheck(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
@@ -675,10 +676,9 @@ int rdb_bitmap_rows(rdb_bitmap* bitmap, uint32_t* rows, uint64_t capacity, uint6
    return guarded(nullptr, [&] {
       if (!bitmap || !n || !bitmap->b.table) fail(RDB_EINVAL, "null argument");
       std::lock_guard<std::recursive_mutex> lock(bitmap->b.table->ctx->mu);
-      const auto v = bitmap->b.rows();
-      *n = v.size();
-      if (v.size() > capacity) fail(RDB_ENOMEM, "output capacity too small");
-      if (!v.empty()) std::copy(v.begin(), v.end(), rows);
+      *n = bitmap->b.cardinality();
+      if (*n > capacity) fail(RDB_ENOMEM, "output capacity too small");
+      bitmap->b.rowsInto(rows);
    });
 }
 
@@ -1083,19 +1083,13 @@ void aggregateRows(Table& t, const DeviceBitmap& f, const char* dims, std::vecto
                    std::vector<uint64_t>& counts) {
    const std::vector<capi::AggDim> ds = capi::parseDims(t, dims);
    GroupDims gd{};
+   PositionDims pd{};
    for (size_t k = 0; k < ds.size(); ++k) {
       if (ds[k].is_seq) {
          const SeqColumn& col = *ds[k].seq;
          const uint32_t p = ds[k].position;
-         const size_t padded = static_cast<size_t>(t.n_chunks) << 16;
-         if (t.labels_scratch[k].bytes() < padded * 4) t.labels_scratch[k] = DeviceBuffer(padded * 4);
-         const uint32_t blk = col.block_of_pos[p];
-         const uint32_t base = col.block_slot_start[blk];
-         hipCheck(launchSymbolLabels(t.seq_views_dev.as<SeqColumnView>() + ds[k].seq_index, t.chunk_sizes_dev.as<uint32_t>(),
-                                     p, t.n_chunks, blk, col.pos_slot_ptr[p] - base, col.pos_slot_ptr[p + 1] - base,
-                                     t.labels_scratch[k].as<uint32_t>(), t.ctx->stream),
-                  "symbol labels");
-         gd.labels[k] = t.labels_scratch[k].as<uint32_t>();
+         pd.dim[pd.n++] = PositionDim{t.seq_views_dev.as<SeqColumnView>() + ds[k].seq_index, p,
+                                      col.block_slot_start[col.block_of_pos[p]]};
       } else {
          gd.labels[k] = ds[k].dict->labels.as<uint32_t>();
       }
@@ -1109,20 +1103,45 @@ void aggregateRows(Table& t, const DeviceBitmap& f, const char* dims, std::vecto
       return;
    }
    const uint64_t bins = capi::dimStrides(ds, gd.stride);
+   Context& ctx = *t.ctx;
+   const uint32_t n_bins = static_cast<uint32_t>(bins);
+   // up to kKeptBins bins: the table's histogram, zero between queries, whose bins a kernel moves to
+   // pinned memory; more: one of the query's own, cleared and copied back
+   constexpr uint32_t kKeptBins = 1u << 18;
+   static_assert(kKeptBins / kEmitBins <= kStamps, "a stamp per work-group");
+   if (bins <= kKeptBins) {
+      if (t.hist.bytes() == 0) {
+         DeviceBuffer kept(4 * static_cast<size_t>(kKeptBins));
+         hipCheck(launchFill(kept.as<uint32_t>(), 0, kKeptBins, ctx.stream), "clear histogram");
+         t.hist = std::move(kept);
+      }
+      auto* pinned = static_cast<uint8_t*>(ctx.pinnedBuffer(kStampBytes + 4 * bins));
+      auto* stamps = reinterpret_cast<unsigned long long*>(pinned);
+      auto* out = reinterpret_cast<uint32_t*>(pinned + kStampBytes);
+      const uint32_t stamp = ++ctx.mail_seq;
+      hipCheck(launchGroupHistogram(t.n_chunks, f.words, f.chunk_cards, t.chunk_sizes_dev.as<uint32_t>(), gd, pd, n_bins,
+                                    t.hist.as<uint32_t>(), ctx.stream),
+               "group histogram");
+      hipCheck(launchEmitHistogram(n_bins, t.hist.as<uint32_t>(), out, stamps, stamp, ctx.stream), "group counts");
+      waitStamps(ctx, reinterpret_cast<const uint64_t*>(stamps), (n_bins + kEmitBins - 1) / kEmitBins, stamp);
+      decodeHistogram(ds, gd.stride, out, bins, ids, counts);
+      return;
+   }
    const size_t hb = bins * 4;
-   void* hist = t.ctx->pool.get(hb);
+   void* hist = ctx.pool.get(hb);
    std::vector<uint32_t> h(bins);
    try {
-      hipCheck(launchGroupHistogram(t.n_chunks, f.words, f.chunk_cards, gd, static_cast<uint32_t>(bins),
-                                    static_cast<uint32_t*>(hist), t.ctx->stream),
+      hipCheck(launchFill(static_cast<uint32_t*>(hist), 0, bins, ctx.stream), "clear histogram");
+      hipCheck(launchGroupHistogram(t.n_chunks, f.words, f.chunk_cards, t.chunk_sizes_dev.as<uint32_t>(), gd, pd, n_bins,
+                                    static_cast<uint32_t*>(hist), ctx.stream),
                "group histogram");
-      hipCheck(hipMemcpyAsync(h.data(), hist, hb, hipMemcpyDeviceToHost, t.ctx->stream), "copy histogram");
-      hipCheck(hipStreamSynchronize(t.ctx->stream), "synchronize");
+      hipCheck(hipMemcpyAsync(h.data(), hist, hb, hipMemcpyDeviceToHost, ctx.stream), "copy histogram");
+      hipCheck(hipStreamSynchronize(ctx.stream), "synchronize");
    } catch (...) {
-      t.ctx->pool.put(hist, hb);
+      ctx.pool.put(hist, hb);
       throw;
    }
-   t.ctx->pool.put(hist, hb);
+   ctx.pool.put(hist, hb);
    decodeHistogram(ds, gd.stride, h.data(), bins, ids, counts);
 }
 

@@ -302,10 +302,9 @@ struct Table {
    TableView view{};
 
    // per-call scratch (sized at finalize)
-   DeviceBuffer slot_counts, heavy_sums, query_state, labels_scratch[4], hist;
+   DeviceBuffer slot_counts, heavy_sums, query_state, hist;
    uint32_t totals_turn = 0;  // the set of query_state's totals that the next Mutations query uses
    size_t result_bytes = 0;  // pinned host memory of the largest Mutations result (see ResultRows)
-   size_t hist_bins_capacity = 0;
    // lanes of the batched path (created on demand)
    std::vector<std::shared_ptr<BatchLane>> lanes;
    uint64_t job_counter = 0;
@@ -385,7 +384,16 @@ struct DeviceBitmap {
 
    uint64_t cardinality();
    std::vector<uint32_t> rows();
+   // the row ids into out[cardinality()]
+   void rowsInto(uint32_t* out);
 };
+
+// Pinned host memory a kernel writes results to: kStamps stamps (numbers of requests, kernels.h), then the
+// data.
+constexpr size_t kStamps = kMaxResultBlocks;
+constexpr size_t kStampBytes = kStamps * 8;
+// Waits until stamps[0 .. n) all hold `stamp` in their high halves.
+void waitStamps(Context& ctx, const uint64_t* stamps, uint32_t n, uint32_t stamp);
 
 // A Mutations result in pinned host memory as the result kernel writes it: the rows of each block of
 // positions, in output order, at a place of the block's own.
@@ -397,20 +405,14 @@ struct ResultRows {
    ResultRows() = default;
    ResultRows(void* pinned, const SeqColumnView& col)
        : stamps(static_cast<const uint64_t*>(pinned)),
-         rows(reinterpret_cast<const MutationRowDev*>(static_cast<uint8_t*>(pinned) + kMaxResultBlocks * 8)),
+         rows(reinterpret_cast<const MutationRowDev*>(static_cast<uint8_t*>(pinned) + kStampBytes)),
          n_blocks(resultBlocks(col)),
          block_rows(resultBlockRows(col)) {}
    static size_t bytes(const SeqColumnView& col) {
-      return kMaxResultBlocks * 8 + sizeof(MutationRowDev) * resultBlocks(col) * static_cast<size_t>(resultBlockRows(col));
+      return kStampBytes + sizeof(MutationRowDev) * resultBlocks(col) * static_cast<size_t>(resultBlockRows(col));
    }
    uint32_t count(uint32_t b) const { return static_cast<uint32_t>(stamps[b]); }
-   void wait(Context& ctx, uint32_t stamp) const {
-      uint32_t b = 0;  // the first block not seen yet
-      ctx.pollHost([&] {
-         while (b < n_blocks && static_cast<uint32_t>(__atomic_load_n(stamps + b, __ATOMIC_ACQUIRE) >> 32) == stamp) ++b;
-         return b == n_blocks;
-      });
-   }
+   void wait(Context& ctx, uint32_t stamp) const { waitStamps(ctx, stamps, n_blocks, stamp); }
    size_t size() const {
       size_t n = 0;
       for (uint32_t b = 0; b < n_blocks; ++b) n += count(b);

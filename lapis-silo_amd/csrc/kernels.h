@@ -12,8 +12,18 @@ namespace rdb {
 
 struct GroupDims {
    uint32_t n;
-   const uint32_t* labels[4];  // per-row labels, padded row indexing
+   const uint32_t* labels[4];  // per-row labels, padded row indexing; null: a position dimension
    uint32_t stride[4];
+};
+// Symbols at sequence positions as dimensions, in the order of the GroupDims' null labels.
+struct PositionDim {
+   const SeqColumnView* col;
+   uint32_t position;
+   uint32_t slot_base;  // first slot of the position's block
+};
+struct PositionDims {
+   uint32_t n;
+   PositionDim dim[4];
 };
 
 hipError_t launchFill(uint32_t* p, uint32_t value, size_t n, hipStream_t stream);
@@ -230,12 +240,21 @@ hipError_t launchPackRows(const uint32_t* n_queries, uint32_t max_queries, const
                           const unsigned long long* cards, const MutationRowDev* rows, uint32_t row_capacity,
                           uint32_t* header, MutationRowDev* packed, hipStream_t stream);
 
-hipError_t launchSymbolLabels(const SeqColumnView* col_dev, const uint32_t* chunk_sizes, uint32_t position,
-                              uint32_t n_chunks, uint32_t block, uint32_t slot_lo, uint32_t slot_hi, uint32_t* labels,
-                              hipStream_t stream);
-
+// Counts the filter's rows by combined label into hist[n_bins], which must be zero.
 hipError_t launchGroupHistogram(uint32_t n_chunks, const uint64_t* filter, const uint32_t* filter_chunk_cards,
-                                const GroupDims& dims, uint32_t n_bins, uint32_t* hist, hipStream_t stream);
+                                const uint32_t* chunk_sizes, const GroupDims& dims, const PositionDims& positions,
+                                uint32_t n_bins, uint32_t* hist, hipStream_t stream);
+// Lets the histogram kernel hold the labels of four position dimensions.
+hipError_t configureHistogramKernel(size_t max_lds_bytes);
+// Moves a histogram to pinned host memory and clears it; kEmitBins bins per stamp (in its high half).
+constexpr uint32_t kEmitBins = 1024;
+hipError_t launchEmitHistogram(uint32_t n_bins, uint32_t* hist, uint32_t* out, unsigned long long* stamps, uint32_t stamp,
+                               hipStream_t stream);
+
+// The row ids of chunks [chunk0, chunk0 + n_chunks) of a filter, in order, to pinned host memory
+// (16-byte aligned); a stamp per quarter chunk (in its high half), unless stamps is null.
+hipError_t launchRowIds(const uint64_t* words, const uint32_t* chunk_cards, uint32_t chunk0, uint32_t n_chunks, uint32_t* out,
+                        unsigned long long* stamps, uint32_t stamp, hipStream_t stream);
 
 // ---- ingestion (ingest.hip) -------------------------------------------------------------------------
 // Diff of aligned sequences against the reference.  Row i's characters are data[row_ptr[i] ..

@@ -2672,135 +2672,169 @@ __global__ __launch_bounds__(kPosBlock) void mutationsFinalizeBatchKernel(Mutati
 }
 
 // ------------------------------------------------------------------------------------------------
-// Group-by: per-row labels of a sequence position (symbol, missing, or null), then a histogram of
-// combined labels over the filter's rows.
+// Group-by: the combined labels of the filter's rows (dictionary ids, symbols at a sequence position)
+// counted into a histogram.  A work-group of kHistThreads takes a quarter chunk.
 // ------------------------------------------------------------------------------------------------
-__global__ void symbolLabelsKernel(const SeqColumnView* __restrict__ colp, const uint32_t* __restrict__ chunk_sizes,
-                                   uint32_t position, uint32_t n_rows_padded, uint32_t* __restrict__ labels) {
-   const SeqColumnView& col = *colp;
-   const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
-   if (r >= n_rows_padded) return;
-   if ((r & 0xFFFFu) >= chunk_sizes[r >> 16]) {
-      labels[r] = kInvalidId;  // not a row of the table
-      return;
-   }
-   const bool is_null = (col.null_bits[r >> 6] >> (r & 63)) & 1ULL;
-   uint32_t label;
-   if (is_null) {
-      label = col.n_symbols;  // null group
-   } else {
-      const uint32_t c = col.cov[r];
-      bool covered = (c & 0xFFFFu) <= position && position < (c >> 16);
-      if (covered) {
-         for (uint32_t j = col.nrun_ptr[r]; j < col.nrun_ptr[r + 1]; ++j) {
-            const uint32_t x = col.nruns[j];
-            if ((x & 0xFFFFu) <= position && position < (x >> 16)) {
-               covered = false;
-               break;
-            }
-         }
-      }
-      label = covered ? col.local_ref[position] : (col.n_symbols == 16 ? 15u : 27u);
-   }
-   labels[r] = label;
-}
+constexpr uint32_t kHistThreads = 1024;
+constexpr uint32_t kHistRows = kChunkRows / 4;
+constexpr uint32_t kNoLabel = 0xFFu;  // a row outside the table
 
-// One work-group per chunk: rows stored under a symbol at `position` get that symbol.
-__global__ void symbolScatterKernel(const SeqColumnView* __restrict__ colp, uint32_t n_chunks, uint32_t block,
-                                    uint32_t slot_lo, uint32_t slot_hi, uint32_t* __restrict__ labels) {
-   const SeqColumnView& col = *colp;
-   const uint32_t c = blockIdx.x;
-   const uint32_t tile = block * n_chunks + c;
-   const uint32_t slot_base = col.block_slot_start[block];
-   uint32_t* lab = labels + (static_cast<size_t>(c) << 16);
-   for (uint32_t k = col.light_ptr[tile] + threadIdx.x; k < col.light_ptr[tile + 1]; k += blockDim.x) {
-      const uint32_t x = col.light[k];
-      const uint32_t slot = x >> 16;
-      if (slot < slot_lo || slot >= slot_hi) continue;
-      const uint32_t sym = col.slot_info[slot_base + slot] >> 16;
-      if (sym < col.n_symbols) lab[x & 0xFFFFu] = sym;
+// The symbol of every row of quarter `quarter` of chunk c at a sequence position, into lab[kHistRows]:
+// the null group's label, the missing symbol outside the covered range and inside missing runs, the
+// symbol the row is stored under, or the local reference.  Found as a filter's leaves find them: the
+// coverage bounds of the 4096-row slices, the missing-run index and the position's record of its
+// tile's entries, so that a quarter reads a few KB.  (Labels of every row in memory, 4 bytes each, read
+// every row's range and runs and then the whole tile: 55 us on 4 M rows.)
+// All threads of the work-group; ends without a barrier.
+__device__ inline void positionLabels(const PositionDim& d, const uint32_t* __restrict__ chunk_sizes, uint32_t c,
+                                      uint32_t quarter, uint8_t* lab) {
+   const SeqColumnView& col = *d.col;
+   const uint32_t t = threadIdx.x, lane = t & 63, wave = t >> 6;
+   const uint32_t p = d.position;
+   const uint32_t missing = col.n_symbols == 16 ? 15u : 27u;
+   const uint32_t local = col.local_ref[p];
+   const uint32_t row0 = quarter * kHistRows + 16 * t;  // this thread's 16 rows of the chunk
+   // every load that does not wait for another
+   const size_t word = static_cast<size_t>(c) * kChunkWords + (row0 >> 6);
+   const uint64_t never = toGlobal<GlobalU64>(col.cov_never)[word] >> (row0 & 63);
+   const uint64_t null_rows = toGlobal<GlobalU64>(col.null_bits)[word] >> (row0 & 63);
+   const uint32_t bounds = toGlobal<GlobalU32>(col.cov_bounds)[c * kSlicesPerChunk + (row0 >> 12)];
+   const uint32_t size = toGlobal<GlobalU32>(chunk_sizes)[c];
+   const GlobalU32* rec = toGlobal<GlobalU32>(col.pos_ranges) + (static_cast<size_t>(c) * col.genome_length + p) * kPosRecord;
+   uint32_t r[6];
+#pragma unroll
+   for (uint32_t k = 0; k < 6; ++k) r[k] = rec[k];
+   const uint32_t nb = col.n_run_buckets;
+   const uint32_t k_hi = p / kRunBucket;
+   const uint32_t k_lo = p + 1 >= kShortRun ? (p + 1 - kShortRun) / kRunBucket : 0;
+   const uint32_t n_lists = k_hi - k_lo + 2;  // the buckets and the long runs
+   uint32_t run_lo = 0, run_hi = 0;           // wavefront w: list w's runs of this quarter's four slices
+   static_assert(kShortRun / kRunBucket + 2 <= kHistThreads / 64, "a list per wavefront");
+   if (wave < n_lists) {
+      const uint32_t k = wave + 1 < n_lists ? k_lo + wave : nb;
+      const GlobalU32* rp = toGlobal<GlobalU32>(col.run_index_ptr) + (static_cast<size_t>(c) * (nb + 1) + k) * kSlicesPerChunk +
+                            4 * quarter;
+      run_lo = rp[0];
+      run_hi = rp[4];
    }
-   for (uint32_t k = col.group_ptr[tile] + threadIdx.x; k < col.group_ptr[tile + 1]; k += blockDim.x) {
-      const uint32_t hdr = col.group_hdr[k];
-      const uint32_t slot = hdr & 0xFFFu;
-      if (slot < slot_lo || slot >= slot_hi) continue;
-      const uint32_t sym = col.slot_info[slot_base + slot] >> 16;
-      if (sym >= col.n_symbols) continue;
-      for (uint32_t q = 0; q <= (hdr >> 12); ++q) lab[col.groups[static_cast<size_t>(k) * 8 + q]] = sym;
+   const bool inside = (bounds & 0xFFFFu) <= p && p < (bounds >> 16);  // the same in the whole wavefront
+   u32x4 cov[4];
+   if (!inside) {
+      const GlobalU32x4* cv = toGlobal<GlobalU32x4>(col.cov + (static_cast<size_t>(c) << 16) + row0);
+#pragma unroll
+      for (uint32_t k = 0; k < 4; ++k) cov[k] = cv[k];
    }
-   for (uint32_t k = col.heavy_ptr[tile]; k < col.heavy_ptr[tile + 1]; ++k) {
-      const Desc d = col.vert.desc[k];
-      const uint32_t slot = descSlot(d.w0);
-      if (slot < slot_lo || slot >= slot_hi) continue;
-      const uint32_t sym = col.slot_info[slot_base + slot] >> 16;
-      if (sym >= col.n_symbols) continue;
-      const uint32_t type = descType(d.w0), card = descCard(d.w0);
-      if (type == CT_INLINE) {
-         if (threadIdx.x < card) lab[(d.w1 >> (16 * threadIdx.x)) & 0xFFFFu] = sym;
-      } else if (type == CT_ARRAY) {
-         for (uint32_t j = threadIdx.x; j < card; j += blockDim.x) lab[col.vert.arr[d.w1 + j]] = sym;
-      } else if (type == CT_RUN) {
-         for (uint32_t j = 0; j < card; ++j) {
-            const uint32_t x = col.vert.runs[d.w1 + j];
-            const uint32_t st = x & 0xFFFFu, e = st + (x >> 16);
-            for (uint32_t v = st + threadIdx.x; v <= e; v += blockDim.x) lab[v] = sym;
-         }
+   u32x4 out = {0, 0, 0, 0};
+#pragma unroll
+   for (uint32_t k = 0; k < 16; ++k) {
+      uint32_t label;
+      if ((never >> k) & 1u) {
+         label = ((null_rows >> k) & 1u) ? col.n_symbols : missing;
+      } else if (inside) {
+         label = local;
       } else {
-         const uint64_t* bits = col.vert.bits + static_cast<size_t>(d.w1) * kChunkWords;
-         for (uint32_t w = threadIdx.x; w < kChunkWords; w += blockDim.x) {
-            uint64_t x = bits[w];
-            while (x) {
-               lab[w * 64 + __builtin_ctzll(x)] = sym;
-               x &= x - 1;
-            }
+         const uint32_t x = cov[k >> 2][k & 3];
+         label = (x & 0xFFFFu) <= p && p < (x >> 16) ? local : missing;
+      }
+      if (row0 + k >= size) label = kNoLabel;
+      out[k >> 2] |= label << (8 * (k & 3));
+   }
+   reinterpret_cast<u32x4*>(lab)[t] = out;
+   __syncthreads();
+   // rows of the position's missing runs and stored symbols (no row is in both)
+   for (uint32_t k = run_lo + lane; k < run_hi; k += 64) {
+      const uint64_t e = toGlobal<GlobalU64>(col.run_index)[k];
+      const uint32_t a = static_cast<uint32_t>(e >> 16) & 0xFFFFu, b = static_cast<uint32_t>(e >> 32) & 0xFFFFu;
+      if (a <= p && p < b) lab[static_cast<uint32_t>(e) & (kHistRows - 1)] = static_cast<uint8_t>(missing);
+   }
+   const GlobalU32* info = toGlobal<GlobalU32>(col.slot_info) + d.slot_base;
+   const auto put = [&](uint32_t slot, uint32_t row) {  // (boundary slots name no symbol of the row)
+      const uint32_t sym = info[slot] >> 16;
+      if (sym < col.n_symbols && row / kHistRows == quarter) lab[row & (kHistRows - 1)] = static_cast<uint8_t>(sym);
+   };
+   for (uint32_t k = r[0] + t; k < r[1]; k += kHistThreads) {
+      const uint32_t x = toGlobal<GlobalU32>(col.light)[k];
+      put(x >> 16, x & 0xFFFFu);
+   }
+   for (uint32_t k = r[2] + t; k < r[3]; k += kHistThreads) {
+      const uint32_t hdr = toGlobal<GlobalU16>(col.group_hdr)[k];
+      const u32x4 rows = toGlobal<GlobalU32x4>(col.groups)[k];
+#pragma unroll
+      for (uint32_t q = 0; q < 8; ++q) {
+         if (q <= (hdr >> 12)) put(hdr & 0xFFFu, (q & 1u) ? rows[q >> 1] >> 16 : rows[q >> 1] & 0xFFFFu);
+      }
+   }
+   for (uint32_t k = r[4]; k < r[5]; ++k) {
+      const u32x2 w = toGlobal<GlobalU32x2>(col.vert.desc)[k];
+      const uint32_t slot = descSlot(w[0]), type = descType(w[0]), card = descCard(w[0]);
+      const uint32_t sym = info[slot] >> 16;
+      if (sym >= col.n_symbols) continue;
+      if (type == CT_BITSET) {
+         uint32_t x = static_cast<uint32_t>(toGlobal<GlobalU64>(col.vert.bits)[static_cast<size_t>(w[1]) * kChunkWords + (row0 >> 6)] >>
+                                            (row0 & 63)) & 0xFFFFu;
+         for (; x; x &= x - 1) lab[16 * t + static_cast<uint32_t>(__builtin_ctz(x))] = static_cast<uint8_t>(sym);
+      } else if (type == CT_ARRAY) {
+         for (uint32_t j = t; j < card; j += kHistThreads) put(slot, toGlobal<GlobalU16>(col.vert.arr + w[1])[j]);
+      } else if (type == CT_RUN) {
+         for (uint32_t j = wave; j < card; j += kHistThreads / 64) {  // a wavefront per run
+            const uint32_t x = toGlobal<GlobalU32>(col.vert.runs + w[1])[j];
+            const uint32_t lo = quarter * kHistRows, st = x & 0xFFFFu, en = st + (x >> 16);
+            const uint32_t from = st > lo ? st : lo, to = en < lo + kHistRows - 1 ? en : lo + kHistRows - 1;
+            for (uint32_t v = from + lane; v <= to; v += 64) lab[v - lo] = static_cast<uint8_t>(sym);
          }
+      } else if (t < card) {
+         put(slot, (w[1] >> (16 * t)) & 0xFFFFu);
       }
    }
 }
 
-// LDS bins per pass: 16-bit counters, two per word (a work-group counts one quarter chunk, at most
-// 16,384 rows, so a counter cannot overflow)
+// LDS counters of a work-group: up to kHistCopyBins bins, 32-bit counters in several copies, a lane's
+// copy given by its number (the group keys of skewed columns repeat within 64 rows, and LDS atomics on
+// one address serialise; combining equal keys of a wavefront first, one round of ballots per distinct
+// key, took 89 us on 4 M rows).  More bins: one 16-bit counter each (a quarter chunk holds at most
+// 16,384 rows), two per word, in ranges of kHistLdsBins.
+constexpr uint32_t kHistCopyBins = 4096;
+constexpr uint32_t kHistCopyWords = 8192;
+constexpr uint32_t kHistMaxCopies = 16;
 constexpr uint32_t kHistLdsBins = 32768;
 constexpr uint32_t kHistLdsWords = kHistLdsBins / 2;
-
-__device__ inline void histAdd(uint32_t* lh, uint32_t k, uint32_t v) { atomicAdd(&lh[k >> 1], v << ((k & 1u) << 4)); }
-__device__ inline uint32_t histGet(const uint32_t* lh, uint32_t k) { return (lh[k >> 1] >> ((k & 1u) << 4)) & 0xFFFFu; }
-// Bin ranges counted in LDS by separate work-groups; bins beyond the last range go to global atomics.
+// Bin ranges counted in LDS by separate work-groups (or passes); bins beyond the last range go to
+// global atomics.
 constexpr uint32_t kHistRanges = 8;
+static_assert(kHistCopyWords <= kHistLdsWords, "both forms of the counters share their LDS");
 
-// Adds one to LDS counter k for every active lane whose k is not ~0u, lanes holding the same k combined
-// first: one LDS atomic per distinct k of the wavefront instead of one per lane (group keys of
-// skewed columns repeat within 64 rows, and same-address LDS atomics serialise).
-__device__ inline void addCombined(uint32_t* lh, uint32_t k) {
-   uint64_t todo = __ballot(k != ~0u);
-   while (todo) {
-      const uint32_t lead = static_cast<uint32_t>(__builtin_ctzll(todo));
-      const uint32_t lk = __shfl(k, static_cast<int>(lead), 64);
-      const uint64_t same = __ballot(k == lk);
-      if ((threadIdx.x & 63) == lead) histAdd(lh, lk, static_cast<uint32_t>(__popcll(same)));
-      todo &= ~same;
-   }
+__device__ inline uint32_t histCopyStride(uint32_t n_bins) { return n_bins | 1u; }  // odd: copies on other banks
+__device__ inline uint32_t histCopies(uint32_t n_bins) {
+   uint32_t r = kHistMaxCopies;
+   while (r > 1 && r * histCopyStride(n_bins) > kHistCopyWords) r >>= 1;
+   return r;
 }
 
-// Histograms of at most this many bins combine equal keys within a wavefront before counting.
-constexpr uint32_t kHistCombineBins = 4096;
-
-// Rows of one quarter chunk (16,384 rows) of a filter, each visited once: for a sparse quarter by
-// iterating the set bits of its words, for a dense one by walking the rows in order (consecutive
-// threads on consecutive rows, so the label loads coalesce).
 // Bin keys of U rows: the labels of every dimension are loaded together (a load behind a
 // per-row condition would wait for the loads before it); ~0u for a row with a null label.
+// lab: the position dimensions' labels of the quarter, kHistRows each, in dimension order.
 constexpr uint32_t kHistBatch = 8;
-template <uint32_t U>
-__device__ inline void binKeys(const GroupDims& dims, const size_t (&r)[U], uint32_t (&key)[U]) {
+template <bool kPositions, uint32_t U>
+__device__ inline void binKeys(const GroupDims& dims, const uint8_t* lab, size_t row_base, const uint32_t (&r)[U],
+                               uint32_t (&key)[U]) {
    const uint32_t n = dims.n;
-   uint32_t lab[4][U];
+   uint32_t x[4][U];
+   uint32_t at = 0;
 #pragma unroll
    for (uint32_t d = 0; d < 4; ++d) {
       if (d < n) {
-         const GlobalU32* l = toGlobal<GlobalU32>(dims.labels[d]);
+         if (!kPositions || dims.labels[d] != nullptr) {
+            const GlobalU32* l = toGlobal<GlobalU32>(dims.labels[d]) + row_base;
 #pragma unroll
-         for (uint32_t u = 0; u < U; ++u) lab[d][u] = l[r[u]];
+            for (uint32_t u = 0; u < U; ++u) x[d][u] = l[r[u]];
+         } else if constexpr (kPositions) {
+#pragma unroll
+            for (uint32_t u = 0; u < U; ++u) {
+               const uint32_t b = lab[at * kHistRows + r[u]];
+               x[d][u] = b == kNoLabel ? kInvalidId : b;
+            }
+            ++at;
+         }
       }
    }
 #pragma unroll
@@ -2810,99 +2844,142 @@ __device__ inline void binKeys(const GroupDims& dims, const size_t (&r)[U], uint
 #pragma unroll
       for (uint32_t d = 0; d < 4; ++d) {
          if (d < n) {
-            ok &= lab[d][u] != kInvalidId;
-            k += lab[d][u] * dims.stride[d];
+            ok &= x[d][u] != kInvalidId;
+            k += x[d][u] * dims.stride[d];
          }
       }
       key[u] = ok ? k : ~0u;
    }
 }
 
-// Calls count(key) for the rows of a quarter chunk (16,384 rows from row_base) in the filter words f,
-// kHistBatch rows per thread at a time, every lane of a wavefront in every call (key ~0u: no row).
-// Dense quarters (chunk_card > 8192) read consecutive rows on consecutive lanes; sparse ones take
-// the set bits of one filter word per thread.  blockDim.x is 256.
-template <typename Count>
+// Calls count(key) for the rows of a quarter chunk (row_base its first row) in the filter words f,
+// several rows per thread at a time (key ~0u: no row).  Dense quarters (chunk_card > 8192) read
+// consecutive rows on consecutive lanes; sparse ones take the set bits of 16 rows per thread.
+template <bool kPositions, typename Count>
 __device__ inline void histQuarter(const uint64_t* __restrict__ f, uint32_t chunk_card, size_t row_base,
-                                   uint64_t* words_lds, const GroupDims& dims, Count count) {
-   const uint32_t tid = threadIdx.x;
+                                   uint64_t* words_lds, const uint8_t* lab, const GroupDims& dims, Count count) {
+   const uint32_t t = threadIdx.x;
    if (chunk_card > 8192) {
-      words_lds[tid] = f[tid];
+      if (t < 256) words_lds[t] = f[t];
       __syncthreads();
-      for (uint32_t i0 = 0; i0 < 16384; i0 += 256 * kHistBatch) {
-         size_t r[kHistBatch];
-         uint32_t key[kHistBatch];
+#pragma unroll 1
+      for (uint32_t i0 = 0; i0 < kHistRows; i0 += kHistThreads * kHistBatch) {
+         uint32_t r[kHistBatch], key[kHistBatch];
 #pragma unroll
-         for (uint32_t u = 0; u < kHistBatch; ++u) r[u] = row_base + i0 + u * 256 + tid;
-         binKeys(dims, r, key);
+         for (uint32_t u = 0; u < kHistBatch; ++u) r[u] = i0 + u * kHistThreads + t;
+         binKeys<kPositions>(dims, lab, row_base, r, key);
 #pragma unroll
          for (uint32_t u = 0; u < kHistBatch; ++u) {
-            const uint32_t i = i0 + u * 256 + tid;
-            count(((words_lds[i >> 6] >> (i & 63)) & 1ULL) ? key[u] : ~0u);
+            count(((words_lds[r[u] >> 6] >> (r[u] & 63)) & 1ULL) ? key[u] : ~0u);
          }
       }
    } else {
-      uint64_t x = f[tid];
+      constexpr uint32_t kSparseBatch = 4;
+      uint32_t x = static_cast<uint32_t>(toGlobal<GlobalU64>(f)[t >> 2] >> (16 * (t & 3))) & 0xFFFFu;
       while (__ballot(x != 0)) {
-         size_t r[kHistBatch];
-         bool have[kHistBatch];
-         uint32_t key[kHistBatch];
+         uint32_t r[kSparseBatch], key[kSparseBatch];
+         bool have[kSparseBatch];
 #pragma unroll
-         for (uint32_t u = 0; u < kHistBatch; ++u) {
+         for (uint32_t u = 0; u < kSparseBatch; ++u) {
             have[u] = x != 0;
-            const uint32_t bit = have[u] ? static_cast<uint32_t>(__builtin_ctzll(x)) : 0u;
+            r[u] = 16 * t + (have[u] ? static_cast<uint32_t>(__builtin_ctz(x)) : 0u);
             x &= x - 1;
-            r[u] = row_base + tid * 64 + bit;
          }
-         binKeys(dims, r, key);
+         binKeys<kPositions>(dims, lab, row_base, r, key);
 #pragma unroll
-         for (uint32_t u = 0; u < kHistBatch; ++u) count(have[u] ? key[u] : ~0u);
+         for (uint32_t u = 0; u < kSparseBatch; ++u) count(have[u] ? key[u] : ~0u);
       }
    }
 }
 
-// Work-group (chunk quarter, bin range y): labels of up to four dimensions combined with strides
-// into one bin; the rows whose bin falls in [y * kHistLdsBins, (y + 1) * kHistLdsBins) are counted
-// in LDS, and the last range also takes every bin above it with global atomics.
-__global__ __launch_bounds__(256) void groupHistogramKernel(uint32_t n_chunks, const uint64_t* __restrict__ filter,
-                                                            const uint32_t* __restrict__ filter_chunk_cards,
-                                                            GroupDims dims, uint32_t n_bins,
-                                                            uint32_t* __restrict__ hist) {
+// One quarter chunk's rows into hist, bins [lo, lo + kHistLdsBins) counted in LDS; `last` also takes every
+// bin above them, with global atomics.
+template <bool kPositions>
+__device__ inline void histCount(const uint64_t* f, uint32_t chunk_card, size_t row_base, uint64_t* words_lds,
+                                 const uint8_t* lab, const GroupDims& dims, uint32_t n_bins, uint32_t lo, bool last,
+                                 uint32_t* lh, uint32_t* __restrict__ hist) {
+   const uint32_t t = threadIdx.x;
+   if (n_bins <= kHistCopyBins) {
+      const uint32_t copies = histCopies(n_bins), stride = histCopyStride(n_bins);
+      for (uint32_t i = t; i < copies * stride; i += kHistThreads) lh[i] = 0;
+      __syncthreads();
+      uint32_t* mine = lh + (t & (copies - 1)) * stride;
+      histQuarter<kPositions>(f, chunk_card, row_base, words_lds, lab, dims, [&](uint32_t key) {
+         if (key != ~0u) atomicAdd(&mine[key], 1u);
+      });
+      __syncthreads();
+      for (uint32_t i = t; i < n_bins; i += kHistThreads) {
+         uint32_t v = 0;
+         for (uint32_t k = 0; k < copies; ++k) v += lh[k * stride + i];
+         if (v) atomicAdd(&hist[i], v);
+      }
+      return;
+   }
+   const uint32_t span = n_bins - lo < kHistLdsBins ? n_bins - lo : kHistLdsBins;
+   for (uint32_t i = t; i < (span + 1) / 2; i += kHistThreads) lh[i] = 0;
+   __syncthreads();
+   histQuarter<kPositions>(f, chunk_card, row_base, words_lds, lab, dims, [&](uint32_t key) {
+      if (key == ~0u) return;
+      const uint32_t k = key - lo;
+      if (key >= lo && k < kHistLdsBins) {
+         atomicAdd(&lh[k >> 1], 1u << ((k & 1u) << 4));
+      } else if (last && key >= lo + kHistLdsBins) {
+         atomicAdd(&hist[key], 1u);
+      }
+   });
+   __syncthreads();
+   for (uint32_t i = t; i < span; i += kHistThreads) {
+      const uint32_t v = (lh[i >> 1] >> ((i & 1u) << 4)) & 0xFFFFu;
+      if (v) atomicAdd(&hist[lo + i], v);
+   }
+}
+
+// Grid (quarter chunks, bin ranges); dynamic LDS: the position dimensions' labels.
+__global__ __launch_bounds__(kHistThreads) void groupHistogramKernel(uint32_t n_chunks, const uint64_t* __restrict__ filter,
+                                                                     const uint32_t* __restrict__ filter_chunk_cards,
+                                                                     const uint32_t* __restrict__ chunk_sizes,
+                                                                     GroupDims dims, PositionDims positions,
+                                                                     uint32_t n_bins, uint32_t* __restrict__ hist) {
    __shared__ uint32_t lh[kHistLdsWords];
    __shared__ uint64_t words[256];
-   const uint32_t c = blockIdx.x >> 2;
-   const uint32_t quarter = blockIdx.x & 3;
+   extern __shared__ u32x4 labels[];
+   uint8_t* lab = reinterpret_cast<uint8_t*>(labels);
+   const uint32_t c = blockIdx.x >> 2, quarter = blockIdx.x & 3;
    const uint32_t lo = blockIdx.y * kHistLdsBins;
    const uint32_t card = filter_chunk_cards[c];
    if (card == 0 || lo >= n_bins) return;
-   const uint32_t span = n_bins - lo < kHistLdsBins ? n_bins - lo : kHistLdsBins;
-   const bool last = blockIdx.y + 1 == gridDim.y;
-   for (uint32_t i = threadIdx.x; i < (span + 1) / 2; i += blockDim.x) lh[i] = 0;
-   __syncthreads();
-   const uint64_t* f = filter + static_cast<size_t>(c) * kChunkWords + quarter * 256;
-   const bool combine = n_bins <= kHistCombineBins;
-   histQuarter(f, card, (static_cast<size_t>(c) << 16) + quarter * 16384u, words, dims, [&](uint32_t key) {
-      const bool in_table = key != ~0u;
-      const bool here = in_table && key >= lo && key - lo < kHistLdsBins;
-      if (combine) {
-         addCombined(lh, here ? key - lo : ~0u);
-      } else if (here) {
-         histAdd(lh, key - lo, 1u);
-      }
-      if (in_table && last && key >= lo + kHistLdsBins) atomicAdd(&hist[key], 1u);
-   });
-   __syncthreads();
-   for (uint32_t i = threadIdx.x; i < span; i += blockDim.x) {
-      const uint32_t v = histGet(lh, i);
-      if (v) atomicAdd(&hist[lo + i], v);
+   for (uint32_t k = 0; k < positions.n; ++k) {
+      positionLabels(positions.dim[k], chunk_sizes, c, quarter, lab + k * kHistRows);
    }
+   __syncthreads();
+   histCount<true>(filter + static_cast<size_t>(c) * kChunkWords + quarter * 256, card,
+             (static_cast<size_t>(c) << 16) + quarter * kHistRows, words, lab, dims, n_bins, lo,
+             blockIdx.y + 1 == gridDim.y, lh, hist);
+}
+
+// The histogram's bins to pinned host memory, kEmitBins per work-group with a stamp each, and cleared
+// for the next query.
+constexpr uint32_t kEmitThreads = 256;
+__global__ __launch_bounds__(kEmitThreads) void emitHistogramKernel(uint32_t n_bins, uint32_t* __restrict__ hist,
+                                                                    uint32_t* __restrict__ out,
+                                                                    unsigned long long* __restrict__ stamps, uint32_t stamp) {
+   const uint32_t base = blockIdx.x * kEmitBins;
+   for (uint32_t i = base + threadIdx.x; i < base + kEmitBins && i < n_bins; i += kEmitThreads) {
+      const uint32_t v = hist[i];
+      storeHost(out + i, v);
+      if (v) hist[i] = 0;
+   }
+   hostStoresDone();
+   __syncthreads();
+   if (threadIdx.x == 0) storeHost(stamps + blockIdx.x, static_cast<unsigned long long>(stamp) << 32);
 }
 
 // Work-group (quarter chunk, entry e): the rows are counted in passes over bin ranges
 // [z * kHistLdsBins, (z + 1) * kHistLdsBins), each in LDS; the last pass also takes every bin above
 // its range, with global atomics.  The passes run inside the work-group so that the grid (fixed for
 // graph replay) does not grow with the bin count.
-__global__ __launch_bounds__(256) void groupHistogramBatchKernel(AggregateBatch a) {
+// (eight wavefronts per SIMD: two work-groups a CU, as their LDS allows)
+__global__ __launch_bounds__(kHistThreads) __attribute__((amdgpu_waves_per_eu(8))) void groupHistogramBatchKernel(AggregateBatch a) {
    __shared__ uint32_t lh[kHistLdsWords];
    __shared__ uint64_t words[256];
    const uint32_t e = blockIdx.y;
@@ -2913,34 +2990,23 @@ __global__ __launch_bounds__(256) void groupHistogramBatchKernel(AggregateBatch 
    const uint32_t quarter = blockIdx.x & 3;
    const uint32_t card = a.chunk_cards[static_cast<size_t>(q) * a.n_chunks + c];
    if (card == 0 || n_bins == 0) return;
-   const GroupDims dims = a.dims[e];
+   GroupDims dims;  // the same in every lane: kept in scalar registers
+   dims.n = uniform(a.dims[e].n);
+#pragma unroll
+   for (uint32_t d = 0; d < 4; ++d) {
+      const uint64_t l = reinterpret_cast<uint64_t>(a.dims[e].labels[d]);
+      dims.labels[d] = reinterpret_cast<const uint32_t*>(uniform(static_cast<uint32_t>(l)) |
+                                                         (static_cast<uint64_t>(uniform(static_cast<uint32_t>(l >> 32))) << 32));
+      dims.stride[d] = uniform(a.dims[e].stride[d]);
+   }
    uint32_t* hist = a.hist + a.hist_offset[e];
    const uint64_t* f = a.filters + static_cast<size_t>(q) * a.n_chunks * kChunkWords + static_cast<size_t>(c) * kChunkWords +
                        quarter * 256;
-   uint32_t passes = (n_bins + kHistLdsBins - 1) / kHistLdsBins;
+   uint32_t passes = n_bins <= kHistCopyBins ? 1 : (n_bins + kHistLdsBins - 1) / kHistLdsBins;
    passes = passes > kHistRanges ? kHistRanges : passes;
-   const bool combine = n_bins <= kHistCombineBins;
    for (uint32_t z = 0; z < passes; ++z) {
-      const uint32_t lo = z * kHistLdsBins;
-      const uint32_t span = n_bins - lo < kHistLdsBins ? n_bins - lo : kHistLdsBins;
-      const bool last = z + 1 == passes;
-      for (uint32_t i = threadIdx.x; i < (span + 1) / 2; i += blockDim.x) lh[i] = 0;
-      __syncthreads();
-      histQuarter(f, card, (static_cast<size_t>(c) << 16) + quarter * 16384u, words, dims, [&](uint32_t key) {
-         const bool in_table = key != ~0u;
-         const bool here = in_table && key >= lo && key - lo < kHistLdsBins;
-         if (combine) {
-            addCombined(lh, here ? key - lo : ~0u);
-         } else if (here) {
-            histAdd(lh, key - lo, 1u);
-         }
-         if (in_table && last && key >= lo + kHistLdsBins) atomicAdd(&hist[key], 1u);
-      });
-      __syncthreads();
-      for (uint32_t i = threadIdx.x; i < span; i += blockDim.x) {
-         const uint32_t v = histGet(lh, i);
-         if (v) atomicAdd(&hist[lo + i], v);
-      }
+      histCount<false>(f, card, (static_cast<size_t>(c) << 16) + quarter * kHistRows, words, nullptr, dims, n_bins,
+                z * kHistLdsBins, z + 1 == passes, lh, hist);
       __syncthreads();
    }
 }
@@ -2959,6 +3025,60 @@ __global__ __launch_bounds__(256) void compactHistogramKernel(AggregateBatch a) 
       const uint32_t k = atomicAdd(&a.n_rows[q], 1u);
       if (k < a.row_capacity) out[k] = MutationRowDev{i, v, 0, 0};
    }
+}
+
+// The row ids of a filter's words, in order, to pinned host memory: a work-group takes a quarter chunk,
+// finds its place from the chunk cardinalities and the quarter's words before it, gathers its rows'
+// low halves in LDS and stores whole 16-byte pieces (a thread's own rows would leave as scattered
+// 4-byte stores).  chunk0: first chunk of this launch, whose ids start at out[0].
+constexpr uint32_t kRowsThreads = 256;
+__global__ __launch_bounds__(kRowsThreads) void rowIdsKernel(const uint64_t* __restrict__ words,
+                                                             const uint32_t* __restrict__ chunk_cards, uint32_t chunk0,
+                                                             uint32_t* __restrict__ out,
+                                                             unsigned long long* __restrict__ stamps, uint32_t stamp) {
+   __shared__ uint16_t ids[kChunkRows / 4];
+   __shared__ uint32_t part[2][kRowsThreads / 64];
+   const uint32_t t = threadIdx.x, lane = t & 63, wave = t >> 6;
+   const uint32_t c = chunk0 + (blockIdx.x >> 2), quarter = blockIdx.x & 3;
+   const GlobalU64* w = toGlobal<GlobalU64>(words) + static_cast<size_t>(c) * kChunkWords;
+   uint64_t x = w[quarter * 256 + t];
+   uint32_t before = 0;  // rows of the chunks and quarters before
+   for (uint32_t k = chunk0 + t; k < c; k += kRowsThreads) before += chunk_cards[k];
+   for (uint32_t q = 0; q < quarter; ++q) before += static_cast<uint32_t>(__popcll(w[q * 256 + t]));
+   const uint32_t n = static_cast<uint32_t>(__popcll(x));
+   const uint32_t upto = waveInclusiveScan<uint32_t>(n);
+   const uint32_t all_before = waveSumDpp(before);
+   if (lane == 63) {
+      part[0][wave] = upto;
+      part[1][wave] = all_before;
+   }
+   __syncthreads();
+   uint32_t o = upto - n, base = 0, total = 0;
+   for (uint32_t k = 0; k < kRowsThreads / 64; ++k) {
+      o += k < wave ? part[0][k] : 0u;
+      total += part[0][k];
+      base += part[1][k];
+   }
+   for (; x; x &= x - 1) ids[o++] = static_cast<uint16_t>(quarter * 16384u + t * 64 + static_cast<uint32_t>(__builtin_ctzll(x)));
+   __syncthreads();
+   const uint32_t high = c << 16;
+   const uint32_t skew = base & 3u;  // ids of the first piece that are another work-group's
+   const uint32_t n_pieces = total ? (skew + total + 3) / 4 : 0;
+   uint32_t* dst = out + (base - skew);
+   for (uint32_t j = t; j < n_pieces; j += kRowsThreads) {
+      const int32_t i = static_cast<int32_t>(4 * j) - static_cast<int32_t>(skew);  // ids[i .. i + 3]
+      if (i >= 0 && i + 4 <= static_cast<int32_t>(total)) {
+         storeHostRow(reinterpret_cast<u32x4*>(dst) + j, u32x4{high | ids[i], high | ids[i + 1], high | ids[i + 2], high | ids[i + 3]});
+      } else {
+         for (int32_t k = 0; k < 4; ++k) {
+            if (i + k >= 0 && i + k < static_cast<int32_t>(total)) storeHost(dst + 4 * j + k, high | ids[i + k]);
+         }
+      }
+   }
+   if (stamps == nullptr) return;
+   hostStoresDone();
+   __syncthreads();
+   if (t == 0) storeHost(stamps + blockIdx.x, static_cast<unsigned long long>(stamp) << 32);
 }
 
 __global__ void fillCountKernel(uint32_t* __restrict__ p, uint32_t value, const uint32_t* __restrict__ n_dev) {
@@ -3265,7 +3385,7 @@ hipError_t launchAggregateBatch(const AggregateBatch& a, hipStream_t stream) {
    hipError_t err = hipGetLastError();
    if (err != hipSuccess) return err;
    if (a.n_chunks == 0) return hipSuccess;  // no rows: the histograms stay zero
-   hipLaunchKernelGGL(groupHistogramBatchKernel, dim3(a.n_chunks * 4, a.max_entries), dim3(256), 0, stream, a);
+   hipLaunchKernelGGL(groupHistogramBatchKernel, dim3(a.n_chunks * 4, a.max_entries), dim3(kHistThreads), 0, stream, a);
    if ((err = hipGetLastError()) != hipSuccess) return err;
    hipLaunchKernelGGL(compactHistogramKernel, dim3(64, a.max_entries), dim3(256), 0, stream, a);
    return hipGetLastError();
@@ -3280,29 +3400,38 @@ hipError_t launchPackRows(const uint32_t* n_queries, uint32_t max_queries, const
    return hipGetLastError();
 }
 
-hipError_t launchSymbolLabels(const SeqColumnView* col_dev, const uint32_t* chunk_sizes, uint32_t position,
-                              uint32_t n_chunks, uint32_t block, uint32_t slot_lo, uint32_t slot_hi, uint32_t* labels,
-                              hipStream_t stream) {
-   const uint32_t n = n_chunks << 16;
+hipError_t launchGroupHistogram(uint32_t n_chunks, const uint64_t* filter, const uint32_t* filter_chunk_cards,
+                                const uint32_t* chunk_sizes, const GroupDims& dims, const PositionDims& positions,
+                                uint32_t n_bins, uint32_t* hist, hipStream_t stream) {
    if (n_chunks == 0) return hipSuccess;
-   hipLaunchKernelGGL(symbolLabelsKernel, dim3((n + 255) / 256), dim3(256), 0, stream, col_dev, chunk_sizes, position, n,
-                      labels);
-   hipError_t err = hipGetLastError();
-   if (err != hipSuccess) return err;
-   hipLaunchKernelGGL(symbolScatterKernel, dim3(n_chunks), dim3(256), 0, stream, col_dev, n_chunks, block, slot_lo,
-                      slot_hi, labels);
+   uint32_t ranges = n_bins <= kHistCopyBins ? 1 : (n_bins + kHistLdsBins - 1) / kHistLdsBins;
+   ranges = ranges > kHistRanges ? kHistRanges : ranges;
+   hipLaunchKernelGGL(groupHistogramKernel, dim3(n_chunks * 4, ranges), dim3(kHistThreads), positions.n * kHistRows, stream,
+                      n_chunks, filter, filter_chunk_cards, chunk_sizes, dims, positions, n_bins, hist);
    return hipGetLastError();
 }
 
-hipError_t launchGroupHistogram(uint32_t n_chunks, const uint64_t* filter, const uint32_t* filter_chunk_cards,
-                                const GroupDims& dims, uint32_t n_bins, uint32_t* hist, hipStream_t stream) {
-   hipError_t err = launchFill(hist, 0, n_bins, stream);
-   if (err != hipSuccess) return err;
+hipError_t configureHistogramKernel(size_t max_lds_bytes) {
+   // its counters and words, and up to four position dimensions' labels
+   const size_t most = 4 * kHistRows;
+   if (4 * kHistLdsWords + 8 * 256 + most > max_lds_bytes) return hipErrorInvalidValue;
+   return hipFuncSetAttribute(reinterpret_cast<const void*>(&groupHistogramKernel),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(most));
+}
+
+hipError_t launchEmitHistogram(uint32_t n_bins, uint32_t* hist, uint32_t* out, unsigned long long* stamps, uint32_t stamp,
+                               hipStream_t stream) {
+   if (n_bins == 0) return hipErrorInvalidValue;
+   hipLaunchKernelGGL(emitHistogramKernel, dim3((n_bins + kEmitBins - 1) / kEmitBins), dim3(kEmitThreads), 0, stream, n_bins,
+                      hist, out, stamps, stamp);
+   return hipGetLastError();
+}
+
+hipError_t launchRowIds(const uint64_t* words, const uint32_t* chunk_cards, uint32_t chunk0, uint32_t n_chunks, uint32_t* out,
+                        unsigned long long* stamps, uint32_t stamp, hipStream_t stream) {
    if (n_chunks == 0) return hipSuccess;
-   uint32_t ranges = (n_bins + kHistLdsBins - 1) / kHistLdsBins;
-   ranges = ranges == 0 ? 1 : (ranges > kHistRanges ? kHistRanges : ranges);
-   hipLaunchKernelGGL(groupHistogramKernel, dim3(n_chunks * 4, ranges), dim3(256), 0, stream, n_chunks, filter,
-                      filter_chunk_cards, dims, n_bins, hist);
+   hipLaunchKernelGGL(rowIdsKernel, dim3(4 * n_chunks), dim3(kRowsThreads), 0, stream, words, chunk_cards, chunk0, out, stamps,
+                      stamp);
    return hipGetLastError();
 }
 

@@ -269,7 +269,7 @@ void* Context::pinnedBuffer(size_t bytes) {
       pinned = nullptr;
       pinned_bytes = 0;
       hipCheck(hipHostMalloc(&pinned, bytes, hipHostMallocDefault), "pinned allocation");
-      std::memset(pinned, 0, std::min<size_t>(bytes, kMaxResultBlocks * 8));  // no query's stamps
+      std::memset(pinned, 0, std::min<size_t>(bytes, kStampBytes));  // no query's stamps
       pinned_bytes = bytes;
    }
    return pinned;
@@ -1483,19 +1483,58 @@ uint64_t DeviceBitmap::cardinality() {
 }
 
 std::vector<uint32_t> DeviceBitmap::rows() {
-   const size_t n_words = static_cast<size_t>(table->n_chunks) * kChunkWords;
-   std::vector<uint64_t> host(n_words);
-   hipCheck(hipMemcpyAsync(host.data(), words, n_words * 8, hipMemcpyDeviceToHost, table->ctx->stream), "copy bitmap");
-   hipCheck(hipStreamSynchronize(table->ctx->stream), "synchronize");
-   std::vector<uint32_t> out;
-   for (size_t w = 0; w < n_words; ++w) {
-      uint64_t x = host[w];
-      while (x) {
-         out.push_back(static_cast<uint32_t>(w * 64 + static_cast<size_t>(std::countr_zero(x))));
-         x &= x - 1;
-      }
-   }
+   std::vector<uint32_t> out(cardinality());
+   rowsInto(out.data());
    return out;
+}
+
+// Pieces of whole chunks of at most kPieceRows rows go through the context's pinned buffer (a larger one
+// would stay allocated for the sake of rare results).
+void DeviceBitmap::rowsInto(uint32_t* out) {
+   constexpr uint64_t kPieceRows = uint64_t{1} << 22;
+   static_assert(kPieceRows >= kChunkRows, "a chunk fits a piece");
+   const uint64_t n = cardinality();
+   if (n == 0) return;
+   Context& ctx = *table->ctx;
+   std::vector<uint32_t> cards;
+   if (n > kPieceRows) {
+      cards.resize(table->n_chunks);
+      hipCheck(hipMemcpyAsync(cards.data(), chunk_cards, cards.size() * 4, hipMemcpyDeviceToHost, ctx.stream), "copy cardinalities");
+      hipCheck(hipStreamSynchronize(ctx.stream), "synchronize");
+   }
+   auto* pinned = static_cast<uint8_t*>(ctx.pinnedBuffer(kStampBytes + 4 * std::min(n, kPieceRows) + 16));
+   auto* stamps = reinterpret_cast<unsigned long long*>(pinned);
+   auto* ids = reinterpret_cast<uint32_t*>(pinned + kStampBytes);
+   uint32_t c0 = 0;
+   while (c0 < table->n_chunks) {
+      uint32_t c1 = table->n_chunks;
+      uint64_t rows = n;
+      if (!cards.empty()) {
+         c1 = c0;
+         rows = 0;
+         while (c1 < table->n_chunks && rows + cards[c1] <= kPieceRows) rows += cards[c1++];
+      }
+      // a stamp per quarter chunk where the stamps suffice, else a synchronization
+      const bool stamped = 4ULL * (c1 - c0) <= kStamps;
+      const uint32_t stamp = ++ctx.mail_seq;
+      hipCheck(launchRowIds(words, chunk_cards, c0, c1 - c0, ids, stamped ? stamps : nullptr, stamp, ctx.stream), "row ids");
+      if (stamped) {
+         waitStamps(ctx, reinterpret_cast<const uint64_t*>(stamps), 4 * (c1 - c0), stamp);
+      } else {
+         hipCheck(hipStreamSynchronize(ctx.stream), "synchronize");
+      }
+      std::memcpy(out, ids, rows * 4);
+      out += rows;
+      c0 = c1;
+   }
+}
+
+void waitStamps(Context& ctx, const uint64_t* stamps, uint32_t n, uint32_t stamp) {
+   uint32_t k = 0;  // the first stamp not seen yet
+   ctx.pollHost([&] {
+      while (k < n && static_cast<uint32_t>(__atomic_load_n(stamps + k, __ATOMIC_ACQUIRE) >> 32) == stamp) ++k;
+      return k == n;
+   });
 }
 
 }  // namespace rdb
