@@ -60,7 +60,9 @@ __device__ inline void storeHost(T* p, T v) {
    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 __device__ inline void storeHostRow(u32x4* p, u32x4 v) {
-   asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1" : : "v"(p), "v"(v) : "memory");
+   // s_nop 1: two wait states before anything may overwrite the registers of a store of more than 8 bytes,
+   // which the compiler does not keep after inline asm
+   asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" : : "v"(p), "v"(v) : "memory");
 }
 __device__ inline void hostStoresDone() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
