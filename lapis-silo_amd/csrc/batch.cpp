@@ -17,14 +17,14 @@ size_t alignUp(size_t x) { return (x + kAlign - 1) / kAlign * kAlign; }
 
 // Layout of a lane's staged inputs (device and pinned host alike).
 struct ParamsLayout {
-   size_t header = 0;        // u32: n_queries, n_agg, total_bins, pad
+   size_t header = 0;        // u32: n_queries, n_agg, total_bins, long programs
    size_t is_mutations = 0;  // u32 [max_queries]
    size_t min_prop = 0;      // f64 [max_queries]
    size_t agg_query = 0;     // u32 [max_queries]
    size_t agg_bins = 0;      // u32 [max_queries]
    size_t agg_offset = 0;    // u32 [max_queries]
    size_t dims = 0;          // GroupDims [max_queries]
-   size_t progs = 0;         // ProgramDesc [max_queries]
+   size_t progs = 0;         // ProgramDesc [max_queries], longest program first
    size_t instrs = 0;        // Instr [instr_capacity]
    size_t ranges = 0;        // u32 [range_capacity]
    size_t bytes = 0;
@@ -152,9 +152,10 @@ void enqueueKernels(Table& t, BatchLane& lane, uint32_t depth, int column, bool 
    auto* cards = lane.cards.as<unsigned long long>();
    auto* chunk_cards = reinterpret_cast<uint32_t*>(lane.cards.as<uint8_t>() + 8ULL * Q);
    hipCheck(launchFill(reinterpret_cast<uint32_t*>(cards), 0, lane.cards.bytes() / 4, lane.stream), "clear cardinalities");
-   hipCheck(launchFilter(t.view, reinterpret_cast<const ProgramDesc*>(pd + pl.progs), reinterpret_cast<const Instr*>(pd + pl.instrs),
-                         reinterpret_cast<const uint32_t*>(pd + pl.ranges), grid_q, depth, lane.filters.as<uint64_t>(), cards,
-                         chunk_cards, static_cast<uint32_t>(ctx.cu_count) * 8, lane.stream, n_queries),
+   hipCheck(launchFilterBatch(t.view, reinterpret_cast<const ProgramDesc*>(pd + pl.progs),
+                              reinterpret_cast<const Instr*>(pd + pl.instrs), reinterpret_cast<const uint32_t*>(pd + pl.ranges),
+                              grid_q, depth, lane.filters.as<uint64_t>(), cards, chunk_cards,
+                              static_cast<uint32_t>(ctx.cu_count) * 32, lane.stream, n_queries),
             "filter kernel");
    if (column >= 0) {
       const SeqColumn& col = *t.seq[column];
@@ -336,7 +337,10 @@ void enqueueJob(Table& t, BatchResult& b, const std::vector<CompiledQuery>& cq, 
    header[0] = n;
    header[1] = n_agg;
    header[2] = total_bins;
-   header[3] = 0;
+   // long programs first: their wavefronts start while there is still other work to run beside them
+   std::stable_sort(progs, progs + n, [](const ProgramDesc& a, const ProgramDesc& b) { return a.n_instr > b.n_instr; });
+   header[3] = static_cast<uint32_t>(
+      std::partition_point(progs, progs + n, [](const ProgramDesc& p) { return p.n_instr >= kVmLongProgram; }) - progs);
    // the header and up to 1 MiB of packed records (the rest, if any, on retirement)
    lane.job_first_bytes = std::min(lane.out_bytes, ol.rows + (size_t{1} << 20));
    try {

@@ -87,9 +87,7 @@ void* Context::stage(const void* host, size_t bytes) {
 }
 
 uint32_t maxFilterDepth(const Context& ctx) {
-   uint32_t d = 1;
-   while (filterLdsBytes(d + 1) <= ctx.max_lds_bytes) ++d;
-   return d;
+   return filterMaxDepth(ctx.max_lds_bytes);
 }
 
 }  // namespace rdb

@@ -37,17 +37,21 @@ constexpr size_t kNoAllocScratchBytes = size_t{128} << 20;
 hipError_t noallocScratch(int device, void** ptr);
 
 size_t filterLdsBytes(uint32_t depth);
+// The deepest operand stack that a program may need.
+uint32_t filterMaxDepth(size_t max_lds_bytes);
 // Lets the filter kernel allocate up to max_lds_bytes of dynamic LDS (deep operator trees).
 hipError_t configureFilterKernel(size_t max_lds_bytes);
 
-// Evaluates n_queries programs over every (chunk, 4096-row slice) of the table (when n_queries_dev
-// is set, the number of programs is read from it and n_queries only sizes the grid).  Output words of
-// query q start at out + q * n_chunks * 1024; cards[q] and chunk_cards[q * n_chunks + c] must be
-// zero on entry and receive the popcounts.
-hipError_t launchFilter(const TableView& tv, const ProgramDesc* progs, const Instr* instrs, const uint32_t* ranges,
-                        uint32_t n_queries, uint32_t depth, uint64_t* out, unsigned long long* cards,
-                        uint32_t* chunk_cards, uint32_t max_blocks, hipStream_t stream,
-                        const uint32_t* n_queries_dev = nullptr);
+// Programs of at least this many instructions count as long ones (launchFilterBatch).  A unit's fixed
+// cost, loading its program and leaf records, is about that of two instructions; 16 of them keep it under
+// an eighth where four slices would otherwise share it.  (The longest tree of a batch of 256 has 350
+// instructions of about 1 us: as units of four slices it took as long as the whole rest.)
+constexpr uint32_t kVmLongProgram = 16;
+// Evaluates a batch's programs: header[0] of them, at most max_queries, in order of decreasing length,
+// the first header[3] of them long.  The cardinalities and per-chunk cardinalities start at zero.
+hipError_t launchFilterBatch(const TableView& tv, const ProgramDesc* progs, const Instr* instrs, const uint32_t* ranges,
+                             uint32_t max_queries, uint32_t depth, uint64_t* out, unsigned long long* cards,
+                             uint32_t* chunk_cards, uint32_t max_blocks, hipStream_t stream, const uint32_t* header);
 
 // A value that a kernel leaves for the host in pinned memory: the host polls `seq` for the number of
 // its request.

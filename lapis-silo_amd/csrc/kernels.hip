@@ -5,6 +5,7 @@
 // lane, so ballots over 64 consecutive rows map directly onto a word.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstddef>
 #include <cstdint>
 #include <type_traits>
@@ -199,8 +200,8 @@ __device__ inline uint64_t waveSum64(uint64_t v) {
 
 // ------------------------------------------------------------------------------------------------
 // Filter VM: one wavefront evaluates one program over one (chunk, slice) item; items of several
-// programs (queries) are spread over the grid.  The operand stack lives in LDS, one 64-word row
-// slice per entry, so any operator tree depth fits that the host sized the launch for.
+// programs (queries) are spread over the grid.  An entry of the operand stack is a 64-word row slice,
+// one word per lane; any operator tree depth fits that the host sized the launch for.
 // ------------------------------------------------------------------------------------------------
 //
 // kSingle: one program, read from the kernel's own arguments (or from `single.staged` when it is too
@@ -209,16 +210,32 @@ __device__ inline uint64_t waveSum64(uint64_t v) {
 // follows.  A count over 100 k rows is then one launch: 42 us with the copy, the clear and the copy
 // back (each 3 to 11 us on the stream), 16 us without.
 struct NoProgram {};
+// The operand stack: its first kVmRegStack entries in registers (picked by the register index mode: an
+// entry's number is the same in every lane), the deeper ones in LDS.  The wavefronts wait for memory
+// half of the time, so more of them help: a stack in LDS takes 512 bytes an entry and wavefront and
+// left room for two work-groups a CU at the 17 to 24 entries that a batch of deep trees needs; with
+// 15 entries in registers it is four.  256 trees over 1 M rows (4,849 leaves): 1,965 us; with the longest
+// programs first and cut finest 1,211; with the stack in registers too 928; with a top entry of its own
+// and counters that stop at the last carry 868 (1,183 with all of that and the stack in LDS).  Seven
+// entries at five wavefronts per SIMD: 1,040.  An entry past the last goes to a register nobody reads, so
+// that the write is unconditional (a conditional one makes the compiler copy all registers).
+constexpr uint32_t kVmRegStack = 15;
+constexpr uint32_t kPlaneGroup = 12;  // planes of a bit-sliced column loaded together (a date has ten or eleven)
+typedef uint64_t VmRegs __attribute__((ext_vector_type(kVmRegStack + 1)));
+__host__ __device__ constexpr size_t vmWaveLdsBytes(uint32_t depth) {
+   return ((depth > kVmRegStack ? depth - kVmRegStack : 0) + 1) * 64 * sizeof(uint64_t) + kPrefetchSlots * 8 * sizeof(uint32_t) +
+          kProgCache * sizeof(Instr);
+}
 template <bool kSingle>
-__global__ __launch_bounds__(kVmThreads) void filterVmKernel(std::conditional_t<kSingle, SingleProgram, NoProgram> single,
+__global__ __launch_bounds__(kVmThreads, 4) void filterVmKernel(std::conditional_t<kSingle, SingleProgram, NoProgram> single,
                                                              TableView tv, const ProgramDesc* __restrict__ progs,
                                                              const Instr* __restrict__ instrs,
-                                                             const uint32_t* __restrict__ ranges, uint32_t n_items,
-                                                             uint32_t depth, uint64_t* __restrict__ out,
+                                                             const uint32_t* __restrict__ ranges, uint32_t depth,
+                                                             uint64_t* __restrict__ out,
                                                              unsigned long long* __restrict__ cards,
                                                              uint32_t* __restrict__ chunk_cards,
-                                                             const uint32_t* __restrict__ n_queries_dev,
-                                                             uint32_t unit_slices) {
+                                                             const uint32_t* __restrict__ batch_header,
+                                                             uint32_t light_slices) {
    extern __shared__ uint64_t lds[];
    if constexpr (kSingle) {
       // the program's words: in this kernel's argument segment, whose first argument `single` is
@@ -232,26 +249,34 @@ __global__ __launch_bounds__(kVmThreads) void filterVmKernel(std::conditional_t<
    }
    const uint32_t wave = threadIdx.x >> 6;
    const uint32_t lane = threadIdx.x & 63;
-   uint64_t* stack = lds + static_cast<size_t>(wave) * (depth + 1) * 64;
-   uint64_t* scratch = stack + static_cast<size_t>(depth) * 64;
-   uint32_t* pf = reinterpret_cast<uint32_t*>(lds + static_cast<size_t>(kVmWaves) * (depth + 1) * 64) +
-                  static_cast<size_t>(wave) * kPrefetchSlots * 8;
-   u32x4* prog = reinterpret_cast<u32x4*>(lds + static_cast<size_t>(kVmWaves) * (depth + 1) * 64 +
-                                          static_cast<size_t>(kVmWaves) * kPrefetchSlots * 4) +
-                 static_cast<size_t>(wave) * kProgCache * 2;
-   // the unit's result words, stored together after its last slice (a store before a later load
-   // would make that load's wait include the store)
-   uint64_t* res = lds + static_cast<size_t>(kVmWaves) * ((depth + 1) * 64 + kPrefetchSlots * 4 + kProgCache * 4) +
-                   static_cast<size_t>(wave) * kVmUnitSlices * 64;
+   // per wavefront: the stack's entries past the register ones, scratch words, the prefetched leaf
+   // records, the cached instructions
+   const uint32_t n_deep = depth > kVmRegStack ? depth - kVmRegStack : 0;
+   uint8_t* mine = reinterpret_cast<uint8_t*>(lds) + wave * vmWaveLdsBytes(depth);
+   uint64_t* deep = reinterpret_cast<uint64_t*>(mine);
+   uint64_t* scratch = deep + n_deep * 64;
+   uint32_t* pf = reinterpret_cast<uint32_t*>(scratch + 64);
+   u32x4* prog = reinterpret_cast<u32x4*>(pf + kPrefetchSlots * 8);
+   VmRegs regs = 0;
+   uint64_t res[kVmUnitSlices] = {};  // the unit's result words, stored together after its last slice (a store
+                                      // before a later load would make that load's wait include the store)
    const uint32_t n_chunks = tv.n_chunks;
    const uint32_t per_query = n_chunks * kSlicesPerChunk;
-   if (n_queries_dev) n_items = uniform(*n_queries_dev * per_query);
-   // A wavefront takes units of unit_slices (1, 2 or 4) consecutive slices of one (program, chunk):
-   // the program (its first kProgCache instructions) and the leaf records are loaded into LDS once
-   // per unit, so that an instruction costs an LDS read instead of a memory round trip.
-   const uint32_t n_units = n_items / unit_slices;
+   // A wavefront takes units of consecutive slices of one (program, chunk): the program (its first
+   // kProgCache instructions) and the leaf records are loaded into LDS once per unit, so that an
+   // instruction costs an LDS read instead of a memory round trip.  A batch's programs come longest
+   // first; its n_long programs of at least kVmLongProgram instructions are cut into units of one slice,
+   // the others into units of light_slices (1, 2 or 4).
+   uint32_t n_programs = 1, n_long = 0;
+   if constexpr (!kSingle) {
+      n_programs = uniform(batch_header[0]);
+      n_long = uniform(batch_header[3]);
+   }
+   const uint32_t long_units = n_long * per_query;
+   const uint32_t n_units = long_units + (n_programs - n_long) * per_query / light_slices;
    for (uint32_t unit = uniform(blockIdx.x * kVmWaves + wave); unit < n_units; unit += gridDim.x * kVmWaves) {
-   const uint32_t unit_item = unit * unit_slices;
+   const uint32_t unit_slices = unit < long_units ? 1u : light_slices;
+   const uint32_t unit_item = unit < long_units ? unit : long_units + (unit - long_units) * light_slices;
    const uint32_t qi = unit_item / per_query;
    const uint32_t chunk = (unit_item - qi * per_query) / kSlicesPerChunk;
    ProgramDesc pd;
@@ -302,13 +327,23 @@ __global__ __launch_bounds__(kVmThreads) void filterVmKernel(std::conditional_t<
       const uint64_t lmask = layoutMask(chunk_size, my_word);
       const size_t row_base = (static_cast<size_t>(chunk) << 16) + slice * 4096u;
       uint32_t sp = 0;
-      auto push = [&](uint64_t v) {
-         stack[sp * 64 + lane] = v;
-         ++sp;
+      // entry k of the stack (k is the same in every lane)
+      auto at = [&](uint32_t k) -> uint64_t { return k < kVmRegStack ? regs[k] : deep[(k - kVmRegStack) * 64 + lane]; };
+      auto put = [&](uint32_t k, uint64_t v) {
+         regs[k < kVmRegStack ? k : kVmRegStack] = v;
+         if (k >= kVmRegStack) deep[(k - kVmRegStack) * 64 + lane] = v;
       };
-      auto pop = [&]() -> uint64_t {
-         --sp;
-         return stack[sp * 64 + lane];
+      // the top entry is `tos` where `held`, else it is in its place like the others
+      uint64_t tos = 0;
+      bool held = false;
+      auto save = [&]() {
+         if (held) put(sp - 1, tos);
+      };
+      auto push = [&](uint64_t v) {
+         save();
+         tos = v;
+         held = true;
+         ++sp;
       };
       // instruction i: from the LDS copy, or (past kProgCache) from memory
       // Instruction i from the LDS copy, a window of kProgCache instructions: a longer program
@@ -457,12 +492,12 @@ __global__ __launch_bounds__(kVmThreads) void filterVmKernel(std::conditional_t<
                if ((cb & 0xFFFFu) <= p && p < (cb >> 16)) {
                   word = ~never;
                } else {
-               for (uint32_t u0 = 0; u0 < 64; u0 += 32) {
-                  uint32_t cs[32];
+               for (uint32_t u0 = 0; u0 < 64; u0 += 16) {
+                  uint32_t cs[16];
 #pragma unroll
-                  for (uint32_t u = 0; u < 32; ++u) cs[u] = cv[(u0 + u) * 64 + lane];
+                  for (uint32_t u = 0; u < 16; ++u) cs[u] = cv[(u0 + u) * 64 + lane];
 #pragma unroll
-                  for (uint32_t u = 0; u < 32; ++u) {
+                  for (uint32_t u = 0; u < 16; ++u) {
                      const uint64_t bw = __ballot((cs[u] & 0xFFFFu) <= p && p < (cs[u] >> 16));
                      if (lane == u0 + u) word = bw;
                   }
@@ -519,30 +554,38 @@ __global__ __launch_bounds__(kVmThreads) void filterVmKernel(std::conditional_t<
                if (np > 0) {
                   // bit-sliced: the lane's word of every plane, then a most-significant-first
                   // comparison of (value - plane_min) with (v - plane_min), rows below and equal
-                  const GlobalU64* pl = toGlobal<GlobalU64>(col.planes) + static_cast<size_t>(chunk) * kChunkWords + my_word;
+                  const GlobalU64* pl = toGlobal<GlobalU64>(col.planes) + static_cast<size_t>(chunk) * kChunkWords;
                   const size_t plane_stride = static_cast<size_t>(n_chunks) * kChunkWords;
-                  uint64_t pw[kMaxIntPlanes];
-#pragma unroll
-                  for (uint32_t p = 0; p < kMaxIntPlanes; ++p) pw[p] = p < np ? pl[p * plane_stride] : 0ull;
-                  auto compareWord = [&](uint32_t cmp, int32_t value) -> uint64_t {
+                  // each comparison's bits below np, and what values outside them decide at once
+                  const auto start = [&](int32_t value, uint32_t& bits, uint64_t& lt, uint64_t& eq) {
                      const int64_t t = static_cast<int64_t>(value) - col.plane_min;
-                     uint64_t lt = 0, eq = 0;
-                     if (t >= (int64_t{1} << np)) {
-                        lt = ~0ull;  // every value is below
-                     } else if (t >= 0) {
-                        eq = ~0ull;
+                     bits = static_cast<uint32_t>(t);
+                     lt = t >= (int64_t{1} << np) ? ~0ull : 0ull;  // every value is below
+                     eq = t >= 0 && lt == 0 ? ~0ull : 0ull;        // t < 0: every value is above
+                  };
+                  uint32_t bits1, bits2;
+                  uint64_t lt1, eq1, lt2, eq2;
+                  start(v, bits1, lt1, eq1);
+                  start(v2, bits2, lt2, eq2);
+                  const auto step = [](uint64_t plane, uint32_t bit, uint64_t& lt, uint64_t& eq) {
+                     const uint64_t set = bit ? ~0ull : 0ull;
+                     lt |= eq & ~plane & set;
+                     eq &= ~(plane ^ set);
+                  };
+                  // kPlaneGroup planes' loads in flight at a time
+                  for (uint32_t top = np; top > 0; top = top > kPlaneGroup ? top - kPlaneGroup : 0) {
+                     uint64_t pw[kPlaneGroup];
 #pragma unroll
-                        for (int p = static_cast<int>(kMaxIntPlanes) - 1; p >= 0; --p) {
-                           if (static_cast<uint32_t>(p) < np) {
-                              if ((t >> p) & 1) {
-                                 lt |= eq & ~pw[p];
-                                 eq &= pw[p];
-                              } else {
-                                 eq &= ~pw[p];
-                              }
-                           }
+                     for (uint32_t u = 0; u < kPlaneGroup; ++u) pw[u] = u < top ? (pl + (top - 1 - u) * plane_stride)[my_word] : 0ull;
+#pragma unroll
+                     for (uint32_t u = 0; u < kPlaneGroup; ++u) {
+                        if (u < top) {
+                           step(pw[u], (bits1 >> (top - 1 - u)) & 1u, lt1, eq1);
+                           if (two) step(pw[u], (bits2 >> (top - 1 - u)) & 1u, lt2, eq2);
                         }
-                     }  // t < 0: every value is above
+                     }
+                  }
+                  const auto select = [](uint32_t cmp, uint64_t lt, uint64_t eq) -> uint64_t {
                      switch (cmp) {
                         case CMP_EQ: return eq;
                         case CMP_LT: return lt;
@@ -552,17 +595,17 @@ __global__ __launch_bounds__(kVmThreads) void filterVmKernel(std::conditional_t<
                         default: return ~eq;
                      }
                   };
-                  word = compareWord(ins.b, v) & (two ? compareWord(ins.e, v2) : ~0ull);
+                  word = select(ins.b, lt1, eq1) & (two ? select(ins.e, lt2, eq2) : ~0ull);
                } else {
                // rows read 64 at a time, consecutive lanes on consecutive rows; the comparison's
                // ballot is the word of those 64 rows, kept by the lane that owns it
                const GlobalU32* vals = toGlobal<GlobalU32>(col.values) + row_base;
-               for (uint32_t u0 = 0; u0 < 64; u0 += 32) {
-                  uint32_t x[32];
+               for (uint32_t u0 = 0; u0 < 64; u0 += 16) {
+                  uint32_t x[16];
 #pragma unroll
-                  for (uint32_t u = 0; u < 32; ++u) x[u] = vals[(u0 + u) * 64 + lane];
+                  for (uint32_t u = 0; u < 16; ++u) x[u] = vals[(u0 + u) * 64 + lane];
 #pragma unroll
-                  for (uint32_t u = 0; u < 32; ++u) {
+                  for (uint32_t u = 0; u < 16; ++u) {
                      const int32_t xv = static_cast<int32_t>(x[u]);
                      const uint64_t bw = __ballot(compareInt(ins.b, xv, v) && (!two || compareInt(ins.e, xv, v2)));
                      if (lane == u0 + u) word = bw;
@@ -588,29 +631,27 @@ __global__ __launch_bounds__(kVmThreads) void filterVmKernel(std::conditional_t<
                push(word);
                break;
             }
-            case OP_AND: {
-               const uint64_t b = pop();
-               const uint64_t a = pop();
-               push(a & b);
+            case OP_AND:
+               --sp;
+               tos = at(sp - 1) & tos;
                break;
-            }
-            case OP_OR: {
-               const uint64_t b = pop();
-               const uint64_t a = pop();
-               push(a | b);
+            case OP_OR:
+               --sp;
+               tos = at(sp - 1) | tos;
                break;
-            }
-            case OP_ANDNOT: {
-               const uint64_t b = pop();
-               const uint64_t a = pop();
-               push(a & ~b);
+            case OP_ANDNOT:
+               --sp;
+               tos = at(sp - 1) & ~tos;
                break;
-            }
             case OP_NOT:
-               push(pop() ^ lmask);
+               tos ^= lmask;
                break;
             case OP_TH_BEGIN:
-               for (uint32_t j = 0; j <= ins.a; ++j) push(0);
+               save();
+               held = false;
+#pragma unroll 1
+               for (uint32_t j = 0; j <= ins.a; ++j) put(sp + j, 0);
+               sp += ins.a + 1;
                break;
             case OP_TH_ADD: {
                // Counting that reproduces Threshold's DP (threshold.cpp:64-138) bit for bit: a row
@@ -618,16 +659,23 @@ __global__ __launch_bounds__(kVmThreads) void filterVmKernel(std::conditional_t<
                // for a negated child) and, once entered, gains one per child through `p` (the
                // child, or the plain set difference for a negated child).  Inside the layout
                // e == p and this is a population count of matching children.
-               const uint64_t x = pop();
+               const uint64_t x = tos;
+               --sp;
+               held = false;
                const uint32_t base = sp - (ins.a + 1);
-               const uint64_t started = stack[base * 64 + lane];
                const uint64_t p = ins.b ? ~x : x;
                const uint64_t e = ins.b ? (x ^ lmask) : x;
+               // a child that no row of the slice matches (most mutations, in most slices) adds nothing, and
+               // the counter's planes end where no row carries on
+               if (__ballot((p | e) != 0ULL) == 0ULL) break;
+               const uint64_t started = at(base);
                uint64_t carry = (started & p) | (~started & e);
-               stack[base * 64 + lane] = started | e;
+               if (__ballot((e & ~started) != 0ULL) != 0ULL) put(base, started | e);
+#pragma unroll 1
                for (uint32_t j = 0; j < ins.a; ++j) {
-                  const uint64_t plane = stack[(base + 1 + j) * 64 + lane];
-                  stack[(base + 1 + j) * 64 + lane] = plane ^ carry;
+                  if (__ballot(carry != 0ULL) == 0ULL) break;
+                  const uint64_t plane = at(base + 1 + j);
+                  put(base + 1 + j, plane ^ carry);
                   carry &= plane;
                }
                break;
@@ -636,7 +684,7 @@ __global__ __launch_bounds__(kVmThreads) void filterVmKernel(std::conditional_t<
                const uint32_t base = sp - (ins.a + 1);
                uint64_t gt = 0, eq = ~0ULL;
                for (int j = static_cast<int>(ins.a) - 1; j >= 0; --j) {
-                  const uint64_t plane = stack[(base + 1 + j) * 64 + lane];
+                  const uint64_t plane = at(base + 1 + j);
                   if ((ins.b >> j) & 1u) {
                      eq &= plane;
                   } else {
@@ -644,8 +692,9 @@ __global__ __launch_bounds__(kVmThreads) void filterVmKernel(std::conditional_t<
                      eq &= ~plane;
                   }
                }
-               sp = base;
-               push(ins.c ? eq : (gt | eq));
+               sp = base + 1;
+               tos = ins.c ? eq : (gt | eq);
+               held = true;
                break;
             }
             case OP_TH_SKIP: {
@@ -656,7 +705,7 @@ __global__ __launch_bounds__(kVmThreads) void filterVmKernel(std::conditional_t<
                   gt = 0;
                   eq = ~0ULL;
                   for (int j = static_cast<int>(ins.b) - 1; j >= 0; --j) {
-                     const uint64_t plane = stack[(base + 1 + j) * 64 + lane];
+                     const uint64_t plane = at(base + 1 + j);
                      if ((k >> j) & 1u) {
                         eq &= plane;
                      } else {
@@ -680,12 +729,12 @@ __global__ __launch_bounds__(kVmThreads) void filterVmKernel(std::conditional_t<
             }
             case OP_SKIP_IF_EMPTY:
                // the slice's partial conjunction is empty: the remaining conjuncts cannot change it
-               if (__ballot(stack[(sp - 1) * 64 + lane] != 0ULL) == 0ULL) {
+               if (__ballot(tos != 0ULL) == 0ULL) {
                   i = ins.a - 1;
                }
                break;
             case OP_SKIP_IF_FULL:
-               if (__ballot(stack[(sp - 1) * 64 + lane] != ~0ULL) == 0ULL) {
+               if (__ballot(tos != ~0ULL) == 0ULL) {
                   i = ins.a - 1;
                }
                break;
@@ -693,13 +742,19 @@ __global__ __launch_bounds__(kVmThreads) void filterVmKernel(std::conditional_t<
                break;
          }
       }
-      const uint64_t result = stack[lane];
-      res[(slice - slice0) * 64 + lane] = result;
+      const uint64_t result = tos;
+#pragma unroll
+      for (uint32_t u = 0; u < kVmUnitSlices; ++u) {
+         if (slice - slice0 == u) res[u] = result;
+      }
       unit_rows += static_cast<uint32_t>(__popcll(result));
    }
    uint64_t* dst = out + static_cast<size_t>(pd.query) * n_chunks * kChunkWords + static_cast<size_t>(chunk) * kChunkWords +
                    slice0 * 64 + lane;
-   for (uint32_t k = 0; k < unit_slices; ++k) dst[k * 64] = res[k * 64 + lane];
+#pragma unroll
+   for (uint32_t u = 0; u < kVmUnitSlices; ++u) {
+      if (u < unit_slices) dst[u * 64] = res[u];
+   }
    const uint32_t n = waveSum(unit_rows);
    if (lane == 0) {
       // A chunk's counter gathers its units' rows in the low 20 bits and their slices above; the
@@ -3165,11 +3220,14 @@ hipError_t configureFilterKernel(size_t max_lds_bytes) {
                               hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(max_lds_bytes));
 }
 
-size_t filterLdsBytes(uint32_t depth) {
-   // per wave: depth stack entries and a scratch entry of 64 words, the prefetched leaf records, the
-   // cached instructions and a unit's result words
-   return static_cast<size_t>(kVmWaves) * ((depth + 1) * 64 * sizeof(uint64_t) + kPrefetchSlots * 8 * sizeof(uint32_t) +
-                                           kProgCache * sizeof(Instr) + kVmUnitSlices * 64 * sizeof(uint64_t));
+size_t filterLdsBytes(uint32_t depth) { return kVmWaves * vmWaveLdsBytes(depth); }
+
+uint32_t filterMaxDepth(size_t max_lds_bytes) {
+   // as deep as if the whole stack were in LDS, beside 6 KiB of a wavefront's own: what programs have
+   // always been accepted up to
+   const size_t entries = (max_lds_bytes / kVmWaves - 6144) / (64 * sizeof(uint64_t));
+   static_assert(kVmWaves * vmWaveLdsBytes(2) <= 64 * 1024, "shallow programs fit the smallest LDS");
+   return std::max<uint32_t>(1, static_cast<uint32_t>(entries) - 1);
 }
 
 namespace {
@@ -3182,18 +3240,15 @@ uint32_t filterUnit(uint32_t n_items) {
 }
 }  // namespace
 
-hipError_t launchFilter(const TableView& tv, const ProgramDesc* progs, const Instr* instrs, const uint32_t* ranges,
-                        uint32_t n_queries, uint32_t depth, uint64_t* out, unsigned long long* cards,
-                        uint32_t* chunk_cards, uint32_t max_blocks, hipStream_t stream,
-                        const uint32_t* n_queries_dev) {
-   const uint32_t n_items = n_queries * tv.n_chunks * kSlicesPerChunk;
+hipError_t launchFilterBatch(const TableView& tv, const ProgramDesc* progs, const Instr* instrs, const uint32_t* ranges,
+                             uint32_t max_queries, uint32_t depth, uint64_t* out, unsigned long long* cards,
+                             uint32_t* chunk_cards, uint32_t max_blocks, hipStream_t stream, const uint32_t* header) {
+   const uint32_t n_items = max_queries * tv.n_chunks * kSlicesPerChunk;
    if (n_items == 0) return hipSuccess;
-   const uint32_t unit = filterUnit(n_items);
-   uint32_t blocks = (n_items / unit + kVmWaves - 1) / kVmWaves;
-   if (max_blocks && blocks > max_blocks) blocks = max_blocks;
+   // a work-group per kVmWaves slices (the most units there can be) up to max_blocks
+   const uint32_t blocks = std::min((n_items + kVmWaves - 1) / kVmWaves, max_blocks);
    hipLaunchKernelGGL(filterVmKernel<false>, dim3(blocks), dim3(kVmThreads), filterLdsBytes(depth), stream,
-                      NoProgram{}, tv, progs, instrs, ranges, n_items, depth, out, cards, chunk_cards, n_queries_dev,
-                      unit);
+                      NoProgram{}, tv, progs, instrs, ranges, depth, out, cards, chunk_cards, header, filterUnit(n_items));
    return hipGetLastError();
 }
 
@@ -3204,7 +3259,7 @@ hipError_t launchFilterSingle(const TableView& tv, const SingleProgram& program,
    const uint32_t unit = filterUnit(n_items);
    hipLaunchKernelGGL(filterVmKernel<true>, dim3((n_items / unit + kVmWaves - 1) / kVmWaves), dim3(kVmThreads),
                       filterLdsBytes(depth), stream, program, tv, static_cast<const ProgramDesc*>(nullptr),
-                      static_cast<const Instr*>(nullptr), static_cast<const uint32_t*>(nullptr), n_items, depth, out, card,
+                      static_cast<const Instr*>(nullptr), static_cast<const uint32_t*>(nullptr), depth, out, card,
                       chunk_cards, static_cast<const uint32_t*>(nullptr), unit);
    return hipGetLastError();
 }

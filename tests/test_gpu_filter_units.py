@@ -1,0 +1,59 @@
+"""Filter programs where the filter kernel's work is cut: stacks around the entries that registers hold
+and deeper, programs around the length that is cut into single slices, counters that carry through every
+plane; alone and in batches of mixed lengths.  Against numpy."""
+import numpy as np
+import pytest
+
+from test_gpu_rows_groups import plain_table
+
+pytestmark = pytest.mark.gpu
+
+
+def leaf(rng, x):
+    lo = int(rng.integers(0, 1000))
+    hi = int(min(999, lo + rng.integers(0, 700)))
+    return f"(int_between x {lo} {hi})", (x >= lo) & (x <= hi)
+
+
+def chain(rng, x, length):
+    """and(leaf, or(leaf, not(and(leaf, ...)))): one stack entry a level."""
+    text, keep = leaf(rng, x)
+    for k in range(length):
+        t, m = leaf(rng, x)
+        if k % 3 == 2:
+            text, keep = f"(not {text})", ~keep
+        if k % 2:
+            text, keep = f"(and {t} {text})", m & keep
+        else:
+            text, keep = f"(or {t} {text})", m | keep
+    return text, keep
+
+
+def nof(rng, x, m, levels, exact):
+    """n of m, whose first child is another one: planes + 1 entries a level."""
+    parts = [nof(rng, x, m, levels - 1, exact) if k == 0 and levels > 1 else leaf(rng, x) for k in range(m)]
+    count = np.sum([p[1] for p in parts], axis=0)
+    n = int(rng.integers(1, m + 1))
+    return f"(nof {n} {int(exact)} " + " ".join(p[0] for p in parts) + ")", count == n if exact else count >= n
+
+
+def programs(rng, x):
+    out = [chain(rng, x, k) for k in (0, 1, 2, 7, 8, 13, 14, 15, 16, 22, 30, 40)]
+    out += [nof(rng, x, m, 1, m % 2 == 0) for m in (2, 3, 7, 8, 15, 16, 20, 33, 70)]
+    out += [nof(rng, x, 20, levels, levels % 2 == 0) for levels in (2, 3, 4)]
+    return out
+
+
+@pytest.mark.parametrize("sizes", [[1], [4096, 65536, 70], [65536] * 9])
+def test_programs(engine, sizes):
+    et, ids, x, _ = plain_table(engine, sizes, seed=len(sizes))
+    try:
+        cases = programs(np.random.default_rng(7), x)
+        for text, keep in cases:
+            assert np.array_equal(et.filter(text), ids[keep]), text
+            assert et.count(text) == int(keep.sum()), text
+        many = cases * 12  # long programs and short ones, more units than wavefronts at nine chunks
+        with et.batch_submit([{"action": "count", "filter": text} for text, _ in many]) as b:
+            assert [b.count(q) for q in range(len(many))] == [int(keep.sum()) for _, keep in many]
+    finally:
+        et.close()
