@@ -73,6 +73,7 @@ void seqBuilderAppend(SeqBuilder& b, const char* data, const uint64_t* row_ptr, 
    const hipStream_t stream = t.ctx->stream;
    try {
       uint64_t a = 0;
+      DeviceBuffer text;
       while (a < n_rows) {
          uint64_t e = a + 1;
          while (e < n_rows && e - a < kPieceRows && row_ptr[e + 1] - row_ptr[a] <= kPieceBytes) ++e;
@@ -83,15 +84,18 @@ void seqBuilderAppend(SeqBuilder& b, const char* data, const uint64_t* row_ptr, 
          std::vector<uint8_t> nulls(n, 0);
          if (is_null) std::copy(is_null + a, is_null + e, nulls.begin());
          DiffBatch d;
-         d.data = upload(bufs, data ? data + row_ptr[a] : nullptr, ptr[n]);
+         if (text.bytes() < ptr[n] + 16) text = DeviceBuffer(ptr[n] + 16);
+         if (ptr[n]) t.ctx->uploadStaged(text.as<void>(), data + row_ptr[a], ptr[n]);
+         d.data = text.as<char>();
          d.row_ptr = upload(bufs, ptr.data(), ptr.size());
          d.offsets = offsets ? upload(bufs, offsets + a, n) : nullptr;
          d.is_null = upload(bufs, nulls.data(), n);
          d.lut = b.lut.as<uint8_t>();
-         d.ref = b.ref.as<uint8_t>();
+         d.ref_text = b.ref_text.as<uint8_t>() + kRefTextPad;
          d.n_rows = n;
          d.length = L;
          d.missing = col.abc->missing;
+         d.missing_char = b.missing_char;
          uint32_t* stats = alloc<uint32_t>(bufs, 5ULL * n);
          d.start = stats;
          d.end = stats + n;
@@ -166,7 +170,7 @@ void seqBuilderFinish(SeqBuilder& b) {
    t.seq.push_back(std::move(b.col));
    b.finished = true;
    b.lut = DeviceBuffer();
-   b.ref = DeviceBuffer();
+   b.ref_text = DeviceBuffer();
 }
 
 // ---- device stages of the index build ------------------------------------------------------------
@@ -206,6 +210,8 @@ void DeviceIndexBuild::adapt(std::vector<uint32_t>& coverage, std::vector<uint8_
    const size_t n_keys = (static_cast<size_t>(L) + 1) * 32;
    a.run_start = alloc<uint32_t>(tmp, n_keys);
    a.run_end = alloc<uint32_t>(tmp, n_keys);
+   a.changes = alloc<int32_t>(tmp, L);
+   a.block_changes = alloc<int32_t>(tmp, L);
    a.coverage = alloc<uint32_t>(tmp, L);
    a.local_ref = alloc<uint8_t>(tmp, L);
    hipCheck(hipMemsetAsync(a.run_start, 0, n_keys * 4, stream), "clear");

@@ -44,7 +44,8 @@ struct SeqBuilder {
    std::vector<uint64_t> mut_ptr{0}, nrun_ptr{0};
    std::vector<uint32_t> mut_pos, nrun_start, nrun_end;
    std::vector<uint8_t> mut_sym;
-   DeviceBuffer lut, ref;
+   DeviceBuffer lut, ref_text;  // (DiffBatch)
+   uint8_t missing_char = 0;
 };
 
 // Diffs n_rows aligned sequences (row i: data[row_ptr[i] .. row_ptr[i + 1]) from position

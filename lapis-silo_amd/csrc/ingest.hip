@@ -16,14 +16,51 @@ namespace {
 
 constexpr uint32_t kDiffWaves = 4;  // rows (one per wavefront) per work-group
 
-__device__ inline uint64_t laneMaskLt(uint32_t lane) { return lane == 0 ? 0ull : (~0ull >> (64 - lane)); }
-
 __device__ inline uint32_t firstBit(uint64_t m) { return static_cast<uint32_t>(__ffsll(static_cast<long long>(m)) - 1); }
 
-// One wavefront per row, 64 consecutive characters per step, classified by ballots.  `j` counts
-// characters of the row, its position is offset + j.  Pass 1 (kWrite false) records the covered
-// range, the number of mutations and internal missing runs and the first illegal character; pass 2
-// writes mutations and runs at the row's offsets.
+// Bits of the bytes of `x` that are not zero, one per byte.
+__device__ inline uint32_t nonzeroBytes(uint32_t x) {
+   const uint32_t high = (((x & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | x) & 0x80808080u;
+   return (high * 0x00204081u) >> 28;  // bits 7, 15, 23 and 31 side by side; no other product reaches them
+}
+__device__ inline uint32_t nonzeroBytes(const uint4& x) {
+   return nonzeroBytes(x.x) | nonzeroBytes(x.y) << 4 | nonzeroBytes(x.z) << 8 | nonzeroBytes(x.w) << 12;
+}
+__device__ inline uint32_t byteOf(const uint4& v, uint32_t k) {
+   const uint32_t lo = k & 4 ? v.y : v.x, hi = k & 4 ? v.w : v.z;
+   return ((k & 8 ? hi : lo) >> (8 * (k & 3))) & 0xFFu;
+}
+// Bits [lo, hi) of 16; bounds outside them are clipped.
+__device__ inline uint32_t bits16(int32_t lo, int32_t hi) {
+   const uint32_t a = static_cast<uint32_t>(min(max(lo, 0), 16)), b = static_cast<uint32_t>(min(max(hi, 0), 16));
+   return ((1u << b) - 1u) & ~((1u << a) - 1u);
+}
+__device__ inline uint32_t waveAdd(uint32_t v) {
+   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+   return v;
+}
+// Sum of v over the lanes below this one; `total` becomes the wavefront's.  Few lanes hold any.
+__device__ inline uint32_t lanesBelow(uint32_t v, uint32_t lane, uint32_t& total) {
+   uint32_t before = 0;
+   total = 0;
+   for (uint64_t some = __ballot(v != 0); some; some &= some - 1) {
+      const uint32_t src = firstBit(some);
+      const uint32_t n = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), static_cast<int>(src)));
+      before += lane > src ? n : 0u;
+      total += n;
+   }
+   return before;
+}
+
+// One wavefront per row, 1,024 characters a step: each lane compares 16 (one aligned load) with the
+// reference's own characters and with the missing character, byte-wise in 32-bit words, and looks up
+// only the bytes that match neither, through the character table.  A row differs from the reference in
+// few places, so a step is two loads and some 60 operations a lane; the count pass is bound by reading
+// the text.  (A character a lane and step, each through the table: 523 us for 8,192 rows of 29,903 and
+// 457 us for the write pass; now KCOUNT and KWRITE.)  `j` counts characters of the row, its position is
+// offset + j.  Pass 1 (kWrite false) records the covered range, the number of mutations and internal
+// missing runs and the first illegal character; pass 2 writes mutations and runs at the row's offsets.
+constexpr uint32_t kDiffStep = 64 * 16;
 template <bool kWrite>
 __global__ __launch_bounds__(64 * kDiffWaves) void diffKernel(DiffBatch d) {
    __shared__ uint8_t lut[256];
@@ -32,7 +69,9 @@ __global__ __launch_bounds__(64 * kDiffWaves) void diffKernel(DiffBatch d) {
    const uint32_t lane = threadIdx.x & 63;
    const uint32_t r = blockIdx.x * kDiffWaves + (threadIdx.x >> 6);
    if (r >= d.n_rows) return;
-   if (d.is_null[r]) {
+   const uint32_t len = static_cast<uint32_t>(d.row_ptr[r + 1] - d.row_ptr[r]);
+   const uint32_t row_start = kWrite ? d.start[r] : 0, row_end = kWrite ? d.end[r] : 0;
+   if (d.is_null[r] || (kWrite && row_start >= row_end)) {
       if (!kWrite && lane == 0) {
          d.start[r] = 0;
          d.end[r] = 0;
@@ -42,54 +81,92 @@ __global__ __launch_bounds__(64 * kDiffWaves) void diffKernel(DiffBatch d) {
       }
       return;
    }
-   const char* s = d.data + d.row_ptr[r];
-   const uint32_t len = static_cast<uint32_t>(d.row_ptr[r + 1] - d.row_ptr[r]);
    const uint32_t off = d.offsets ? d.offsets[r] : 0;
-   const uint8_t* ref = d.ref + off;
-   const uint32_t row_start = kWrite ? d.start[r] : 0, row_end = kWrite ? d.end[r] : 0;
+   // lane k's first 16 characters start at the k-th aligned 16 bytes from the row's first character on
+   const char* s = d.data + d.row_ptr[r];
+   const int32_t skew = static_cast<int32_t>(reinterpret_cast<uintptr_t>(s) & 15);
+   const uint32_t miss_word = d.missing_char * 0x01010101u;
    uint64_t mut_w = kWrite ? d.mut_off[r] : 0, run_sw = kWrite ? d.run_off[r] : 0, run_ew = run_sw;
    uint32_t first = 0xFFFFFFFFu, last = 0, n_mut = 0, n_starts = 0, err = 0xFFFFFFFFu;
-   uint64_t prev_miss = 0;
-   for (uint32_t base = 0; base < len; base += 64) {
-      const uint32_t j = base + lane;
-      const bool valid = j < len;
-      const uint8_t sym = valid ? lut[static_cast<uint8_t>(s[j])] : 0;
-      const bool illegal = valid && sym == 0xFF;
-      const bool miss = valid && sym == d.missing;
-      const bool mut = valid && !illegal && !miss && sym != ref[j];
-      const uint64_t bm = __ballot(miss), bmut = __ballot(mut), bill = __ballot(illegal), bvalid = __ballot(valid);
-      const uint64_t before = (bm << 1) | prev_miss;  // bit k: character k - 1 is missing
-      const uint64_t starts = bm & ~before;
-      const uint64_t nonmiss = bvalid & ~bm & ~bill;
+   uint32_t carry = 0;  // the character before the step's first is missing
+   const int32_t n = static_cast<int32_t>(len);
+   uint4 next_t, next_c;
+   const auto load = [&](int32_t j) {  // (aligned blocks that hold a character of the row, and the reference's there)
+      if (j < n) {
+         next_t = *reinterpret_cast<const uint4*>(s + j);
+         __builtin_memcpy(&next_c, d.ref_text + (static_cast<int32_t>(off) + j), 16);
+      }
+   };
+   next_t = next_c = make_uint4(0, 0, 0, 0);
+   load(static_cast<int32_t>(lane * 16) - skew);
+   for (int32_t base = -skew; base < n; base += static_cast<int32_t>(kDiffStep)) {
+      const int32_t j = base + static_cast<int32_t>(lane * 16);
+      const uint4 t = next_t, c = next_c;
+      load(j + static_cast<int32_t>(kDiffStep));
+      const uint32_t valid = bits16(-j, n - j);
+      uint32_t miss = valid & ~nonzeroBytes(make_uint4(t.x ^ miss_word, t.y ^ miss_word, t.z ^ miss_word, t.w ^ miss_word));
+      const uint32_t other = valid & ~miss & nonzeroBytes(make_uint4(t.x ^ c.x, t.y ^ c.y, t.z ^ c.z, t.w ^ c.w));
+      uint32_t mut = 0, illegal = 0;
+      for (uint32_t rest = other; rest; rest &= rest - 1) {
+         const uint32_t k = firstBit(rest);
+         const uint32_t sym = lut[byteOf(t, k)];
+         const uint32_t bit = 1u << k;
+         if (sym == 0xFFu) {
+            illegal |= bit;
+         } else if (sym == d.missing) {
+            miss |= bit;
+         } else if (sym != lut[byteOf(c, k)]) {
+            mut |= bit;
+         }
+      }
+      const uint32_t prev = __shfl_up(miss >> 15, 1, 64);
+      const uint32_t before = miss << 1 | (lane == 0 ? carry : prev);  // bit k: character k - 1 is missing
+      carry = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(miss >> 15), 63));
+      const uint32_t starts = miss & ~before;
+      const uint32_t nonmiss = valid & ~miss & ~illegal;
       if constexpr (!kWrite) {
-         n_mut += static_cast<uint32_t>(__popcll(bmut));
-         n_starts += static_cast<uint32_t>(__popcll(starts));
+         n_mut += static_cast<uint32_t>(__popc(mut));
+         n_starts += static_cast<uint32_t>(__popc(starts));
          if (nonmiss) {
-            if (first == 0xFFFFFFFFu) first = base + firstBit(nonmiss);
-            last = base + 64 - static_cast<uint32_t>(__clzll(static_cast<long long>(nonmiss)));
+            first = min(first, static_cast<uint32_t>(j + __ffs(static_cast<int>(nonmiss)) - 1));
+            last = static_cast<uint32_t>(j + 32 - __clz(static_cast<int>(nonmiss)));
          }
-         if (bill && err == 0xFFFFFFFFu) err = off + base + firstBit(bill);
+         if (illegal) err = min(err, off + static_cast<uint32_t>(j + __ffs(static_cast<int>(illegal)) - 1));
       } else {
-         const uint32_t p = off + j;
-         if (mut) {
-            const uint64_t o = mut_w + __popcll(bmut & laneMaskLt(lane));
-            d.mut_pos[o] = p;
-            d.mut_sym[o] = sym;
+         const uint32_t p = static_cast<uint32_t>(static_cast<int32_t>(off) + j);
+         uint32_t total;
+         if (__ballot(mut != 0)) {
+            uint64_t o = mut_w + lanesBelow(static_cast<uint32_t>(__popc(mut)), lane, total);
+            mut_w += total;
+            for (uint32_t rest = mut; rest; rest &= rest - 1, ++o) {
+               const uint32_t k = firstBit(rest);
+               d.mut_pos[o] = p + k;
+               d.mut_sym[o] = lut[byteOf(t, k)];
+            }
          }
-         mut_w += __popcll(bmut);
          // internal runs: starts, and ends (the first non-missing character after a run), strictly
          // inside the covered range
-         const uint64_t bin = __ballot(valid && p > row_start && p < row_end);
-         const uint64_t is = starts & bin;
-         const uint64_t ie = nonmiss & before & bin;
-         if ((is >> lane) & 1ull) d.run_start[run_sw + __popcll(is & laneMaskLt(lane))] = p;
-         if ((ie >> lane) & 1ull) d.run_end[run_ew + __popcll(ie & laneMaskLt(lane))] = p;
-         run_sw += __popcll(is);
-         run_ew += __popcll(ie);
+         const int32_t p0 = static_cast<int32_t>(p);
+         const uint32_t inside = bits16(static_cast<int32_t>(row_start) + 1 - p0, static_cast<int32_t>(row_end) - p0);
+         const uint32_t is = starts & inside, ie = nonmiss & before & inside;
+         if (__ballot((is | ie) != 0)) {
+            uint64_t o = run_sw + lanesBelow(static_cast<uint32_t>(__popc(is)), lane, total);
+            run_sw += total;
+            for (uint32_t rest = is; rest; rest &= rest - 1) d.run_start[o++] = p + firstBit(rest);
+            o = run_ew + lanesBelow(static_cast<uint32_t>(__popc(ie)), lane, total);
+            run_ew += total;
+            for (uint32_t rest = ie; rest; rest &= rest - 1) d.run_end[o++] = p + firstBit(rest);
+         }
       }
-      prev_miss = (bm >> 63) & 1ull;
    }
    if constexpr (!kWrite) {
+      n_mut = waveAdd(n_mut);
+      n_starts = waveAdd(n_starts);
+      for (int o = 32; o > 0; o >>= 1) {
+         first = min(first, static_cast<uint32_t>(__shfl_xor(first, o, 64)));
+         last = max(last, static_cast<uint32_t>(__shfl_xor(last, o, 64)));
+         err = min(err, static_cast<uint32_t>(__shfl_xor(err, o, 64)));
+      }
       if (lane == 0) {
          d.err[r] = err;
          if (first == 0xFFFFFFFFu) {  // nothing covered
@@ -141,49 +218,83 @@ __global__ void adaptRunsKernel(const uint32_t* __restrict__ keys, uint64_t n, u
 
 __device__ inline uint32_t adaptCount(const AdaptCount& a, uint32_t key) { return a.run_end[key] - a.run_start[key]; }
 
-// One work-group: coverage[p] = prefix sum of the coverage events; per position the reference
-// symbol's count is the coverage minus the other symbols' counts, and the local reference is the
-// reference symbol unless another symbol's count is strictly larger (the first such symbol with
-// the largest count).
-constexpr uint32_t kAdaptThreads = 1024;
-__global__ __launch_bounds__(kAdaptThreads) void adaptRuleKernel(AdaptCount a) {
-   __shared__ long long part[kAdaptThreads];
+// The adapted local reference, in two kernels over blocks of kRulePositions positions; half a wavefront
+// takes a position, a lane per code, so that a position's 32 counts are one line of each array.  The first
+// leaves each position's change of coverage and each block's sum of them.  The second adds up the blocks
+// before its own and its positions' changes to the coverage; then the reference symbol's count is the
+// coverage minus the other symbols' counts, and the local reference is the reference symbol unless
+// another symbol's count is strictly larger (the first such symbol with the largest count).  (One
+// work-group over all positions, a thread per 30 of them: 1,061 us at 29,903; now 15
+// in both.)
+constexpr uint32_t kRuleThreads = 256;
+constexpr uint32_t kRulePositions = 64;
+constexpr uint32_t kRuleAtOnce = kRuleThreads / 32;
+static_assert(kAdaptCodeDown < 32, "a lane per code");
+
+__global__ __launch_bounds__(kRuleThreads) void adaptChangesKernel(AdaptCount a) {
+   __shared__ int32_t change[kRulePositions];
+   const uint32_t L = a.rows.length;
+   const uint32_t p0 = blockIdx.x * kRulePositions;
+   for (uint32_t k = threadIdx.x / 32; k < kRulePositions; k += kRuleAtOnce) {
+      const uint32_t p = p0 + k, code = threadIdx.x & 31;
+      const bool event = p < L && (code == kAdaptCodeUp || code == kAdaptCodeDown);
+      const int32_t n = event ? static_cast<int32_t>(adaptCount(a, p << 5 | code)) : 0;
+      const int32_t up = __shfl(n, kAdaptCodeUp, 32), down = __shfl(n, kAdaptCodeDown, 32);
+      if (code == 0) {
+         change[k] = up - down;
+         if (p < L) a.changes[p] = up - down;
+      }
+   }
+   __syncthreads();
+   if (threadIdx.x < 64) {
+      int32_t sum = change[threadIdx.x];
+      for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+      if (threadIdx.x == 0) a.block_changes[blockIdx.x] = sum;
+   }
+}
+
+__global__ __launch_bounds__(kRuleThreads) void adaptRuleKernel(AdaptCount a) {
+   static_assert(kRulePositions == 64, "a wavefront scans a block's changes");
+   __shared__ int32_t part[kRuleThreads / 64];
+   __shared__ uint32_t coverage[kRulePositions];
    const DiffRowsDev& R = a.rows;
    const uint32_t L = R.length, nsym = R.n_symbols;
-   const uint32_t per = (L + kAdaptThreads - 1) / kAdaptThreads;
-   const uint32_t lo = min(L, threadIdx.x * per), hi = min(L, lo + per);
-   auto change = [&](uint32_t p) -> long long {
-      return static_cast<long long>(adaptCount(a, p << 5 | kAdaptCodeUp)) -
-             static_cast<long long>(adaptCount(a, p << 5 | kAdaptCodeDown));
-   };
-   long long sum = 0;
-   for (uint32_t p = lo; p < hi; ++p) sum += change(p);
-   part[threadIdx.x] = sum;
+   const uint32_t p0 = blockIdx.x * kRulePositions;
+   int32_t sum = 0;
+   for (uint32_t b = threadIdx.x; b < blockIdx.x; b += kRuleThreads) sum += a.block_changes[b];
+   for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+   if ((threadIdx.x & 63) == 0) part[threadIdx.x / 64] = sum;
    __syncthreads();
-   for (uint32_t step = 1; step < kAdaptThreads; step <<= 1) {
-      const long long v = threadIdx.x >= step ? part[threadIdx.x - step] : 0;
-      __syncthreads();
-      part[threadIdx.x] += v;
-      __syncthreads();
-   }
-   long long coverage = part[threadIdx.x] - sum;
-   for (uint32_t p = lo; p < hi; ++p) {
-      coverage += change(p);
-      a.coverage[p] = static_cast<uint32_t>(coverage);
-      const uint32_t current = R.reference[p];
-      uint32_t ref_count = static_cast<uint32_t>(coverage);
-      for (uint32_t s = 0; s < nsym; ++s) {
-         if (s != current) ref_count -= adaptCount(a, p << 5 | s);
+   if (threadIdx.x < 64) {
+      int32_t at = p0 + threadIdx.x < L ? a.changes[p0 + threadIdx.x] : 0;
+      for (uint32_t o = 1; o < 64; o <<= 1) {
+         const int32_t v = __shfl_up(at, o, 64);
+         if (threadIdx.x >= o) at += v;
       }
-      uint32_t best = current, best_count = ref_count;
-      for (uint32_t s = 0; s < nsym; ++s) {
-         const uint32_t c = adaptCount(a, p << 5 | s);
-         if (s != current && c > best_count) {
-            best = s;
-            best_count = c;
+      for (uint32_t w = 0; w < kRuleThreads / 64; ++w) at += part[w];
+      coverage[threadIdx.x] = static_cast<uint32_t>(at);
+      if (p0 + threadIdx.x < L) a.coverage[p0 + threadIdx.x] = static_cast<uint32_t>(at);
+   }
+   __syncthreads();
+   for (uint32_t k = threadIdx.x / 32; k < kRulePositions; k += kRuleAtOnce) {
+      const uint32_t p = p0 + k, s = threadIdx.x & 31;
+      if (p >= L) continue;  // (the same in all lanes that shuffle with each other)
+      const uint32_t current = R.reference[p];
+      const bool other = s < nsym && s != current;
+      const uint32_t n = other ? adaptCount(a, p << 5 | s) : 0u;
+      uint32_t others = n;
+      for (int o = 16; o > 0; o >>= 1) others += __shfl_xor(others, o, 32);
+      const uint32_t ref_count = coverage[k] - others;
+      // the larger count wins, and among equal ones the smaller symbol
+      uint32_t best_count = n, best = s;
+      for (int o = 16; o > 0; o >>= 1) {
+         const uint32_t c2 = __shfl_xor(best_count, o, 32), s2 = __shfl_xor(best, o, 32);
+         if (c2 > best_count || (c2 == best_count && s2 < best)) {
+            best_count = c2;
+            best = s2;
          }
       }
-      a.local_ref[p] = static_cast<uint8_t>(best);
+      if (s == 0) a.local_ref[p] = static_cast<uint8_t>(best_count > ref_count ? best : current);
    }
 }
 
@@ -280,7 +391,10 @@ hipError_t launchAdapt(const AdaptCount& a, void* temp, size_t* temp_bytes, hipS
                          buf.Current(), a.key_count, past, a.run_start, a.run_end);
       if ((err = hipGetLastError()) != hipSuccess) return err;
    }
-   hipLaunchKernelGGL(adaptRuleKernel, dim3(1), dim3(kAdaptThreads), 0, stream, a);
+   const uint32_t blocks = (a.rows.length + kRulePositions - 1) / kRulePositions;
+   hipLaunchKernelGGL(adaptChangesKernel, dim3(blocks), dim3(kRuleThreads), 0, stream, a);
+   if ((err = hipGetLastError()) != hipSuccess) return err;
+   hipLaunchKernelGGL(adaptRuleKernel, dim3(blocks), dim3(kRuleThreads), 0, stream, a);
    return hipGetLastError();
 }
 

@@ -266,16 +266,20 @@ hipError_t launchRowIds(const uint64_t* words, const uint32_t* chunk_cards, uint
 // per row the covered range [start, end) ([0, 0) when nothing is covered), the number of mutations
 // and of internal missing runs, and the first illegal character's position (0xFFFFFFFF: none); the
 // write pass writes the mutations at mut_off[i] and the runs at run_off[i].
+constexpr size_t kRefTextPad = 16;
 struct DiffBatch {
-   const char* data = nullptr;
+   const char* data = nullptr;  // 16-byte aligned, readable up to a multiple of 16 bytes
    const uint64_t* row_ptr = nullptr;
    const uint32_t* offsets = nullptr;
    const uint8_t* is_null = nullptr;
    const uint8_t* lut = nullptr;  // 256 entries: the symbol of a character, 0xFF for an illegal one
-   const uint8_t* ref = nullptr;  // reference symbols
+   // a character of each position's reference symbol, readable from kRefTextPad before the first
+   // position to kRefTextPad past the last
+   const uint8_t* ref_text = nullptr;
    uint32_t n_rows = 0;
    uint32_t length = 0;
-   uint32_t missing = 0;  // the missing symbol
+   uint32_t missing = 0;       // the missing symbol
+   uint32_t missing_char = 0;  // a character of it
    uint32_t* start = nullptr;
    uint32_t* end = nullptr;
    uint32_t* n_mut = nullptr;
@@ -321,6 +325,8 @@ struct AdaptCount {
    uint64_t key_count = 0;
    uint32_t* run_start = nullptr;
    uint32_t* run_end = nullptr;
+   int32_t* changes = nullptr;        // [length]
+   int32_t* block_changes = nullptr;  // [length]
    uint32_t* coverage = nullptr;
    uint8_t* local_ref = nullptr;
 };
