@@ -36,7 +36,6 @@ hipError_t launchStreamRead(const void* src, size_t bytes, uint32_t* out, uint32
 constexpr size_t kNoAllocScratchBytes = size_t{128} << 20;
 hipError_t noallocScratch(int device, void** ptr);
 
-size_t filterLdsBytes(uint32_t depth);
 // The deepest operand stack that a program may need.
 uint32_t filterMaxDepth(size_t max_lds_bytes);
 // Lets the filter kernel allocate up to max_lds_bytes of dynamic LDS (deep operator trees).

@@ -222,12 +222,16 @@ struct NoProgram {};
 constexpr uint32_t kVmRegStack = 15;
 constexpr uint32_t kPlaneGroup = 12;  // planes of a bit-sliced column loaded together (a date has ten or eleven)
 typedef uint64_t VmRegs __attribute__((ext_vector_type(kVmRegStack + 1)));
-__host__ __device__ constexpr size_t vmWaveLdsBytes(uint32_t depth) {
-   return ((depth > kVmRegStack ? depth - kVmRegStack : 0) + 1) * 64 * sizeof(uint64_t) + kPrefetchSlots * 8 * sizeof(uint32_t) +
-          kProgCache * sizeof(Instr);
+// A single program's wavefronts are too few to fill the chip (992 on 4 M rows), so its stack stays in LDS,
+// whose entries cost less to reach: row ids of an n-of-m filter on 4 M rows 4 % slower with
+// registers.
+__host__ __device__ constexpr size_t vmWaveLdsBytes(uint32_t depth, bool single) {
+   const uint32_t in_registers = single ? 0 : kVmRegStack;
+   return ((depth > in_registers ? depth - in_registers : 0) + 1) * 64 * sizeof(uint64_t) +
+          kPrefetchSlots * 8 * sizeof(uint32_t) + kProgCache * sizeof(Instr);
 }
 template <bool kSingle>
-__global__ __launch_bounds__(kVmThreads, 4) void filterVmKernel(std::conditional_t<kSingle, SingleProgram, NoProgram> single,
+__global__ __launch_bounds__(kVmThreads, kSingle ? 1 : 4) void filterVmKernel(std::conditional_t<kSingle, SingleProgram, NoProgram> single,
                                                              TableView tv, const ProgramDesc* __restrict__ progs,
                                                              const Instr* __restrict__ instrs,
                                                              const uint32_t* __restrict__ ranges, uint32_t depth,
@@ -251,8 +255,9 @@ __global__ __launch_bounds__(kVmThreads, 4) void filterVmKernel(std::conditional
    const uint32_t lane = threadIdx.x & 63;
    // per wavefront: the stack's entries past the register ones, scratch words, the prefetched leaf
    // records, the cached instructions
-   const uint32_t n_deep = depth > kVmRegStack ? depth - kVmRegStack : 0;
-   uint8_t* mine = reinterpret_cast<uint8_t*>(lds) + wave * vmWaveLdsBytes(depth);
+   constexpr uint32_t kRegs = kSingle ? 0 : kVmRegStack;
+   const uint32_t n_deep = depth > kRegs ? depth - kRegs : 0;
+   uint8_t* mine = reinterpret_cast<uint8_t*>(lds) + wave * vmWaveLdsBytes(depth, kSingle);
    uint64_t* deep = reinterpret_cast<uint64_t*>(mine);
    uint64_t* scratch = deep + n_deep * 64;
    uint32_t* pf = reinterpret_cast<uint32_t*>(scratch + 64);
@@ -328,10 +333,10 @@ __global__ __launch_bounds__(kVmThreads, 4) void filterVmKernel(std::conditional
       const size_t row_base = (static_cast<size_t>(chunk) << 16) + slice * 4096u;
       uint32_t sp = 0;
       // entry k of the stack (k is the same in every lane)
-      auto at = [&](uint32_t k) -> uint64_t { return k < kVmRegStack ? regs[k] : deep[(k - kVmRegStack) * 64 + lane]; };
+      auto at = [&](uint32_t k) -> uint64_t { return k < kRegs ? regs[k] : deep[(k - kRegs) * 64 + lane]; };
       auto put = [&](uint32_t k, uint64_t v) {
-         regs[k < kVmRegStack ? k : kVmRegStack] = v;
-         if (k >= kVmRegStack) deep[(k - kVmRegStack) * 64 + lane] = v;
+         if constexpr (kRegs != 0) regs[k < kRegs ? k : kRegs] = v;
+         if (k >= kRegs) deep[(k - kRegs) * 64 + lane] = v;
       };
       // the top entry is `tos` where `held`, else it is in its place like the others
       uint64_t tos = 0;
@@ -3220,13 +3225,13 @@ hipError_t configureFilterKernel(size_t max_lds_bytes) {
                               hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(max_lds_bytes));
 }
 
-size_t filterLdsBytes(uint32_t depth) { return kVmWaves * vmWaveLdsBytes(depth); }
+static size_t filterLdsBytes(uint32_t depth, bool single) { return kVmWaves * vmWaveLdsBytes(depth, single); }
 
 uint32_t filterMaxDepth(size_t max_lds_bytes) {
    // as deep as if the whole stack were in LDS, beside 6 KiB of a wavefront's own: what programs have
    // always been accepted up to
    const size_t entries = (max_lds_bytes / kVmWaves - 6144) / (64 * sizeof(uint64_t));
-   static_assert(kVmWaves * vmWaveLdsBytes(2) <= 64 * 1024, "shallow programs fit the smallest LDS");
+   static_assert(kVmWaves * vmWaveLdsBytes(2, true) <= 64 * 1024, "shallow programs fit the smallest LDS");
    return std::max<uint32_t>(1, static_cast<uint32_t>(entries) - 1);
 }
 
@@ -3247,7 +3252,7 @@ hipError_t launchFilterBatch(const TableView& tv, const ProgramDesc* progs, cons
    if (n_items == 0) return hipSuccess;
    // a work-group per kVmWaves slices (the most units there can be) up to max_blocks
    const uint32_t blocks = std::min((n_items + kVmWaves - 1) / kVmWaves, max_blocks);
-   hipLaunchKernelGGL(filterVmKernel<false>, dim3(blocks), dim3(kVmThreads), filterLdsBytes(depth), stream,
+   hipLaunchKernelGGL(filterVmKernel<false>, dim3(blocks), dim3(kVmThreads), filterLdsBytes(depth, false), stream,
                       NoProgram{}, tv, progs, instrs, ranges, depth, out, cards, chunk_cards, header, filterUnit(n_items));
    return hipGetLastError();
 }
@@ -3258,7 +3263,7 @@ hipError_t launchFilterSingle(const TableView& tv, const SingleProgram& program,
    if (n_items == 0) return hipErrorInvalidValue;
    const uint32_t unit = filterUnit(n_items);
    hipLaunchKernelGGL(filterVmKernel<true>, dim3((n_items / unit + kVmWaves - 1) / kVmWaves), dim3(kVmThreads),
-                      filterLdsBytes(depth), stream, program, tv, static_cast<const ProgramDesc*>(nullptr),
+                      filterLdsBytes(depth, true), stream, program, tv, static_cast<const ProgramDesc*>(nullptr),
                       static_cast<const Instr*>(nullptr), static_cast<const uint32_t*>(nullptr), depth, out, card,
                       chunk_cards, static_cast<const uint32_t*>(nullptr), unit);
    return hipGetLastError();
