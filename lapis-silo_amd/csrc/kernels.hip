@@ -130,12 +130,33 @@ __device__ inline void accumulateContainer(const Desc d, const ContainerArenas& 
       acc |= toGlobal<GlobalU64>(ar.bits)[static_cast<size_t>(d.w1) * kChunkWords + my_word];
    } else if (type == CT_ARRAY) {
       const GlobalU16* a = toGlobal<GlobalU16>(ar.arr + d.w1);
-      const uint32_t b = waveLowerBound(0, card, [&](uint32_t i) { return static_cast<uint32_t>(a[i]) < lo; });
-      const uint32_t e = hi >= kChunkRows ? card
-                                          : waveLowerBound(b, card, [&](uint32_t i) { return static_cast<uint32_t>(a[i]) < hi; });
-      for (uint32_t k = b + lane; k < e; k += 64) {
-         const uint32_t v = a[k];
-         atomicOr(reinterpret_cast<unsigned long long*>(&scratch[(v >> 6) & 63]), 1ULL << (v & 63));
+      // 64 evenly spaced samples, one per lane, bound the slice's rows: all rows up to the last sample below
+      // it are below it, all from the first sample past it are past it.  What lies between is loaded
+      // in one more round and tested (a search for each end took four dependent rounds).
+      const uint32_t step = (card + 63) / 64;
+      const uint32_t idx = lane * step;
+      const uint32_t sample = idx < card ? a[idx] : kChunkRows;
+      const auto set = [&](uint32_t v) {
+         if (v >= lo && v < hi) atomicOr(reinterpret_cast<unsigned long long*>(&scratch[(v >> 6) & 63]), 1ULL << (v & 63));
+      };
+      if (step == 1) {  // the samples are the rows
+         set(sample);
+      } else {
+         const uint32_t below = static_cast<uint32_t>(__popcll(__ballot(sample < lo)));
+         const uint32_t upto = static_cast<uint32_t>(__popcll(__ballot(sample < hi)));
+         const uint32_t begin = below ? (below - 1) * step + 1 : 0u;
+         const uint32_t end = upto * step < card ? upto * step : card;
+         constexpr uint32_t kLoads = 4;  // in flight; an evenly spread container has at most 384 rows here
+         for (uint32_t k0 = begin; k0 < end; k0 += 64 * kLoads) {
+            uint32_t v[kLoads];
+#pragma unroll
+            for (uint32_t u = 0; u < kLoads; ++u) {
+               const uint32_t k = k0 + 64 * u + lane;
+               v[u] = k < end ? a[k] : kChunkRows;
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < kLoads; ++u) set(v[u]);
+         }
       }
    } else {
       const GlobalU32* r = toGlobal<GlobalU32>(ar.runs + d.w1);
@@ -1418,10 +1439,10 @@ __global__ __launch_bounds__(256) void sparseCountKernel(const SeqColumnView* __
 //   c: internal missing runs starting at p minus those ending at p.
 constexpr uint32_t kMaxSymbols = 28;
 struct BlockValues {
-   uint32_t v[kMaxSymbols][kPosBlock];
    uint32_t a[kPosBlock];
    uint32_t b[kPosBlock];
    int32_t c[kPosBlock];
+   uint32_t v[kMaxSymbols][kPosBlock];  // the alphabet's symbols only are there (finalizeLdsBytes)
 };
 
 // Sources of the per-position quantities for the totals and finalize kernels; stage() fills a
@@ -1443,16 +1464,12 @@ struct SlotSource {
    uint32_t n_more = 0;
    uint32_t* heavy = nullptr;
 
-   __device__ uint32_t value(uint32_t s, bool clear) const {
+   __device__ uint32_t value(uint32_t s, uint32_t& heavy_part) const {
       uint32_t v = partial[s];
       if (partial_b) v += partial_b[s];
       for (uint32_t k = 0; k < n_more; ++k) v += partial_c[k * plane + s];
-      if (heavy) {
-         const uint32_t h = heavy[s];
-         v += h;
-         if (clear && h) heavy[s] = 0;
-      }
-      return v;
+      heavy_part = heavy ? heavy[s] : 0u;
+      return v + heavy_part;
    }
 
    __device__ void stage(uint32_t p0, BlockValues& bv, bool clear) const {
@@ -1468,44 +1485,55 @@ struct SlotSource {
       const GlobalU32* info = toGlobal<GlobalU32>(col->slot_info);
       const uint32_t s0 = pos_ptr[p0];
       const uint32_t s1 = pos_ptr[p0 + kPosBlock < L ? p0 + kPosBlock : L];
-      for (uint32_t s = s0 + t; s < s1; s += kPosBlock) {
-         const uint32_t x = info[s];
-         const uint32_t v = value(s, clear);
-         const uint32_t pl = (x & 0xFFFFu) - p0;
-         const uint32_t sym = x >> 16;
-         if (sym < ns) {
-            bv.v[sym][pl] = v;
-         } else {
-            switch (sym - ns) {
-               case BND_COV_START: bv.a[pl] = v; break;
-               case BND_COV_END: bv.b[pl] = v; break;
-               case BND_N_START: atomicAdd(&bv.c[pl], static_cast<int32_t>(v)); break;
-               default: atomicSub(&bv.c[pl], static_cast<int32_t>(v)); break;
+      constexpr uint32_t kLoads = 4;  // slots of a thread whose loads are all in flight
+      for (uint32_t base = s0 + t; base < s1; base += kLoads * kPosBlock) {
+         uint32_t x[kLoads], v[kLoads], hv[kLoads];
+#pragma unroll
+         for (uint32_t u = 0; u < kLoads; ++u) {
+            const uint32_t s = base + u * kPosBlock < s1 ? base + u * kPosBlock : base;
+            x[u] = info[s];
+            v[u] = value(s, hv[u]);
+         }
+#pragma unroll
+         for (uint32_t u = 0; u < kLoads; ++u) {
+            const uint32_t s = base + u * kPosBlock;
+            if (s >= s1) break;
+            if (clear && hv[u]) heavy[s] = 0;
+            const uint32_t pl = (x[u] & 0xFFFFu) - p0;
+            const uint32_t sym = x[u] >> 16;
+            if (sym < ns) {
+               bv.v[sym][pl] = v[u];
+            } else {
+               switch (sym - ns) {
+                  case BND_COV_START: bv.a[pl] = v[u]; break;
+                  case BND_COV_END: bv.b[pl] = v[u]; break;
+                  case BND_N_START: atomicAdd(&bv.c[pl], static_cast<int32_t>(v[u])); break;
+                  default: atomicSub(&bv.c[pl], static_cast<int32_t>(v[u])); break;
+               }
             }
          }
       }
       __syncthreads();
    }
    __device__ uint32_t implicitSymbol(uint32_t p) const { return col->local_ref[p]; }
-   // this thread's share of the block sums of a, b and c (boundary slots are the last of a position)
+   // this thread's share of the block sums of a, b and c: its position's boundary slots (found from one
+   // word, without looking through the block's slots for them)
    __device__ void blockSums(uint32_t p0, int64_t& a, int64_t& b, int64_t& c) const {
-      const uint32_t L = col->genome_length;
-      const uint32_t ns = col->n_symbols;
-      const GlobalU32* pos_ptr = toGlobal<GlobalU32>(col->pos_slot_ptr);
-      const GlobalU32* info = toGlobal<GlobalU32>(col->slot_info);
-      const uint32_t s0 = pos_ptr[p0];
-      const uint32_t s1 = pos_ptr[p0 + kPosBlock < L ? p0 + kPosBlock : L];
-      for (uint32_t s = s0 + threadIdx.x; s < s1; s += kPosBlock) {
-         const uint32_t sym = info[s] >> 16;
-         if (sym < ns) continue;
-         const int64_t v = value(s, false);
-         switch (sym - ns) {
-            case BND_COV_START: a += v; break;
-            case BND_COV_END: b += v; break;
-            case BND_N_START: c += v; break;
-            default: c -= v; break;
-         }
+      const uint32_t p = p0 + threadIdx.x;
+      if (p >= col->genome_length) return;
+      const uint32_t x = toGlobal<GlobalU32>(col->boundary_slots)[p];
+      uint32_t s = x & kBoundarySlotMask;
+      int64_t v[4];
+#pragma unroll
+      for (uint32_t k = 0; k < 4; ++k) {
+         const uint32_t have = (x >> (kBoundarySlotBits + k)) & 1u;
+         uint32_t heavy_part;
+         v[k] = have ? value(s, heavy_part) : 0u;
+         s += have;
       }
+      a += v[BND_COV_START];
+      b += v[BND_COV_END];
+      c += v[BND_N_START] - v[BND_N_END];
    }
 };
 
@@ -1520,17 +1548,28 @@ struct SparseSource {
       const uint32_t p = p0 + t;
       const uint32_t ns = col->n_symbols;
       if (p < L) {
-         for (uint32_t k = 0; k < ns; ++k) {
-            bv.v[k][t] = counts[static_cast<size_t>(k) * L + p];
-            if (clear) counts[static_cast<size_t>(k) * L + p] = 0;
+         // all loads before any store (a store between two loads keeps the second waiting for the first's
+         // value), and only what is not zero, a few of each position's counts, is cleared
+         constexpr uint32_t kLoads = 16;
+         const int32_t bnd_p[3] = {bnd[p], bnd[L + p], bnd[2 * L + p]};
+         for (uint32_t k0 = 0; k0 < ns; k0 += kLoads) {
+            uint32_t x[kLoads];
+#pragma unroll
+            for (uint32_t u = 0; u < kLoads; ++u) x[u] = k0 + u < ns ? counts[static_cast<size_t>(k0 + u) * L + p] : 0u;
+#pragma unroll
+            for (uint32_t u = 0; u < kLoads; ++u) {
+               if (k0 + u < ns) bv.v[k0 + u][t] = x[u];
+               if (clear && x[u] != 0) counts[static_cast<size_t>(k0 + u) * L + p] = 0;
+            }
          }
-         bv.a[t] = static_cast<uint32_t>(bnd[p]);
-         bv.b[t] = static_cast<uint32_t>(bnd[L + p]);
-         bv.c[t] = bnd[2 * L + p];
+         bv.a[t] = static_cast<uint32_t>(bnd_p[0]);
+         bv.b[t] = static_cast<uint32_t>(bnd_p[1]);
+         bv.c[t] = bnd_p[2];
          if (clear) {
-            bnd[p] = 0;
-            bnd[L + p] = 0;
-            bnd[2 * L + p] = 0;
+#pragma unroll
+            for (uint32_t k = 0; k < 3; ++k) {
+               if (bnd_p[k] != 0) bnd[k * L + p] = 0;
+            }
          }
       } else {
          for (uint32_t k = 0; k < ns; ++k) bv.v[k][t] = 0;
@@ -1602,14 +1641,18 @@ __device__ __forceinline__ void totalsBody(const Src& src, uint32_t pblock, int6
 
 // LDS of the finalize step, one instance per kernel whichever sources it finalizes
 struct FinalizeShared {
-   BlockValues bv;
    int64_t scan_tmp[kPosWaves];
-   int64_t part[4][kPosWaves];
-   int64_t prefix[4];  // previous-block sums of a, b, c and the total of a
+   int64_t part[2][kPosWaves];
+   int64_t prefix[2];  // previous blocks' sum of a - b - c, and the total of a
+   BlockValues bv;
 };
+// (20 KB for nucleotides, so that eight work-groups fit a CU, 32 KB for amino acids)
+constexpr size_t finalizeLdsBytes(uint32_t n_symbols) {
+   return sizeof(FinalizeShared) - (kMaxSymbols - n_symbols) * kPosBlock * sizeof(uint32_t);
+}
 __device__ inline FinalizeShared& finalizeShared() {
-   __shared__ FinalizeShared sh;
-   return sh;
+   extern __shared__ uint64_t lds[];
+   return *reinterpret_cast<FinalizeShared*>(lds);
 }
 
 template <typename Src>
@@ -1626,23 +1669,19 @@ __device__ __forceinline__ void finalizeBody(const Src& src, uint32_t pblock, co
    {
       // block totals: thread k < n_pblocks (<= kPosBlock for genome lengths below 2^16) takes block k
       const uint32_t k = threadIdx.x;
-      int64_t a = 0, b = 0, c = 0, ta = 0;
+      int64_t net = 0, starts = 0;
       if (k < n_pblocks) {
-         ta = totals[3 * k];
-         if (k < pblock) {
-            a = ta;
-            b = totals[3 * k + 1];
-            c = totals[3 * k + 2];
-         }
+         starts = totals[3 * k];
+         if (k < pblock) net = starts - totals[3 * k + 1] - totals[3 * k + 2];
       }
-      const int64_t v[4] = {a, b, c, ta};
+      const int64_t v[2] = {net, starts};
       const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-      for (int q = 0; q < 4; ++q) {
+      for (int q = 0; q < 2; ++q) {
          const int64_t x = waveTotal(v[q]);
          if (lane == 0) part[q][wave] = x;
       }
       __syncthreads();
-      if (threadIdx.x < 4) {
+      if (threadIdx.x < 2) {
          int64_t sum = 0;
          for (int w = 0; w < kPosWaves; ++w) sum += part[threadIdx.x][w];
          prefix[threadIdx.x] = sum;
@@ -1652,14 +1691,13 @@ __device__ __forceinline__ void finalizeBody(const Src& src, uint32_t pblock, co
    const uint32_t L = col.genome_length;
    const uint32_t t = threadIdx.x;
    const uint32_t p = pblock * kPosBlock + t;
-   const int64_t pa = blockInclusiveScan<int64_t>(bv.a[t], scan_tmp) + prefix[0];
-   const int64_t pb = blockInclusiveScan<int64_t>(bv.b[t], scan_tmp) + prefix[1];
-   const int64_t pc = blockInclusiveScan<int64_t>(bv.c[t], scan_tmp) + prefix[2];
+   const int64_t net = static_cast<int64_t>(bv.a[t]) - static_cast<int64_t>(bv.b[t]) - bv.c[t];
+   const int64_t up_to = blockInclusiveScan<int64_t>(net, scan_tmp) + prefix[0];
    if (p >= L) return;
    const uint32_t ns = col.n_symbols;
    const int64_t card = static_cast<int64_t>(filter_card);
    // rows covered at p: not starting after p, not ended at or before p, not inside a missing run
-   const int64_t covered = card - (prefix[3] - pa) - pb - pc;
+   const int64_t covered = card - prefix[1] + up_to;
    int64_t stored = 0;
    for (uint32_t sym = 0; sym < ns; ++sym) stored += bv.v[sym][t];
    const uint32_t implicit_count = card == 0 ? 0u : static_cast<uint32_t>(covered - stored);
@@ -3477,7 +3515,8 @@ hipError_t launchMutationsBatch(const MutationsBatch& m, hipStream_t stream) {
    hipLaunchKernelGGL(mutationsTotalsBatchKernel, dim3(n_pblocks, gq), dim3(kPosBlock), 0, stream, m,
                       n_pblocks, dense_parts);
    if ((err = hipGetLastError()) != hipSuccess) return err;
-   hipLaunchKernelGGL(mutationsFinalizeBatchKernel, dim3(n_pblocks, gq), dim3(kPosBlock), 0, stream, m,
+   hipLaunchKernelGGL(mutationsFinalizeBatchKernel, dim3(n_pblocks, gq), dim3(kPosBlock),
+                      finalizeLdsBytes(h.n_symbols), stream, m,
                       n_pblocks, dense_parts);
    return hipGetLastError();
 }
