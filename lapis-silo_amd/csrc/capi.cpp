@@ -103,39 +103,6 @@ static void streamCopy(uint8_t* to, const uint8_t* from, size_t n) {
    _mm_sfence();  // before the copy that reads it is enqueued
 }
 
-// The runtime's copy from pageable memory takes one host thread through its own staging buffers (29 GB/s;
-// 8.5 ms for 245 MB); the pool fills pinned memory faster than the link empties it, so the copies follow
-// each other without a gap (6.5 ms).  Below kLeast the runtime's copy is as fast.
-void Context::uploadStaged(void* dst, const void* src, size_t bytes) {
-   constexpr size_t kGroupSlots = 8, kGroups = kStageSlots / kGroupSlots, kGroupBytes = kGroupSlots * kStageSlotBytes;
-   constexpr size_t kPiece = size_t{256} << 10, kLeast = size_t{2} << 20;
-   hipCheck(hipStreamSynchronize(stream), "synchronize");  // no slot of the ring is in use any more
-   std::fill(std::begin(stage_used), std::end(stage_used), false);
-   if (bytes < kLeast) {
-      hipCheck(hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice), "upload");
-      return;
-   }
-   const auto* from = static_cast<const uint8_t*>(src);
-   auto* to = static_cast<uint8_t*>(dst);
-   try {
-      for (size_t g = 0, at = 0; at < bytes; ++g, at += kGroupBytes) {
-         const size_t slot = g % kGroups * kGroupSlots;
-         if (g >= kGroups) hipCheck(hipEventSynchronize(stage_events[slot]), "staging slot wait");
-         const size_t n = std::min(kGroupBytes, bytes - at);
-         auto* host = static_cast<uint8_t*>(stage_host) + slot * kStageSlotBytes;
-         parallelFor((n + kPiece - 1) / kPiece, [&](size_t k) {
-            streamCopy(host + k * kPiece, from + at + k * kPiece, std::min(kPiece, n - k * kPiece));
-         });
-         hipCheck(hipMemcpyAsync(to + at, host, n, hipMemcpyHostToDevice, stream), "upload");
-         hipCheck(hipEventRecord(stage_events[slot], stream), "hipEventRecord");
-      }
-   } catch (...) {
-      (void)hipStreamSynchronize(stream);  // no copy reads the ring after this
-      throw;
-   }
-   hipCheck(hipStreamSynchronize(stream), "upload");
-}
-
 uint32_t maxFilterDepth(const Context& ctx) {
    return filterMaxDepth(ctx.max_lds_bytes);
 }

@@ -163,9 +163,6 @@ struct Context {
    bool stage_used[kStageSlots] = {};
    size_t stage_next = 0;
    DeviceBuffer stage_big;
-   // A large host array to the device through the ring, copied into it by the worker pool while the parts
-   // before are on their way; done on return.
-   void uploadStaged(void* dst, const void* src, size_t bytes);
    // Copies `bytes` of host data to device memory that stays valid for work enqueued afterwards on
    // `stream` until the ring wraps (64 further uploads); large uploads synchronize the stream.
    void* stage(const void* host, size_t bytes);

@@ -85,7 +85,7 @@ void seqBuilderAppend(SeqBuilder& b, const char* data, const uint64_t* row_ptr, 
          if (is_null) std::copy(is_null + a, is_null + e, nulls.begin());
          DiffBatch d;
          if (text.bytes() < ptr[n] + 16) text = DeviceBuffer(ptr[n] + 16);
-         if (ptr[n]) t.ctx->uploadStaged(text.as<void>(), data + row_ptr[a], ptr[n]);
+         if (ptr[n]) hipCheck(hipMemcpy(text.as<void>(), data + row_ptr[a], ptr[n], hipMemcpyHostToDevice), "upload");
          d.data = text.as<char>();
          d.row_ptr = upload(bufs, ptr.data(), ptr.size());
          d.offsets = offsets ? upload(bufs, offsets + a, n) : nullptr;
