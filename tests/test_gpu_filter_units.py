@@ -57,3 +57,31 @@ def test_programs(engine, sizes):
             assert [b.count(q) for q in range(len(many))] == [int(keep.sum()) for _, keep in many]
     finally:
         et.close()
+
+
+@pytest.mark.parametrize("n", [3, 63, 64, 65, 127, 129, 500, 1025, 4095, 4096])
+def test_array_containers(engine, n):
+    """Array containers around the sizes where a sample stands for one row, or a slice for several rounds:
+    spread evenly, at random, crowded at either end, around one slice's edge.  (Rows two apart: no runs.)"""
+    from silo_amd import table
+
+    rng = np.random.default_rng(n)
+    size = 65536
+    sets = [np.arange(n) * (size // n), rng.choice(size // 2, n, replace=False) * 2, np.arange(n) * 2, size - 1 - np.arange(n) * 2,
+            8191 + 2 * (np.arange(n) - n // 2)]
+    spec = table.TableSpec(chunk_sizes=np.array([size, 700], np.uint32))
+    want = []
+    for k, rows in enumerate(sets):
+        rows = np.unique(np.clip(rows, 0, size - 1))
+        ids = np.zeros(size + 700, np.uint32)
+        ids[rows] = 1
+        spec.dict_columns.append(table.DictColumnData(f"d{k}", ids, np.zeros(size + 700, np.uint8), ["other", "mine"]))
+        want.append(rows)
+    et = engine.table(spec)
+    try:
+        for k, rows in enumerate(want):
+            assert np.array_equal(et.filter(f'(str_eq d{k} "mine")'), spec.global_ids()[rows]), k
+        with et.batch_submit([{"action": "count", "filter": f'(str_eq d{k} "mine")'} for k in range(len(want))]) as b:
+            assert [b.count(k) for k in range(len(want))] == [len(rows) for rows in want]
+    finally:
+        et.close()
