@@ -1,6 +1,6 @@
 """The diff of aligned sequences where its kernel's work is cut: rows that start at any byte of an aligned
 16, differences and missing runs at the edges of a lane's 16 characters and of a step's 1,024, rows that
-differ everywhere, lower case, references with missing positions; appends larger than the staging ring;
+differ everywhere, lower case, references with missing positions; an append of 74 MB;
 the adapted reference at the edges of the blocks of 64 positions that the rule is cut into.  Layouts equal
 those of the oracle's diff, uploaded in diff form, byte for byte."""
 import numpy as np
@@ -54,7 +54,7 @@ def test_edges(engine, alphabet, length):
     check(engine, table.TableSpec(chunk_sizes=np.array([100, 80], np.uint32)), alphabet, ref, rows, 1, 77)
 
 
-def test_larger_than_the_staging_ring(engine):
+def test_large_append(engine):
     from silo_amd import table
 
     rng = np.random.default_rng(5)
