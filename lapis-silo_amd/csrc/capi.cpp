@@ -952,6 +952,14 @@ int rdb_mutations_query_noalloc(rdb_table* table, const char* filter, const char
       }
       auto* base = static_cast<uint8_t*>(t.ctx->noalloc_scratch);
       hipStream_t stream = t.ctx->stream;
+      // Every context of this GPU shares the scratch, and each has a stream of its own.  The result's stamps
+      // arrive before its kernel has retired, and what that kernel stored in the scratch leaves the XCDs'
+      // L2s only when it retires: the call ends, however it ends, with its stream drained, so that the next
+      // one, from any context, finds the scratch at rest.
+      struct Drain {
+         hipStream_t stream;
+         ~Drain() { (void)hipStreamSynchronize(stream); }
+      } drain{stream};
       if (!blob.empty()) {
          hipCheck(hipMemcpyAsync(base + c.blob, blob.data(), blob.size(), hipMemcpyHostToDevice, stream), "stage program");
       }
@@ -997,6 +1005,7 @@ int rdb_mutations_query_noalloc(rdb_table* table, const char* filter, const char
       hipCheck(launchMutations(m, stream), "mutations kernels");
       rows.wait(*t.ctx, m.stamp);
       capi::emitMutationRows(col, rows, position, from, to, count, coverage, proportion, capacity, n);
+      hipCheck(hipStreamSynchronize(stream), "synchronize");  // (here most of the wait is over)
    });
 }
 

@@ -1,7 +1,8 @@
 """The allocation-free Mutations entry point (rdb_mutations_query_noalloc), called through the C ABI:
 its rows equal rdb_mutations_query's on two calls in a row, the second on a smaller table (the shared
 scratch keeps the first call's contents), with the dense and the sparse method; a table too large
-for the scratch is rejected with RDB_EINVAL."""
+for the scratch is rejected with RDB_EINVAL; calls from two contexts of the GPU, which share the scratch,
+may follow each other without a wait between them."""
 import ctypes
 
 import numpy as np
@@ -69,3 +70,37 @@ def test_noalloc_rejects_a_table_too_large(engine):
         assert call(et, "rdb_mutations_query", "(true)", "main", 0.0) == []
     finally:
         et.close()
+
+
+def test_noalloc_calls_of_two_contexts_in_turn(tables, engine):
+    """Each call, one whose rows do not fit the caller's arrays too, leaves the shared scratch to the
+    next context's: a large table's calls and a small one's, which cut the scratch differently, in
+    turn, one dense while the other is sparse."""
+    from silo_amd.engine import Engine, lib
+
+    (big_ds, eb), (small_ds, _) = tables
+    _, small = small_spec(seed=62, n_rows=5000, L=300, chunk=2048)
+    saved = engine.get_tuning("sparse_max_rows")
+    other = Engine(0)
+    es = other.table(small)
+    try:
+        exprs = [("(true)", "(true)")] + [tuple(f'(str_eq country "{ds.country_names[k]}")' for ds in (big_ds, small_ds))
+                                          for k in range(3)]
+        want = [(call(eb, "rdb_mutations_query", b, "main", 0.0), call(es, "rdb_mutations_query", s, "main", 0.0))
+                for b, s in exprs]
+        assert want[0][0]
+        for here, there in ((-1, 1 << 40), (1 << 40, -1)):
+            engine.set_tuning("sparse_max_rows", here)
+            other.set_tuning("sparse_max_rows", there)
+            for _ in range(5):
+                for (b, s), (rows_b, rows_s) in zip(exprs, want):
+                    assert call(eb, "rdb_mutations_query_noalloc", b, "main", 0.0) == rows_b, (here, b)
+                    assert call(es, "rdb_mutations_query_noalloc", s, "main", 0.0) == rows_s, (there, s)
+                n = ctypes.c_uint64()
+                assert lib().rdb_mutations_query_noalloc(eb.handle, b"(true)", b"main", 0.0, None, None, None, None, None,
+                                                         None, 0, ctypes.byref(n)) != 0
+                assert n.value == len(want[0][0])
+    finally:
+        engine.set_tuning("sparse_max_rows", saved)
+        es.close()
+        other.close()
