@@ -269,6 +269,7 @@ void launchLane(Table& t, BatchLane& lane, uint32_t depth, int column, bool aggr
       } catch (...) {
          (void)hipStreamEndCapture(lane.stream, &graph);
          if (graph) (void)hipGraphDestroy(graph);
+         (void)hipGetLastError();  // (of the capture that was given up: see failHip)
          throw;
       }
       hipCheck(hipStreamEndCapture(lane.stream, &graph), "end capture");

@@ -29,8 +29,16 @@ struct Error : std::runtime_error {
 
 [[noreturn]] inline void fail(int code, const std::string& msg) { throw Error(code, msg); }
 
+// Throws for an error of the runtime.  The runtime keeps the thread's last error until somebody asks for
+// it, and the launch functions ask after their kernels: the error is taken out of that record here, or
+// the next launch, which succeeds, would be reported as failed.
+[[noreturn]] inline void failHip(int code, const std::string& msg) {
+   (void)hipGetLastError();
+   fail(code, msg);
+}
+
 inline void hipCheck(hipError_t e, const char* what) {
-   if (e != hipSuccess) fail(RDB_EDEVICE, std::string(what) + ": " + hipGetErrorString(e));
+   if (e != hipSuccess) failHip(RDB_EDEVICE, std::string(what) + ": " + hipGetErrorString(e));
 }
 
 // Runs f(i) for i in [0, n) on up to `threads` host threads.

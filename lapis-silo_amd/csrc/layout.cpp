@@ -210,7 +210,7 @@ DeviceBuffer::DeviceBuffer(size_t bytes) : bytes_(bytes) {
    if (bytes_ == 0) return;
    if (hipMalloc(&ptr_, bytes_) != hipSuccess) {
       ptr_ = nullptr;
-      fail(RDB_ENOMEM, "device allocation of " + std::to_string(bytes) + " bytes failed");
+      failHip(RDB_ENOMEM, "device allocation of " + std::to_string(bytes) + " bytes failed");
    }
 }
 
@@ -253,7 +253,7 @@ void* DevicePool::get(size_t bytes) {
       }
    }
    void* p = nullptr;
-   if (hipMalloc(&p, bytes) != hipSuccess) fail(RDB_ENOMEM, "device allocation of " + std::to_string(bytes) + " bytes failed");
+   if (hipMalloc(&p, bytes) != hipSuccess) failHip(RDB_ENOMEM, "device allocation of " + std::to_string(bytes) + " bytes failed");
    return p;
 }
 

@@ -1,0 +1,47 @@
+"""Calls after one that failed answer as if it had not been made."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from helpers import small_spec
+
+pytestmark = pytest.mark.gpu
+
+
+def answers(et, country):
+    """Every action on a table, single and batched."""
+    expr = f'(and (str_eq country "{country}") (not (has_mut main 17)))'
+    out = [et.count(expr), et.filter(expr).tolist(), et.mutation_counts(expr, "main").tolist()]
+    for p in (0.0, 0.05):
+        out.append(et.mutations_query(expr, "main", p))
+    for dims in ([], ["country"], ["main@20", "country"]):
+        out.append(et.aggregate(expr, dims))
+    out.append(et.batch([{"filter": expr, "action": "mutations", "column": "main", "min_proportion": 0.05},
+                         {"filter": expr, "action": "aggregate", "dims": ["country"]},
+                         {"filter": expr, "action": "count"}]))
+    return out
+
+
+def test_failed_allocation(engine):
+    """A device allocation larger than any GPU's memory fails its own call only: the kernels launched
+    next, each action's first and last, are not taken for failed ones."""
+    from silo_amd.engine import EngineError
+
+    ds, ts = small_spec(seed=91, n_rows=9000, L=400, chunk=4096)
+    et = engine.table(ts)
+    try:
+        country = ds.country_names[0]
+        want = answers(et, country)
+        calls = [lambda: et.count("(true)"), lambda: et.mutation_counts("(true)", "main").sum(),
+                 lambda: et.mutations_query("(true)", "main", 0.05), lambda: et.aggregate("(true)", ["country"]),
+                 lambda: et.batch([{"filter": "(true)", "action": "count"}])]
+        for call in calls:
+            expected = call()
+            with pytest.raises(EngineError) as err:
+                engine.read_bandwidth(1 << 50, 1)
+            assert err.value.status == "RDB_ENOMEM"
+            assert np.array_equal(call(), expected) if not isinstance(expected, list) else call() == expected
+        assert answers(et, country) == want
+    finally:
+        et.close()
