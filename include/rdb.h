@@ -416,7 +416,10 @@ int rdb_set_planner(rdb_ctx* ctx, int mode, rdb_mlp* mlp);
  *                      column's index build run on the GPU (default), 0: on the host;
  *   "batch_fail_job"   fault injection for tests: the n-th lane job enqueued from now on fails with
  *                      RDB_ENOMEM after its inputs were staged, failing its rdb_batch_submit (0, the
- *                      default: never).
+ *                      default: never);
+ *   "query_fail"       fault injection for tests: the n-th Mutations or Aggregated query outside batches
+ *                      from now on fails with RDB_EDEVICE after its counting kernels were enqueued and
+ *                      before its result kernel (0, the default: never).
  * Results never depend on them.  RDB_EINVAL for an unknown key or an out-of-range value. */
 int rdb_set_tuning(rdb_ctx* ctx, const char* key, int64_t value);
 int rdb_get_tuning(rdb_ctx* ctx, const char* key, int64_t* value);

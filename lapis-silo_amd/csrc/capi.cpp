@@ -175,6 +175,7 @@ MutationsLaunch mutationsLaunch(Table& t, int idx, const DeviceBitmap& f) {
    m.heavy_sums = t.ctx->mutation_packed ? t.heavy_sums.as<uint32_t>() : nullptr;
    m.sparse_counts = col.sparse_counts.as<uint32_t>();
    m.sparse_bnd = col.sparse_bnd.as<int32_t>();
+   m.fail = t.ctx->failsNow();
    auto* state = t.query_state.as<QueryState>();
    m.totals = state->totals[t.totals_turn];
    t.totals_turn ^= 1;
@@ -316,6 +317,9 @@ int rdb_set_tuning(rdb_ctx* ctx, const char* key, int64_t value) {
       } else if (k == "batch_fail_job") {
          if (value < 0 || value > 1000000) fail(RDB_EINVAL, "batch_fail_job must be in [0, 10^6]");
          ctx->c.batch_fail_job = static_cast<uint32_t>(value);
+      } else if (k == "query_fail") {
+         if (value < 0 || value > 1000000) fail(RDB_EINVAL, "query_fail must be in [0, 10^6]");
+         ctx->c.query_fail = static_cast<uint32_t>(value);
       } else if (k == "index_build_device") {
          if (value != 0 && value != 1) fail(RDB_EINVAL, "index_build_device must be 0 or 1");
          ctx->c.index_build_device = static_cast<uint32_t>(value);
@@ -356,6 +360,8 @@ int rdb_get_tuning(rdb_ctx* ctx, const char* key, int64_t* value) {
          *value = ctx->c.batch_row_capacity;
       } else if (k == "batch_fail_job") {
          *value = ctx->c.batch_fail_job;
+      } else if (k == "query_fail") {
+         *value = ctx->c.query_fail;
       } else if (k == "index_build_device") {
          *value = ctx->c.index_build_device;
       } else {
@@ -761,11 +767,13 @@ int rdb_mutation_counts(rdb_table* table, const rdb_bitmap* filter, const char* 
       const size_t bytes = static_cast<size_t>(col.abc->count) * col.genome_length * 4;
       void* dev = t.ctx->pool.get(bytes);
       try {
+         ScratchUse scratch(t);
          MutationsLaunch m = mutationsLaunch(t, idx, f);
          m.counts_out = static_cast<uint32_t*>(dev);
          hipCheck(launchMutations(m, t.ctx->stream), "mutations kernels");
          hipCheck(hipMemcpyAsync(counts, dev, bytes, hipMemcpyDeviceToHost, t.ctx->stream), "copy counts");
          hipCheck(hipStreamSynchronize(t.ctx->stream), "synchronize");
+         scratch.done();
       } catch (...) {
          t.ctx->pool.put(dev, bytes);
          throw;
@@ -783,6 +791,7 @@ namespace rdb::capi {
 ResultRows mutationResult(Table& t, const DeviceBitmap& f, int idx, double min_proportion) {
    Context& ctx = *t.ctx;
    void* pinned = ctx.pinnedBuffer(t.result_bytes);
+   ScratchUse scratch(t);
    MutationsLaunch m = mutationsLaunch(t, idx, f);
    m.min_proportion = min_proportion;
    const ResultRows r(pinned, t.seq[idx]->view);
@@ -796,6 +805,7 @@ ResultRows mutationResult(Table& t, const DeviceBitmap& f, int idx, double min_p
    hipCheck(launchMutations(m, ctx.stream), "mutations kernels");
    if (ctx.profiling) ctx.profileAccumulate(0);
    r.wait(ctx, m.stamp);
+   scratch.done();
    return r;
 }
 
@@ -1156,11 +1166,14 @@ void aggregateRows(Table& t, const DeviceBitmap& f, const char* dims, std::vecto
       auto* stamps = reinterpret_cast<unsigned long long*>(pinned);
       auto* out = reinterpret_cast<uint32_t*>(pinned + kStampBytes);
       const uint32_t stamp = ++ctx.mail_seq;
+      ScratchUse scratch(t);
       hipCheck(launchGroupHistogram(t.n_chunks, f.words, f.chunk_cards, t.chunk_sizes_dev.as<uint32_t>(), gd, pd, n_bins,
                                     t.hist.as<uint32_t>(), ctx.stream),
                "group histogram");
+      if (ctx.failsNow()) fail(RDB_EDEVICE, "injected query failure");
       hipCheck(launchEmitHistogram(n_bins, t.hist.as<uint32_t>(), out, stamps, stamp, ctx.stream), "group counts");
       waitStamps(ctx, reinterpret_cast<const uint64_t*>(stamps), (n_bins + kEmitBins - 1) / kEmitBins, stamp);
+      scratch.done();
       decodeHistogram(ds, gd.stride, out, bins, ids, counts);
       return;
    }

@@ -120,7 +120,7 @@ class DevicePool {
 
 // Table scratch of the single-query kernels (one query at a time runs on the context's stream).  The
 // filter's counters are zero between queries; the two sets of totals take turns, each cleared by the
-// Mutations query that uses the other.  Per-chunk counters of the filter kernel follow it in memory.
+// Mutations query that uses the other (after one that failed: ScratchUse).  Per-chunk counters of the filter kernel follow it in memory.
 struct QueryState {
    unsigned long long totals[2][3 * kMaxResultBlocks];
    unsigned long long filter_total;
@@ -199,6 +199,10 @@ struct Context {
    // fault injection for tests: the n-th lane job enqueued from now on fails with RDB_ENOMEM after
    // its inputs were staged (0: never)
    uint32_t batch_fail_job = 0;
+   // the n-th single Mutations or Aggregated query from now on fails with RDB_EDEVICE before its
+   // result kernel, after its counting kernels were enqueued (0: never)
+   uint32_t query_fail = 0;
+   bool failsNow() { return query_fail > 0 && --query_fail == 0; }
    // sequence index build: 1 local-reference adaptation and container entries on the device, 0 host
    uint32_t index_build_device = 1;
    // planner of the batched path: 0 reference order, 1 independence estimates, 2 learned estimator
@@ -312,6 +316,9 @@ struct Table {
    // per-call scratch (sized at finalize)
    DeviceBuffer slot_counts, heavy_sums, query_state, hist;
    uint32_t totals_turn = 0;  // the set of query_state's totals that the next Mutations query uses
+   // a query failed between its first kernel and its result: what queries leave zero in the scratch
+   // (query_state, heavy_sums, hist, the columns' sparse arrays) may not be
+   bool scratch_dirty = false;
    size_t result_bytes = 0;  // pinned host memory of the largest Mutations result (see ResultRows)
    // lanes of the batched path (created on demand)
    std::vector<std::shared_ptr<BatchLane>> lanes;
@@ -394,6 +401,21 @@ struct DeviceBitmap {
    std::vector<uint32_t> rows();
    // the row ids into out[cardinality()]
    void rowsInto(uint32_t* out);
+};
+
+// A query's use of its table's scratch, from before its first kernel to its result: on scratch that starts
+// zero, also when the query before failed half way.
+class ScratchUse {
+  public:
+   explicit ScratchUse(Table& t) : table_(t) {
+      if (t.scratch_dirty) clear();
+      t.scratch_dirty = true;
+   }
+   void done() { table_.scratch_dirty = false; }
+
+  private:
+   void clear();
+   Table& table_;
 };
 
 // Pinned host memory a kernel writes results to: kStamps stamps (numbers of requests, kernels.h), then the

@@ -141,6 +141,7 @@ struct MutationsLaunch {
    uint32_t stamp = 0;
    hipEvent_t count_start = nullptr;  // recorded around the dense counting kernel when set
    hipEvent_t count_stop = nullptr;
+   bool fail = false;  // fault injection for tests: an error in place of the result kernel
 };
 
 hipError_t launchMutations(const MutationsLaunch& m, hipStream_t stream);

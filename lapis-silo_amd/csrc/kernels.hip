@@ -3408,6 +3408,7 @@ hipError_t launchMutations(const MutationsLaunch& m, hipStream_t stream) {
                          n_words, m.filter, m.filter_card, m.sparse_max, m.sparse_counts, m.sparse_bnd, m.totals);
       if ((err = hipGetLastError()) != hipSuccess) return err;
    }
+   if (m.fail) return hipErrorOutOfMemory;
    MutationsResult r;
    r.partial = m.partial;
    r.n_parts = n_parts;

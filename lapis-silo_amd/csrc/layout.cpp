@@ -1439,6 +1439,21 @@ void finalizeTable(Table& t) {
    t.finalized = true;
 }
 
+// (on the stream, behind whatever the failed query enqueued)
+void ScratchUse::clear() {
+   hipStream_t stream = table_.ctx->stream;
+   const auto zero = [&](const DeviceBuffer& b) {
+      hipCheck(launchFill(b.as<uint32_t>(), 0, b.bytes() / 4, stream), "clear scratch");
+   };
+   zero(table_.query_state);
+   zero(table_.heavy_sums);
+   zero(table_.hist);
+   for (const auto& c : table_.seq) {
+      zero(c->sparse_counts);
+      zero(c->sparse_bnd);
+   }
+}
+
 // ---- device bitmaps ----------------------------------------------------------------------------
 DeviceBitmap::DeviceBitmap(Table* t) : table(t) {
    const size_t n_words = static_cast<size_t>(t->n_chunks) * kChunkWords;

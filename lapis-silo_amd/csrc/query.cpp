@@ -117,21 +117,21 @@ DeviceBitmap runProgram(Table& t, const Emitter& program, bool post) {
       const std::vector<uint8_t> blob = programBlob(program);
       dev = static_cast<uint8_t*>(ctx.stage(blob.data(), blob.size()));
    }
+   ScratchUse scratch(t);
    launchProgram(t, program, dev, out.words, out.card_dev, out.chunk_cards, t.query_state.as<QueryState>(),
                  post ? ctx.mail : nullptr, post ? ++ctx.mail_seq : 0);
+   if (post) {
+      out.card = t.n_chunks == 0 ? 0 : ctx.waitMail(ctx.mail_seq);
+      out.card_known = true;
+   }
+   scratch.done();  // (one kernel: it runs whole, and leaves its counters zero, or not at all)
    return out;
 }
 
 DeviceBitmap Operator::evaluate(bool post) const {
    Emitter e;
    emit(e);
-   DeviceBitmap out = runProgram(*table, e, post);
-   if (post) {
-      Context& ctx = *table->ctx;
-      out.card = table->n_chunks == 0 ? 0 : ctx.waitMail(ctx.mail_seq);
-      out.card_known = true;
-   }
-   return out;
+   return runProgram(*table, e, post);
 }
 
 // ---- predicates --------------------------------------------------------------------------------

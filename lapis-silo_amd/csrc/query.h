@@ -70,8 +70,8 @@ class Emitter {
    }
 };
 
-// Runs one emitted program over the table.  `post`: the cardinality is reported to the context's mail
-// (as request ctx.mail_seq), to be waited for at once.
+// Runs one emitted program over the table.  `post`: its cardinality is reported to the context's mail
+// and waited for.
 DeviceBitmap runProgram(Table& table, const Emitter& program, bool post = false);
 // The staged form of one program: its ProgramDesc, instructions, ranges and prefetch codes.
 std::vector<uint8_t> programBlob(const Emitter& program);

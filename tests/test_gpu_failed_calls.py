@@ -45,3 +45,40 @@ def test_failed_allocation(engine):
         assert answers(et, country) == want
     finally:
         et.close()
+
+
+@pytest.mark.parametrize("knobs", [{}, {"mutation_packed": 1}, {"mutation_coop": 0}, {"sparse_max_rows": 1 << 40}])
+def test_failure_between_kernels(engine, knobs):
+    """A query that fails after its counting kernels leaves its sums in the table's scratch: the next
+    queries, of the same action and of the others, start from zero all the same, and twice in a row
+    (the totals of two Mutations queries take turns)."""
+    from silo_amd.engine import EngineError
+
+    ds, ts = small_spec(seed=92, n_rows=9000, L=400, chunk=4096)
+    saved = {k: engine.get_tuning(k) for k in knobs}
+    et = engine.table(ts)
+    try:
+        for k, v in knobs.items():
+            engine.set_tuning(k, v)
+        country = ds.country_names[0]
+        want = answers(et, country)
+        for call in (lambda: et.mutations_query("(true)", "main", 0.05), lambda: et.mutation_counts("(true)", "main"),
+                     lambda: et.aggregate("(true)", ["country"]), lambda: et.aggregate("(true)", ["main@20", "country"])):
+            for n in (1, 2):  # fails at once, or after one that succeeds
+                engine.set_tuning("query_fail", n)
+                for _ in range(n - 1):
+                    call()
+                with pytest.raises(EngineError) as err:
+                    call()
+                assert err.value.status == "RDB_EDEVICE" and engine.get_tuning("query_fail") == 0
+                if n == 2:  # two failures in a row
+                    engine.set_tuning("query_fail", 1)
+                    with pytest.raises(EngineError):
+                        call()
+                assert answers(et, country) == want
+                assert answers(et, country) == want
+    finally:
+        engine.set_tuning("query_fail", 0)
+        for k, v in saved.items():
+            engine.set_tuning(k, v)
+        et.close()
