@@ -415,8 +415,9 @@ int rdb_set_planner(rdb_ctx* ctx, int mode, rdb_mlp* mlp);
  *   "index_build_device" 1: the local-reference adaptation and container entries of a sequence
  *                      column's index build run on the GPU (default), 0: on the host;
  *   "batch_fail_job"   fault injection for tests: the n-th lane job enqueued from now on fails with
- *                      RDB_ENOMEM after its inputs were staged, failing its rdb_batch_submit (0, the
- *                      default: never);
+ *                      RDB_ENOMEM after its inputs were staged or, with batch_graphs 0, with RDB_EDEVICE
+ *                      after its Mutations were counted, failing its rdb_batch_submit (0, the default:
+ *                      never);
  *   "query_fail"       fault injection for tests: the n-th Mutations or Aggregated query outside batches
  *                      from now on fails with RDB_EDEVICE after its counting kernels were enqueued and
  *                      before its result kernel (0, the default: never).

@@ -199,6 +199,7 @@ void enqueueKernels(Table& t, BatchLane& lane, uint32_t depth, int column, bool 
          m.scan_stop = lane.scan_events[1];
          lane.job_timed = true;
       }
+      m.fail = lane.fail;
       hipCheck(launchMutationsBatch(m, lane.stream), "batched Mutations kernels");
    } else {
       hipCheck(launchFill(lane.n_rows.as<uint32_t>(), 0, Q, lane.stream), "clear row counts");
@@ -346,14 +347,17 @@ void enqueueJob(Table& t, BatchResult& b, const std::vector<CompiledQuery>& cq, 
    lane.job_first_bytes = std::min(lane.out_bytes, ol.rows + (size_t{1} << 20));
    try {
       hipCheck(hipMemcpyAsync(lane.params.as<void>(), hp, pl.bytes, hipMemcpyHostToDevice, lane.stream), "stage batch");
-      if (t.ctx->batch_fail_job > 0 && --t.ctx->batch_fail_job == 0) fail(RDB_ENOMEM, "injected lane-job failure");
+      lane.fail = t.ctx->batch_fail_job > 0 && --t.ctx->batch_fail_job == 0;
+      if (lane.fail && t.ctx->batch_graphs) fail(RDB_ENOMEM, "injected lane-job failure");
       launchLane(t, lane, depth, job.column, n_agg > 0, n);
       hipCheck(hipMemcpyAsync(lane.host_out, lane.out.as<void>(), lane.job_first_bytes, hipMemcpyDeviceToHost, lane.stream),
                "copy batch results");
       hipCheck(hipEventRecord(lane.done, lane.stream), "hipEventRecord");
    } catch (...) {
-      // whatever was enqueued finishes before the lane takes another job; the lane stays free
+      // whatever was enqueued finishes, and the lane goes: a job that failed between its kernels may have
+      // left sums in the accumulators that each job finds zero and leaves zero
       (void)hipStreamSynchronize(lane.stream);
+      t.lanes.erase(std::find_if(t.lanes.begin(), t.lanes.end(), [&](const auto& l) { return l.get() == &lane; }));
       throw;
    }
    // the lane holds the job only once all of its work is enqueued

@@ -53,6 +53,7 @@ struct BatchLane {
    // timing of the job's dense counting kernel (profiling only)
    hipEvent_t scan_events[2] = {nullptr, nullptr};
    bool job_timed = false;
+   bool fail = false;  // fault injection for tests (Context::batch_fail_job)
 
    BatchLane() = default;
    BatchLane(const BatchLane&) = delete;

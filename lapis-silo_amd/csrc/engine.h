@@ -197,7 +197,7 @@ struct Context {
    uint32_t batch_octet_threads = 1024;  // work-group size of the eight-query scan (512 or 1024)
    uint32_t batch_octet_groups = 0;      // its persistent work-groups (0: one per CU)
    // fault injection for tests: the n-th lane job enqueued from now on fails with RDB_ENOMEM after
-   // its inputs were staged (0: never)
+   // its inputs were staged or, without graphs, with RDB_EDEVICE after its Mutations were counted (0: never)
    uint32_t batch_fail_job = 0;
    // the n-th single Mutations or Aggregated query from now on fails with RDB_EDEVICE before its
    // result kernel, after its counting kernels were enqueued (0: never)

@@ -209,6 +209,7 @@ struct MutationsBatch {
    uint32_t* n_rows = nullptr;                 // [max_queries]
    hipEvent_t scan_start = nullptr;            // recorded around the dense counting kernel when set
    hipEvent_t scan_stop = nullptr;
+   bool fail = false;                          // fault injection for tests: an error in place of the totals kernel
 };
 
 hipError_t launchMutationsBatch(const MutationsBatch& m, hipStream_t stream);

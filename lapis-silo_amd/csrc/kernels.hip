@@ -3511,6 +3511,7 @@ hipError_t launchMutationsBatch(const MutationsBatch& m, hipStream_t stream) {
                          dim3(kSparseBatchThreads), 0, stream, m);
       if ((err = hipGetLastError()) != hipSuccess) return err;
    }
+   if (m.fail) return hipErrorOutOfMemory;
    const uint32_t dense_parts = mode == 2 ? kOctetParts : (mode == 1 ? 2u : 1u);
    const uint32_t n_pblocks = (h.genome_length + kPosBlock - 1) / kPosBlock;
    hipLaunchKernelGGL(mutationsTotalsBatchKernel, dim3(n_pblocks, gq), dim3(kPosBlock), 0, stream, m,

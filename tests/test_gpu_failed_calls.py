@@ -4,7 +4,7 @@ import ctypes
 import numpy as np
 import pytest
 
-from helpers import small_spec
+from helpers import bitset_table, small_spec
 
 pytestmark = pytest.mark.gpu
 
@@ -79,6 +79,36 @@ def test_failure_between_kernels(engine, knobs):
                 assert answers(et, country) == want
     finally:
         engine.set_tuning("query_fail", 0)
+        for k, v in saved.items():
+            engine.set_tuning(k, v)
+        et.close()
+
+
+@pytest.mark.parametrize("knobs", [{"sparse_max_rows": 1 << 40}, {"batch_shared_scan": 1}, {"batch_shared_scan": 2}])
+def test_lane_job_failure_between_kernels(engine, knobs):
+    """A lane job launched kernel by kernel that fails after its Mutations were counted leaves nothing
+    to the next job: not the sparse counts, not the shared scans' sums of bitset containers."""
+    from silo_amd.engine import EngineError
+
+    spec, _, _ = bitset_table()
+    knobs = dict(knobs, batch_graphs=0, batch_lanes=1, batch_max_queries=8)
+    saved = {k: engine.get_tuning(k) for k in knobs}
+    et = engine.table(spec)
+    try:
+        for k, v in knobs.items():
+            engine.set_tuning(k, v)
+        queries = [{"filter": f, "action": "mutations", "column": "main", "min_proportion": 0.0}
+                   for f in ("(true)", "(date_between date 18262 18263)", '(str_eq country "c1")')]
+        want = [et.mutations_query(q["filter"], "main", 0.0) for q in queries]
+        assert et.batch(queries) == want
+        engine.set_tuning("batch_fail_job", 1)
+        with pytest.raises(EngineError) as err:
+            et.batch(queries)
+        assert err.value.status == "RDB_EDEVICE" and engine.get_tuning("batch_fail_job") == 0
+        assert et.batch(queries) == want
+        assert et.batch(queries) == want
+    finally:
+        engine.set_tuning("batch_fail_job", 0)
         for k, v in saved.items():
             engine.set_tuning(k, v)
         et.close()
