@@ -30,7 +30,11 @@ void Context::init(int dev) {
       (void)hipGetLastError();
       max_lds_bytes = 64 * 1024;
    }
-   hipCheck(configureHistogramKernel(max_lds_bytes), "histogram kernel");
+   max_positions = histogramPositions(max_lds_bytes);
+   if (max_positions > 0 && configureHistogramKernel(max_positions) != hipSuccess) {
+      (void)hipGetLastError();
+      max_positions = 0;
+   }
    hipCheck(hipHostMalloc(&stage_host, kStageSlots * kStageSlotBytes, hipHostMallocDefault), "pinned staging");
    stage_dev = DeviceBuffer(kStageSlots * kStageSlotBytes);
    for (auto& e : stage_events) hipCheck(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
@@ -1140,6 +1144,9 @@ void aggregateRows(Table& t, const DeviceBitmap& f, const char* dims, std::vecto
       } else {
          gd.labels[k] = ds[k].dict->labels.as<uint32_t>();
       }
+   }
+   if (pd.n > t.ctx->max_positions) {
+      fail(RDB_EDEVICE, "grouping by " + std::to_string(pd.n) + " sequence positions needs more LDS than a work-group has");
    }
    gd.n = static_cast<uint32_t>(ds.size());
    if (ds.empty()) {

@@ -141,6 +141,7 @@ struct Context {
    // device address of this GPU's allocation-free scratch (resolved by init)
    void* noalloc_scratch = nullptr;
    size_t max_lds_bytes = 64 * 1024;  // LDS a work-group may allocate
+   uint32_t max_positions = 0;        // sequence positions an Aggregated query may group by with it (0..4)
    // pinned host staging
    void* pinned = nullptr;
    size_t pinned_bytes = 0;

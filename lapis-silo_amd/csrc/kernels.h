@@ -249,8 +249,10 @@ hipError_t launchPackRows(const uint32_t* n_queries, uint32_t max_queries, const
 hipError_t launchGroupHistogram(uint32_t n_chunks, const uint64_t* filter, const uint32_t* filter_chunk_cards,
                                 const uint32_t* chunk_sizes, const GroupDims& dims, const PositionDims& positions,
                                 uint32_t n_bins, uint32_t* hist, hipStream_t stream);
-// Lets the histogram kernel hold the labels of four position dimensions.
-hipError_t configureHistogramKernel(size_t max_lds_bytes);
+// How many position dimensions' labels (16 KiB each) the histogram kernel can hold beside its counters
+// (66 KiB) in the LDS of a work-group: all four in 160 KiB.  configureHistogramKernel lets it.
+uint32_t histogramPositions(size_t max_lds_bytes);
+hipError_t configureHistogramKernel(uint32_t positions);
 // Moves a histogram to pinned host memory and clears it; kEmitBins bins per stamp (in its high half).
 constexpr uint32_t kEmitBins = 1024;
 hipError_t launchEmitHistogram(uint32_t n_bins, uint32_t* hist, uint32_t* out, unsigned long long* stamps, uint32_t stamp,

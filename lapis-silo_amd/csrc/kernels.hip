@@ -3559,12 +3559,14 @@ hipError_t launchGroupHistogram(uint32_t n_chunks, const uint64_t* filter, const
    return hipGetLastError();
 }
 
-hipError_t configureHistogramKernel(size_t max_lds_bytes) {
-   // its counters and words, and up to four position dimensions' labels
-   const size_t most = 4 * kHistRows;
-   if (4 * kHistLdsWords + 8 * 256 + most > max_lds_bytes) return hipErrorInvalidValue;
+uint32_t histogramPositions(size_t max_lds_bytes) {
+   constexpr size_t own = 4 * kHistLdsWords + 8 * 256;  // its counters and words
+   return max_lds_bytes < own ? 0 : static_cast<uint32_t>(std::min<size_t>(4, (max_lds_bytes - own) / kHistRows));
+}
+
+hipError_t configureHistogramKernel(uint32_t positions) {
    return hipFuncSetAttribute(reinterpret_cast<const void*>(&groupHistogramKernel),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(most));
+                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(positions * kHistRows));
 }
 
 hipError_t launchEmitHistogram(uint32_t n_bins, uint32_t* hist, uint32_t* out, unsigned long long* stamps, uint32_t stamp,

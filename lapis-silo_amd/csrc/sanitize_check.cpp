@@ -6,7 +6,8 @@
 //   sanitize_check host    entry points without device work: the diff of aligned sequences, the
 //                          saved-state scanners and bitmap decoder on whole, truncated and
 //                          corrupted buffers, the
-//                          NDJSON and Arrow IPC writers with every capacity below the needed one;
+//                          NDJSON and Arrow IPC writers with every capacity below the needed one,
+//                          the limits that a work-group's LDS sets;
 //   sanitize_check device  on GPU 0: tables built from the same rows by the device builder and by
 //                          the diff-form upload (equal digests), sequence, date, integer,
 //                          dictionary and lineage columns, every filter leaf kind, Count /
@@ -25,6 +26,7 @@
 #include <utility>
 #include <vector>
 
+#include "kernels.h"
 #include "rdb.h"
 
 namespace {
@@ -58,6 +60,19 @@ void put(std::vector<uint8_t>& b, T v) {
 }
 
 // ---- host mode ------------------------------------------------------------------------------------
+
+// What an engine may do with less LDS than the GPU has (Context::init falls back to 64 KiB): fewer grouping
+// positions and shallower filters, never none at all.
+void checkLdsLimits() {
+   CHECK(rdb::histogramPositions(64 * 1024) == 0);
+   CHECK(rdb::histogramPositions(66 * 1024 - 1) == 0 && rdb::histogramPositions(66 * 1024) == 0);
+   for (uint32_t n = 1; n <= 4; ++n) {
+      CHECK(rdb::histogramPositions((66 + 16 * n) * 1024 - 1) == n - 1);
+      CHECK(rdb::histogramPositions((66 + 16 * n) * 1024) == n);
+   }
+   CHECK(rdb::histogramPositions(160 * 1024) == 4);
+   CHECK(rdb::filterMaxDepth(64 * 1024) >= 15 && rdb::filterMaxDepth(160 * 1024) > rdb::filterMaxDepth(64 * 1024));
+}
 
 void checkDiff(Rng& rng) {
    const char* nuc = "ACGT-RYSWKMBDHVN";
@@ -719,6 +734,7 @@ int main(int argc, char** argv) {
       checkArchiveScanners(rng);
       checkBitmapRuns(rng);
       checkSinks(rng);
+      checkLdsLimits();
    } else if (mode == "device") {
       if (deviceMode() != 0) return 1;
    } else {

@@ -4,8 +4,8 @@
 (the counterpart of the reference's Debug build with ASAN, CMakeLists.txt:11) and linked with a
 driver of the C ABI.  Its host mode runs the entry points that need no device: the diff of aligned
 sequences, the saved-state scanners and bitmap decoder on whole, truncated and corrupted buffers,
-and the NDJSON and
-Arrow IPC writers at every capacity below the one needed.  Any sanitizer finding ends the process
+the NDJSON and Arrow IPC writers at every capacity below the one needed, and the limits that a
+work-group's LDS sets.  Any sanitizer finding ends the process
 with a report and a non-zero status."""
 import os
 import subprocess
