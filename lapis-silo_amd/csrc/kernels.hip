@@ -243,16 +243,17 @@ struct NoProgram {};
 constexpr uint32_t kVmRegStack = 15;
 constexpr uint32_t kPlaneGroup = 12;  // planes of a bit-sliced column loaded together (a date has ten or eleven)
 typedef uint64_t VmRegs __attribute__((ext_vector_type(kVmRegStack + 1)));
-// A single program's wavefronts are too few to fill the chip (992 on 4 M rows), so its stack stays in LDS,
-// whose entries cost less to reach: row ids of an n-of-m filter on 4 M rows 4 % slower with
-// registers.
-__host__ __device__ constexpr size_t vmWaveLdsBytes(uint32_t depth, bool single) {
-   const uint32_t in_registers = single ? 0 : kVmRegStack;
+// Where the wavefronts are few (a single program's, 992 on 4 M rows, and a small batch's) more of them do
+// not help, and the stack stays in LDS, whose entries cost less to reach: row ids of an n-of-m filter on
+// 4 M rows are 4 % slower with registers, and so are small batches of counts, trees of depth 5, call and
+// all (8 on 1 M rows: 845 us against 814; 4 on 2 M: 384 against 361; one on 4 M: 324 against 301).  See
+// filterStackInLds.
+__host__ __device__ constexpr size_t vmWaveLdsBytes(uint32_t depth, uint32_t in_registers) {
    return ((depth > in_registers ? depth - in_registers : 0) + 1) * 64 * sizeof(uint64_t) +
           kPrefetchSlots * 8 * sizeof(uint32_t) + kProgCache * sizeof(Instr);
 }
-template <bool kSingle>
-__global__ __launch_bounds__(kVmThreads, kSingle ? 1 : 4) void filterVmKernel(std::conditional_t<kSingle, SingleProgram, NoProgram> single,
+template <bool kSingle, uint32_t kRegs>
+__global__ __launch_bounds__(kVmThreads, kRegs == 0 ? 1 : 4) void filterVmKernel(std::conditional_t<kSingle, SingleProgram, NoProgram> single,
                                                              TableView tv, const ProgramDesc* __restrict__ progs,
                                                              const Instr* __restrict__ instrs,
                                                              const uint32_t* __restrict__ ranges, uint32_t depth,
@@ -276,9 +277,8 @@ __global__ __launch_bounds__(kVmThreads, kSingle ? 1 : 4) void filterVmKernel(st
    const uint32_t lane = threadIdx.x & 63;
    // per wavefront: the stack's entries past the register ones, scratch words, the prefetched leaf
    // records, the cached instructions
-   constexpr uint32_t kRegs = kSingle ? 0 : kVmRegStack;
    const uint32_t n_deep = depth > kRegs ? depth - kRegs : 0;
-   uint8_t* mine = reinterpret_cast<uint8_t*>(lds) + wave * vmWaveLdsBytes(depth, kSingle);
+   uint8_t* mine = reinterpret_cast<uint8_t*>(lds) + wave * vmWaveLdsBytes(depth, kRegs);
    uint64_t* deep = reinterpret_cast<uint64_t*>(mine);
    uint64_t* scratch = deep + n_deep * 64;
    uint32_t* pf = reinterpret_cast<uint32_t*>(scratch + 64);
@@ -3301,24 +3301,35 @@ hipError_t launchFill(uint32_t* p, uint32_t value, size_t n, hipStream_t stream)
 
 hipError_t configureFilterKernel(size_t max_lds_bytes) {
    if (max_lds_bytes <= 64 * 1024) return hipSuccess;
-   const hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(&filterVmKernel<false>),
-                                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(max_lds_bytes));
-   if (err != hipSuccess) return err;
-   return hipFuncSetAttribute(reinterpret_cast<const void*>(&filterVmKernel<true>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(max_lds_bytes));
+   for (const void* kernel : {reinterpret_cast<const void*>(&filterVmKernel<true, 0>),
+                              reinterpret_cast<const void*>(&filterVmKernel<false, 0>),
+                              reinterpret_cast<const void*>(&filterVmKernel<false, kVmRegStack>)}) {
+      const hipError_t err =
+         hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(max_lds_bytes));
+      if (err != hipSuccess) return err;
+   }
+   return hipSuccess;
 }
 
-static size_t filterLdsBytes(uint32_t depth, bool single) { return kVmWaves * vmWaveLdsBytes(depth, single); }
+static size_t filterLdsBytes(uint32_t depth, uint32_t in_registers) { return kVmWaves * vmWaveLdsBytes(depth, in_registers); }
 
 uint32_t filterMaxDepth(size_t max_lds_bytes) {
    // as deep as if the whole stack were in LDS, beside 6 KiB of a wavefront's own: what programs have
    // always been accepted up to
    const size_t entries = (max_lds_bytes / kVmWaves - 6144) / (64 * sizeof(uint64_t));
-   static_assert(kVmWaves * vmWaveLdsBytes(2, true) <= 64 * 1024, "shallow programs fit the smallest LDS");
+   static_assert(kVmWaves * vmWaveLdsBytes(2, 0) <= 64 * 1024, "shallow programs fit the smallest LDS");
    return std::max<uint32_t>(1, static_cast<uint32_t>(entries) - 1);
 }
 
 namespace {
+// The operand stack of a batch lies in LDS where all its work-groups are resident at once that way (256
+// CUs of 160 KiB): up to 4,096 slices with stacks of eight entries, 2,048 with 24.  Past that registers
+// win, on 62 chunks with 8 trees of depth 5 (1,066 us against 1,317) or 16 of depth 3 (922 against 1,004).
+bool filterStackInLds(uint32_t n_items, uint32_t depth) {
+   constexpr size_t kCus = 256, kCuLdsBytes = 160 * 1024;
+   return n_items <= kCus * (kCuLdsBytes / filterLdsBytes(depth, 0)) * kVmWaves;
+}
+
 // Slices per unit and work-groups of a filter launch over n_items slices: more slices a unit only
 // where the units still outnumber the wavefronts well (a single query needs every slice in
 // parallel); unit_slices divides kSlicesPerChunk
@@ -3335,8 +3346,15 @@ hipError_t launchFilterBatch(const TableView& tv, const ProgramDesc* progs, cons
    if (n_items == 0) return hipSuccess;
    // a work-group per kVmWaves slices (the most units there can be) up to max_blocks
    const uint32_t blocks = std::min((n_items + kVmWaves - 1) / kVmWaves, max_blocks);
-   hipLaunchKernelGGL(filterVmKernel<false>, dim3(blocks), dim3(kVmThreads), filterLdsBytes(depth, false), stream,
-                      NoProgram{}, tv, progs, instrs, ranges, depth, out, cards, chunk_cards, header, filterUnit(n_items));
+   const uint32_t unit = filterUnit(n_items);
+   if (filterStackInLds(n_items, depth)) {
+      hipLaunchKernelGGL((filterVmKernel<false, 0>), dim3(blocks), dim3(kVmThreads), filterLdsBytes(depth, 0), stream,
+                         NoProgram{}, tv, progs, instrs, ranges, depth, out, cards, chunk_cards, header, unit);
+   } else {
+      hipLaunchKernelGGL((filterVmKernel<false, kVmRegStack>), dim3(blocks), dim3(kVmThreads),
+                         filterLdsBytes(depth, kVmRegStack), stream, NoProgram{}, tv, progs, instrs, ranges, depth, out,
+                         cards, chunk_cards, header, unit);
+   }
    return hipGetLastError();
 }
 
@@ -3345,8 +3363,8 @@ hipError_t launchFilterSingle(const TableView& tv, const SingleProgram& program,
    const uint32_t n_items = tv.n_chunks * kSlicesPerChunk;
    if (n_items == 0) return hipErrorInvalidValue;
    const uint32_t unit = filterUnit(n_items);
-   hipLaunchKernelGGL(filterVmKernel<true>, dim3((n_items / unit + kVmWaves - 1) / kVmWaves), dim3(kVmThreads),
-                      filterLdsBytes(depth, true), stream, program, tv, static_cast<const ProgramDesc*>(nullptr),
+   hipLaunchKernelGGL((filterVmKernel<true, 0>), dim3((n_items / unit + kVmWaves - 1) / kVmWaves), dim3(kVmThreads),
+                      filterLdsBytes(depth, 0), stream, program, tv, static_cast<const ProgramDesc*>(nullptr),
                       static_cast<const Instr*>(nullptr), static_cast<const uint32_t*>(nullptr), depth, out, card,
                       chunk_cards, static_cast<const uint32_t*>(nullptr), unit);
    return hipGetLastError();

@@ -1,6 +1,6 @@
 """Filter programs where the filter kernel's work is cut: stacks around the entries that registers hold
 and deeper, programs around the length that is cut into single slices, counters that carry through every
-plane; alone and in batches of mixed lengths.  Against numpy."""
+plane; alone, in batches of mixed lengths and in small batches.  Against numpy."""
 import numpy as np
 import pytest
 
@@ -55,6 +55,21 @@ def test_programs(engine, sizes):
         many = cases * 12  # long programs and short ones, more units than wavefronts at nine chunks
         with et.batch_submit([{"action": "count", "filter": text} for text, _ in many]) as b:
             assert [b.count(q) for q in range(len(many))] == [int(keep.sum()) for _, keep in many]
+    finally:
+        et.close()
+
+
+@pytest.mark.parametrize("chunks,n", [(1, 1), (1, 24), (3, 8), (9, 4), (9, 8), (16, 8), (16, 16)])
+def test_small_batches(engine, chunks, n):
+    """Batches of n programs around the number of slices up to which the operand stack lies in LDS, for
+    shallow stacks (4,096: 16 chunks, 16 programs) and for deeper ones (3,072 to 1,024)."""
+    et, _, x, _ = plain_table(engine, [65536] * (chunks - 1) + [4500], seed=chunks)
+    try:
+        cases = programs(np.random.default_rng(11), x)
+        for k in range(0, len(cases), n):
+            some = cases[k:k + n]
+            with et.batch_submit([{"action": "count", "filter": text} for text, _ in some]) as b:
+                assert [b.count(q) for q in range(len(some))] == [int(keep.sum()) for _, keep in some], k
     finally:
         et.close()
 
