@@ -1,6 +1,7 @@
 """The diff of aligned sequences where its kernel's work is cut: rows that start at any byte of an aligned
 16, differences and missing runs at the edges of a lane's 16 characters and of a step's 1,024, rows that
-differ everywhere, lower case, references with missing positions; an append of 74 MB;
+differ everywhere, lower case, references with missing positions; an append of 74 MB in one piece, and
+appends cut after 2^20 rows whose second piece has more characters than the first or fewer;
 the adapted reference at the edges of the blocks of 64 positions that the rule is cut into.  Layouts equal
 those of the oracle's diff, uploaded in diff form, byte for byte."""
 import numpy as np
@@ -65,19 +66,57 @@ def test_large_append(engine):
     check(engine, table.TableSpec(chunk_sizes=sizes), 0, ref, rows, copies, 300 * copies)
 
 
-def check(engine, spec, alphabet, ref, rows, copies, batch_rows):
+@pytest.mark.parametrize("grows", [True, False])
+def test_append_of_several_pieces(engine, grows):
+    """One append of 2^20 + 30,720 rows: the builder's text buffer goes from one piece to the next, and
+    either grows or holds the first piece's characters past the second's end, whose last rows end
+    at any byte of an aligned 16."""
     from silo_amd import table
 
-    c = oracle_column("main", alphabet, ref, rows)
-    # the rows `copies` times
-    def times(ptr):
-        step = np.diff(ptr.astype(np.int64))
-        return np.concatenate([[0], np.cumsum(np.tile(step, copies))]).astype(np.uint64)
+    rng = np.random.default_rng(6 + grows)
+    ref = "".join(rng.choice(list("ACGT"), 400))
 
-    host = table.SeqColumnData("main", alphabet, c.reference, *[np.tile(a, copies) for a in (c.is_null, c.cov_start, c.cov_end)],
-                               times(c.mut_ptr), np.tile(c.mut_pos, copies), np.tile(c.mut_sym, copies), times(c.nrun_ptr),
-                               np.tile(c.nrun_start, copies), np.tile(c.nrun_end, copies))
-    spec.seq_columns = [aligned_column("main", alphabet, ref, rows * copies, batch_rows)]
+    def some(lo, hi, n):  # rows of lo .. hi characters somewhere, a few differences and missing runs in each
+        rows = []
+        for i in range(n):
+            m = int(rng.integers(lo, hi + 1))
+            o = int(rng.integers(0, 400 - m + 1))
+            s = list(ref[o:o + m])
+            for p in rng.integers(0, m, size=2 if m else 0):
+                s[p] = "ACGTRN-n"[int(rng.integers(0, 8))]
+            rows.append((None if i % 97 == 5 else "".join(s), o))
+        return rows
+
+    short, long = some(0, 8, 1024), some(300, 400, 1024)
+    first, then = (short, long) if grows else (some(9, 40, 1024), short)
+    parts = [(first, 1024), (then, 30)]
+    n = 1024 * 1054
+    sizes = np.array([65536] * (n // 65536) + [n % 65536], np.uint32)
+    check_parts(engine, table.TableSpec(chunk_sizes=sizes), 0, ref, parts, n)
+
+
+def check(engine, spec, alphabet, ref, rows, copies, batch_rows):
+    check_parts(engine, spec, alphabet, ref, [(rows, copies)], batch_rows)
+
+
+def check_parts(engine, spec, alphabet, ref, parts, batch_rows):
+    """The rows of each part, as many times as it says."""
+    from silo_amd import table
+
+    columns = [(oracle_column("main", alphabet, ref, rows), copies) for rows, copies in parts]
+
+    def times(name):
+        return np.concatenate([np.tile(getattr(c, name), copies) for c, copies in columns])
+
+    def ptr_times(name):
+        step = np.concatenate([np.tile(np.diff(getattr(c, name).astype(np.int64)), copies) for c, copies in columns])
+        return np.concatenate([[0], np.cumsum(step)]).astype(np.uint64)
+
+    host = table.SeqColumnData("main", alphabet, columns[0][0].reference, *map(times, ("is_null", "cov_start", "cov_end")),
+                               ptr_times("mut_ptr"), times("mut_pos"), times("mut_sym"), ptr_times("nrun_ptr"),
+                               times("nrun_start"), times("nrun_end"))
+    rows = [row for part, copies in parts for row in part * copies]
+    spec.seq_columns = [aligned_column("main", alphabet, ref, rows, batch_rows)]
     built = engine.table(spec)
     spec.seq_columns = [host]
     engine.set_tuning("index_build_device", 0)
