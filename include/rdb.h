@@ -47,7 +47,11 @@ typedef struct rdb_table rdb_table;   /* row layout + device-resident columns */
 typedef struct rdb_bitmap rdb_bitmap; /* device-resident row set (result of a filter) */
 
 /* ---- context ---------------------------------------------------------------------------------- */
-/* Replaces: nothing in the reference (the reference has no device); owns the HIP stream. */
+/* Replaces: nothing in the reference (the reference has no device); owns the HIP stream.  Held until
+ * rdb_close, besides 64 MiB of staging on the host and on the GPU: pinned host memory for the largest result so
+ * far (a table's finalize reserves 16 bytes per position and valid symbol of its longest column; groups take
+ * 4 bytes per bin up to 1 MiB, row ids up to 16 MiB), and per table 1 MiB of histogram once groups
+ * were counted. */
 int rdb_open(int device, rdb_ctx** out);
 void rdb_close(rdb_ctx* ctx);
 const char* rdb_last_error(const rdb_ctx* ctx);
@@ -225,9 +229,11 @@ int rdb_mutations_query(rdb_table* table, const char* filter, const char* column
  * same results, but every device buffer the call needs beyond the table (staged filter program,
  * filter words, partial sums, accumulators) is carved from one file-scope device array of
  * 128 MiB per GPU, held until the process ends; the call makes no hipMalloc, hipFree or pinned
- * allocation.  RDB_EINVAL when the table needs more scratch than that (about 8 KiB per chunk for
- * the filter plus 4 bytes per (position, symbol) slot per chunk group).  All calls on one GPU share
- * the array: calls that overlap on one GPU (from different contexts or threads) race. */
+ * allocation.  RDB_EINVAL when the table needs more scratch than that: about 8 KiB per chunk for
+ * the filter, 4 bytes per (position, symbol) slot for its heavy sum and for each part of its partial sums
+ * (up to 32, or as few as one when the rest leaves no room), and 4 bytes per position for each symbol and
+ * three boundary sums.  All calls on one GPU share the array: calls that overlap on one GPU (from different
+ * contexts or threads) race; a call that has returned has left it. */
 int rdb_mutations_query_noalloc(rdb_table* table, const char* filter, const char* column, double min_proportion,
                                 uint32_t* position, uint8_t* from, uint8_t* to, uint32_t* count, uint32_t* coverage,
                                 double* proportion, uint64_t capacity, uint64_t* n);
@@ -359,7 +365,9 @@ void rdb_batch_free(rdb_batch* batch);
 typedef struct rdb_mlp rdb_mlp;
 
 /* Parameters: per layer W (out x in, row-major) then b; inputs -> n_hidden_layers x n_hidden -> 1.
- * He-uniform initial weights from `seed`, zero biases. */
+ * He-uniform initial weights from `seed`, zero biases.  Until rdb_mlp_free the handle keeps, in device
+ * memory, the largest training set it was given, the buffers of its largest batch and, for networks of up to
+ * 128 inputs and hidden units, up to 256 sets of partial gradients (38 MB for 32 -> 3 x 128 -> 1). */
 int rdb_mlp_create(rdb_ctx* ctx, uint32_t n_in, uint32_t n_hidden, uint32_t n_hidden_layers, uint64_t seed,
                    rdb_mlp** out);
 void rdb_mlp_free(rdb_mlp* mlp);

@@ -1,9 +1,7 @@
 // The C ABI (include/rdb.h): status codes at the boundary, exceptions inside.
 #include <algorithm>
-#include <chrono>
 #include <cmath>
 #include <cstring>
-#include <emmintrin.h>
 #include <new>
 #include <string>
 
@@ -91,22 +89,6 @@ void* Context::stage(const void* host, size_t bytes) {
    return d;
 }
 
-// memcpy to a 16-byte aligned place that the CPU does not read again: stores past the caches.
-static void streamCopy(uint8_t* to, const uint8_t* from, size_t n) {
-   size_t i = 0;
-   for (; i + 64 <= n; i += 64) {
-      const auto* a = reinterpret_cast<const __m128i*>(from + i);
-      auto* b = reinterpret_cast<__m128i*>(to + i);
-      const __m128i v0 = _mm_loadu_si128(a), v1 = _mm_loadu_si128(a + 1), v2 = _mm_loadu_si128(a + 2), v3 = _mm_loadu_si128(a + 3);
-      _mm_stream_si128(b, v0);
-      _mm_stream_si128(b + 1, v1);
-      _mm_stream_si128(b + 2, v2);
-      _mm_stream_si128(b + 3, v3);
-   }
-   std::memcpy(to + i, from + i, n - i);
-   _mm_sfence();  // before the copy that reads it is enqueued
-}
-
 uint32_t maxFilterDepth(const Context& ctx) {
    return filterMaxDepth(ctx.max_lds_bytes);
 }
@@ -139,8 +121,11 @@ const DeviceBitmap& filterOf(const Table& t, const rdb_bitmap* f) {
 // a group per four chunks (one per wavefront); when the work-group shares each tile, a group per
 // three and a half chunks (measured fastest on 62-chunk tables: 18 groups, every work-group
 // resident at once at six wavefronts per SIMD), or a chunk each up to kResidentParts chunks.
+// The lines hold for every column: the index build cuts each, of any length, into about 64 blocks of equal
+// bytes (66 to 69 at 29,903 nucleotides and for a gene of 1,273 amino acids), more only where a
+// block is full of slots.
 constexpr uint32_t kResidentParts = 18;  // parts of a 66-block column resident at once: 1,188 work-groups
-uint32_t mutationGroups(const Table& t, const SeqColumn& /*col*/) {
+uint32_t mutationGroups(const Table& t) {
    if (t.ctx->mutation_groups) {
       return std::clamp<uint32_t>(t.ctx->mutation_groups, 1 + t.n_chunks / kMaxGroupChunks, kMaxGroups);
    }
@@ -167,7 +152,7 @@ MutationsLaunch mutationsLaunch(Table& t, int idx, const DeviceBitmap& f) {
    m.col_host = &col.view;
    m.chunk_sizes = t.chunk_sizes_dev.as<uint32_t>();
    m.n_chunks = t.n_chunks;
-   m.n_groups = mutationGroups(t, col);
+   m.n_groups = mutationGroups(t);
    m.n_splits = mutationSplits(t, m.n_groups);
    m.unroll = t.ctx->mutation_unroll;
    m.coop = t.ctx->mutation_coop != 0;
@@ -909,8 +894,9 @@ int rdb_mutations_query(rdb_table* table, const char* filter, const char* column
 }
 
 // Mutations query whose kernels use only the device's file-scope scratch array: the staged filter
-// program, the filter words, partial sums, heavy sums, totals, sparse accumulators and rows are
-// carved from it (256-byte aligned); nothing is allocated on the device or pinned on the host.
+// program, the filter words, partial sums, heavy sums, totals and sparse accumulators are carved from it
+// (256-byte aligned), and the rows go to the pinned buffer that the context has held since the table's
+// finalize; nothing is allocated on the device or pinned on the host.
 int rdb_mutations_query_noalloc(rdb_table* table, const char* filter, const char* column, double min_proportion,
                                 uint32_t* position, uint8_t* from, uint8_t* to, uint32_t* count, uint32_t* coverage,
                                 double* proportion, uint64_t capacity, uint64_t* n) {
@@ -950,7 +936,7 @@ int rdb_mutations_query_noalloc(rdb_table* table, const char* filter, const char
          c.sparse_bnd = take(4ULL * 3 * L);
          c.end = o;
       };
-      uint32_t groups = mutationGroups(t, col), splits = mutationSplits(t, groups);
+      uint32_t groups = mutationGroups(t), splits = mutationSplits(t, groups);
       layout(groups * splits);
       while (c.end > kNoAllocScratchBytes && groups * splits > 1) {
          if (splits > 1) {

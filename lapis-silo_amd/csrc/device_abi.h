@@ -124,7 +124,7 @@ struct SeqColumnView {
    const uint32_t* run_index_ptr;     // [(c * (n_run_buckets + 1) + k) * 16 + s], and one more
    const uint64_t* run_index;
    const uint64_t* null_bits;         // [n_chunks * 1024]
-   const uint32_t* pos_ranges;        // [(chunk * L + position) * 6]: [lo, hi) of the position's light
+   const uint32_t* pos_ranges;        // [(chunk * L + position) * kPosRecord]: [lo, hi) of the position's light
                                       // entries, groups and descriptors in its tile
    const uint32_t* row_mut_ptr;       // [n_chunks * 2^16 + 1] row-major mutations (sparse path)
    const uint32_t* row_muts;          // position | symbol << 16, original-reference frame

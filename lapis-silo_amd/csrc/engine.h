@@ -254,7 +254,7 @@ struct SeqColumn {
    uint64_t row_major_bytes = 0;             // row-major mutation CSR (sparse path)
    RawVector<uint32_t> row_mut_ptr, row_nrun_ptr;  // host copies over padded rows (traffic accounting)
    DeviceBuffer boundary_slots;
-   DeviceBuffer sparse_counts, sparse_bnd;   // zero between calls; cleared by the sparse finalize
+   DeviceBuffer sparse_counts, sparse_bnd;   // zero between calls; cleared by the result kernel
    // wall time (ms) of the index build's phases: checks, adaptation, containers, slots and tiles,
    // row-level arrays, layout checks, upload
    double build_ms[kBuildPhases] = {};

@@ -1229,7 +1229,7 @@ __global__ __launch_bounds__(kMutThreads) __attribute__((amdgpu_waves_per_eu(kCo
 // global atomics.  Work is proportional to the filter's rows, not to the index.
 //   counts[s * L + p]  rows of F with symbol s at p (s != reference[p])
 //   bnd[p], bnd[L + p], bnd[2L + p]  A(p), B(p), C(p) as in the dense path
-// Both arrays must be zero on entry; the sparse finalize kernel clears what it reads.
+// Both arrays must be zero on entry; the result and finalize kernels clear what they read.
 // ------------------------------------------------------------------------------------------------
 // Sparse counts go through a per-work-group LDS table before global memory: rows of one filter share
 // most of their mutations (a lineage's) and their covered-range ends, so global atomics would pile

@@ -187,7 +187,9 @@ __device__ inline f32x16 rowsTimesPacked(const float* a, const uint16_t* b, uint
 // hidden units 32 w .. 32 w + 31, and weights are read once per tile from their packed BF16 copies
 // (74 KB for the planner's network: L2).  The layer-by-layer form wrote and re-read every activation,
 // and its weight gradients (128 x 128 outputs over thousands of rows) ran in four work-groups.
-// Bound by the FP32 matrix rate (256 flop per cycle and CU): about 11 us a training tile.  32 rows
+// Bound by the chain of dependent layers: a launch of one training tile per work-group takes 56 us, in which
+// the matrix instructions keep a SIMD busy for 11 (26.6 k cycles, SQ_VALU_MFMA_BUSY_CYCLES); its one wavefront
+// waits for half of its cycles (SQ_WAIT_ANY), for weights, LDS and the barriers between layers.  32 rows
 // keep one tile per work-group at the training batch of 4,096 (128 work-groups); 16 would fill all
 // CUs but double the partial gradients written.
 // C layout of the 32x32 products: register i of lane l is row 8 (i / 4) + 4 (l / 32) + i % 4, column

@@ -3,10 +3,11 @@
 // One file-scope device array, `scratch`, holds everything that entry point's kernels need beyond
 // their inputs and outputs: a filter program too long for the kernel's arguments, the filter's row
 // words and cardinalities, the Mutations kernels' partial sums, heavy sums, counters and totals, and
-// sparse accumulators (the rows go straight to pinned host memory that the context keeps).  Each GPU the library runs on holds its own copy for the
-// life of the process.  Its device address comes from hipGetSymbolAddress, resolved once per
+// sparse accumulators (the rows go straight to pinned host memory that the context keeps).  Each GPU the
+// library runs on holds its own copy for the life of the process.  Its device address comes from hipGetSymbolAddress, resolved once per
 // device with that device current (the array's name is only a host-side stand-in); all host code
-// uses that address.  Every call on one GPU shares the array: calls that overlap on one GPU race.
+// uses that address.  Every call on one GPU shares the array: calls that overlap on one GPU race; one that
+// has returned has left it.
 #include <hip/hip_runtime.h>
 
 #include <mutex>
